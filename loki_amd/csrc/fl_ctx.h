@@ -62,8 +62,8 @@ struct FLCtx {
     // pinned, device-mapped copy of the last code a kernel reported (null if the host allocation failed): every
     // fl_moe_layer call checks it without waiting for the stream, fl_sync reports and clears it
     int * herr = nullptr, * herr_dev = nullptr;   // host pointer, and the address kernels store to
-    // prefill grouped GEMM on MFMA (batches above the decode sizes): fp16 table image, columns, fp16 activation copies
-    int pf_mfma = 1, pf_ready = 0; DBuf<uint4> ptab; DBuf<int4> pcols; DBuf<int> pncols; DBuf<_Float16> xh, hh;
+    // prefill grouped GEMM on MFMA (batches above the decode sizes): digit table image, columns, fp16 activation copies (K-quants)
+    int pf_mfma = 1, pf_ready = 0; DBuf<uint4> ptab; DBuf<int4> pcols, pcolsk; DBuf<int> pncols; DBuf<_Float16> xh, hh;
     struct Compat * compat = nullptr;          // reference-API state (compat.hip), created on first use
     // formats of fl_moe_layer's matrices (fl_set_layer_formats): routed down, shared gate, up, down; K-quant matrices
     // are read in place (ggml layout), IQ2_XXS ones tiled

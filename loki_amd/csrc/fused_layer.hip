@@ -128,7 +128,7 @@ extern "C" void fl_free(FLCtx * c) {
     c->sel.release(); c->counts.release(); c->offsets.release(); c->perm.release(); c->inv.release(); c->act.release(); c->nact.release();
     compat_free(c); c->zero_i.release(); c->terms.release(); c->cnt.release();
     c->tab.release(); c->derr.release(); c->dlogit.release(); c->dth.release(); c->dto.release(); c->dxq.release();
-    c->ptab.release(); c->pcols.release(); c->pncols.release(); c->xh.release(); c->hh.release();
+    c->ptab.release(); c->pcols.release(); c->pcolsk.release(); c->pncols.release(); c->xh.release(); c->hh.release();
     c->ksg.release(); c->ksu.release(); c->rcnt.release(); c->rpart.release(); c->dscr.release();
     for (auto & v : c->ev_free) { for (auto e : v) { (void) hipEventDestroy(e); } }
     for (auto & v : c->ev_pending) { for (auto e : v) { (void) hipEventDestroy(e); } }
@@ -503,6 +503,7 @@ int prefill_ready(FLCtx * c) {
     if (c->pf_ready) { return FL_OK; }
     ALLOC(c, c->ptab, prefill_table_bytes() / 16);
     TRY(c, build_prefill_tables(c->ptab.p, c->st));
+    if (!c->tab.p) { ALLOC(c, c->tab, TAB_BYTES / 16); TRY(c, build_table_image(c->tab.p, c->st)); }
     TRY(c, prefill_init());
     TRY(c, kq_gemm_init());
     if (!c->derr.p) { ALLOC(c, c->derr, 1); TRY(c, hipMemsetAsync(c->derr.p, 0, sizeof(int), c->st)); }
@@ -591,8 +592,8 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     }
     if (mfma) {
         if (int rc = prefill_ready(c)) { return rc; }
-        ALLOC(c, c->xh, (size_t) n * E); ALLOC(c, c->hh, rows * H);
-        ALLOC(c, c->pcols, rows / 32 + NEXP_MAX + 2); ALLOC(c, c->pncols, PF_NCOLS);
+        ALLOC(c, c->pcols, rows / pf_tok(n) + NEXP_MAX + 4); ALLOC(c, c->pncols, 2 * PF_NCOLS);
+        if (kq) { ALLOC(c, c->xh, (size_t) n * E); ALLOC(c, c->hh, rows * H); ALLOC(c, c->pcolsk, rows / KQ_TOK + NEXP_MAX + 4); }
     }
     prof_mark(c, ev, 0);
     if (prenorm) {   // the per-pass path normalises into a context buffer first (k_rmsnorm: the same arithmetic)
@@ -601,7 +602,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         x = c->xn.p;
     }
     TRY(c, launch_quant_q8k(x, n, E, c->xq.p, c->xd.p, st));
-    if (mfma) { TRY(c, launch_q8_to_h(c->xq.p, c->xh.p, (int64_t) n * E, st)); }
+    if (mfma && kq) { TRY(c, launch_q8_to_h(c->xq.p, c->xh.p, (int64_t) n * E, st)); }
     prof_mark(c, ev, 1);
     double * rp = nullptr;   // the K-split tiles' parts (n from RL_SPLIT_MIN to RL_SPLIT_MAX)
     if (const size_t nd = router_split_doubles(n, ne, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
@@ -619,26 +620,30 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     if (const size_t nd = dispatch_scratch_ints(P)) { ALLOC(c, c->dscr, nd); dsc = c->dscr.p; }
     TRY(c, launch_dispatch(c->sel.p, P, ne, c->counts.p, c->offsets.p, c->perm.p, c->inv.p, c->act.p, c->nact.p, st, dsc));
     if (mfma) {
-        TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, n, P, c->pcols.p, c->pncols.p, st));
+        const PfTable iq = { c->pcols.p, c->pncols.p, pf_tok(n), pf_few(n) };
+        const PfTable kt = { kq ? c->pcolsk.p : nullptr, c->pncols.p + PF_NCOLS, KQ_TOK, 0 };
+        TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, n, P, iq, kt, st));
         prof_mark(c, ev, 4);
         // Columns: the shared expert's first (nsh of them), then the routed experts'. Each matrix runs where its format
         // does: IQ2_XXS on the IQ2_XXS GEMM, Q2_K / Q3_K / Q6_K downs and a Q5_K shared gate / up on the K-quant GEMM,
         // any other K-quant on the mat-vecs.
-        const int nsh = prefill_shared_cols(n);
+        const int nsh = prefill_shared_cols(n, KQ_TOK), nshi = prefill_shared_cols(n, iq.tok);   // K-quant, IQ2_XXS tables
+        const auto iq2_gemm = iq.tok == FEW_TOK ? launch_few_gemm : launch_prefill_gemm;
         PrefillArgs g{};
         g.ptab = c->ptab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
         g.estride = (size_t) H * (E / 256) * IQ2B; g.sh[0] = (const uint8_t *) L->sh_gate; g.sh[1] = (const uint8_t *) L->sh_up;
-        g.perm = c->perm.p; g.topk = tk; g.P = P; g.R = H; g.K = E; g.nmat = 2; g.cols = c->pcols.p; g.ncols = c->pncols.p;
-        g.bh = c->xh.p; g.bd = c->xd.p; g.out = c->h.p; g.gdbg = c->dbg_gu ? c->g.p : nullptr; g.udbg = c->dbg_gu ? c->u.p : nullptr;
+        g.perm = c->perm.p; g.topk = tk; g.P = P; g.R = H; g.K = E; g.nmat = 2;
+        g.cols = iq.cols; g.ncols = iq.ncols; g.most = n;
+        g.bq = c->xq.p; g.tab = c->tab.p; g.bd = c->xd.p; g.out = c->h.p; g.gdbg = c->dbg_gu ? c->g.p : nullptr; g.udbg = c->dbg_gu ? c->u.p : nullptr;
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
-        g.col0 = lf[1] == FL_IQ2 ? 0 : nsh;
-        TRY(c, launch_prefill_gemm(g, c->ncu, st));
+        g.col0 = lf[1] == FL_IQ2 ? 0 : nshi;
+        TRY(c, iq2_gemm(g, c->ncu, st));
         if (lf[1] == FL_Q5K && lf[2] == FL_Q5K) {   // the real shards' shared gate / up: ksg / ksu rows 0 .. n - 1
             ALLOC(c, c->ksg, (size_t) n * H); ALLOC(c, c->ksu, (size_t) n * H);
             for (int m = 0; m < 2; ++m) {
                 PrefillArgs k{};
                 k.sh[0] = (const uint8_t *) (m ? L->sh_up : L->sh_gate); k.w[0] = k.sh[0];
-                k.R = H; k.K = E; k.cols = c->pcols.p; k.ncols = c->pncols.p; k.col0 = 0; k.col1 = nsh;
+                k.R = H; k.K = E; k.cols = kt.cols; k.ncols = kt.ncols; k.col0 = 0; k.col1 = nsh;
                 k.bh = c->xh.p; k.bd = c->xd.p; k.arow0 = P; k.orow0 = P; k.out = m ? c->ksu.p : c->ksg.p;
                 TRY(c, launch_kq_gemm(k, FL_Q5K, c->ncu, st));
             }
@@ -647,24 +652,24 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
             if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, st)) { return rc; }
         }
         TRY(c, launch_quant_q8k(c->h.p, (int64_t) rows, H, c->hq.p, c->hd.p, st));
-        TRY(c, launch_q8_to_h(c->hq.p, c->hh.p, (int64_t) rows * H, st));
+        if (kq) { TRY(c, launch_q8_to_h(c->hq.p, c->hh.p, (int64_t) rows * H, st)); }
         prof_mark(c, ev, 5);
         PrefillArgs d = g;   // the down pass: activations Q8_K(h) of every slot, o rows by slot
         d.w[0] = (const uint8_t *) L->down_exps; d.w[1] = nullptr; d.sh[0] = (const uint8_t *) L->sh_down; d.sh[1] = nullptr;
-        d.R = E; d.K = H; d.nmat = 1; d.bh = c->hh.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr;
+        d.R = E; d.K = H; d.nmat = 1; d.bq = c->hq.p; d.bh = c->hh.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr;
         const bool sh_iq = lf[3] == FL_IQ2, sh_kg = lf[3] == FL_Q2K || lf[3] == FL_Q3K || lf[3] == FL_Q6K;
         if (lf[0] == FL_IQ2) {   // routed (+ the shared expert when it is IQ2_XXS)
-            d.col0 = sh_iq ? 0 : nsh;
-            TRY(c, launch_prefill_gemm(d, c->ncu, st));
+            d.col0 = sh_iq ? 0 : nshi;
+            TRY(c, iq2_gemm(d, c->ncu, st));
         } else {
             PrefillArgs k = d;
-            k.estride = fmt_mat_bytes(lf[0], E, H); k.col0 = nsh;
+            k.estride = fmt_mat_bytes(lf[0], E, H); k.cols = kt.cols; k.ncols = kt.ncols; k.col0 = nsh;
             TRY(c, launch_kq_gemm(k, lf[0], c->ncu, st));
-            if (sh_iq) { d.col0 = 0; d.col1 = nsh; TRY(c, launch_prefill_gemm(d, c->ncu, st)); }
+            if (sh_iq) { d.col0 = 0; d.col1 = nshi; TRY(c, iq2_gemm(d, c->ncu, st)); }
         }
         if (sh_kg) {
             PrefillArgs k = d;
-            k.col0 = 0; k.col1 = nsh;
+            k.cols = kt.cols; k.ncols = kt.ncols; k.col0 = 0; k.col1 = nsh;
             TRY(c, launch_kq_gemm(k, lf[3], c->ncu, st));
         } else if (!sh_iq) {
             if (int rc = shared_down_sep(c, L, n, P, E, H, tk, st)) { return rc; }

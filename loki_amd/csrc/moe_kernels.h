@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stddef.h>
+#include "moe_common.h"
 
 namespace lk {
 
@@ -130,15 +131,35 @@ hipError_t decode1_init(int ncu, int * ok);
 size_t decode1_lds_bytes();
 hipError_t launch_moe_decode1(const DecodeArgs & a, bool cooperative, hipStream_t st);
 
+// Column tables. launch_prefill_cols cuts every expert's slots (the shared expert's first) into columns of at most tok
+// slots, the fewest possible and of equal size (rounded up to 16); the routed columns are ordered by class. Sized >= P /
+// tok + n / tok + NEXP_MAX + 2 entries. Classes by slots: broad 65..112, wide 33..64, narrow few + 1..32, few 1..few.
+// ncols[0] all columns; [1 + k] end of the shared columns of class k; [PF_NCLS + 1 + k] end of the routed ones.
+constexpr int PF_TOK = 112, KQ_TOK = 64, FEW_TOK = 8;   // tok of the IQ2_XXS GEMMs, the K-quant GEMM, the few kernel
+enum { PF_BROAD = 0, PF_WIDE = 1, PF_NARROW = 2, PF_FEW = 3, PF_NCLS = 4 };
+constexpr int PF_NCOLS = 2 * PF_NCLS + 1;
+struct PfTable { int4 * cols; int * ncols; int tok, few; };
+// one or two tables (t1.cols may be null)
+hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, const PfTable & t0, const PfTable & t1, hipStream_t st);
+constexpr int prefill_shared_cols(int n, int tok) { return (n + tok - 1) / tok; }   // the shared expert's columns (the first ones)
+// IQ2_XXS tables by batch size: up to PF_SPLIT_N tokens every column has at most 8 slots (launch_few_gemm alone), up to
+// PF_FEW_N the columns of at most 8 run on the few kernel, above on the narrow one
+constexpr int PF_SPLIT_N = 64, PF_FEW_N = 256;
+constexpr int pf_tok(int n) { return n <= PF_SPLIT_N ? FEW_TOK : PF_TOK; }
+constexpr int pf_few(int n) { return n <= PF_FEW_N ? FEW_TOK : 0; }
+
 // ---------------------------------------------------------------- prefill grouped GEMM on MFMA (moe_prefill.hip)
 struct PrefillArgs {
-    const uint4 * ptab;                  // fp16 table image (build_prefill_tables)
+    const uint4 * ptab;                  // digit table image (build_prefill_tables)
+    int most;                            // no expert has more slots than this (classes above it are not launched)
     const uint8_t * w[2]; size_t estride;   // routed matrices (tiled), expert e at + e * estride
     const uint8_t * sh[2];               // shared expert matrices (tiled)
     const int * perm; int topk, P;       // gate/up: slot -> token = perm[slot] / topk (shared slots P + t -> t)
     int R, K, nmat;                      // rows, columns; nmat 2 = gate/up, 1 = down
     const int4 * cols; const int * ncols;   // launch_prefill_cols
-    const _Float16 * bh; const float * bd;  // activations: Q8_K integers as fp16 [rows][K] and scales [rows][K/256]
+    const int8_t * bq; const float * bd; // activations: Q8_K integers [rows][K] and scales [rows][K/256]
+    const _Float16 * bh;                 // the integers as fp16 (launch_kq_gemm only)
+    const uint4 * tab;                   // the decode table image (build_table_image), for that kernel
     float * out;                         // gate/up: h [P+n][R] (silu(g) * u); down: o [P+n][R]
     float * gdbg, * udbg;                // optional gate / up outputs
     int * err;                           // bit 4: the LDS base is not 64 KB aligned
@@ -150,16 +171,34 @@ struct PrefillArgs {
     // read the tokens' rows and write rows 0 .. n - 1 of their own outputs)
     int arow0, orow0;
 };
+// the columns of one class inside [col0, col1): two runs [a0, a0 + na) and [b0, b0 + nb) of the column table
+struct PfRuns {
+    int a0, na, b0, nb;
+    __device__ int count() const { return na + nb; }
+    __device__ int col(int j) const { return j < na ? a0 + j : b0 + (j - na); }
+};
+__device__ __forceinline__ int pf_clip(int lo, int hi, int c0, int c1, int & start) {
+    start = lo > c0 ? lo : c0;
+    const int end = hi < c1 ? hi : c1;
+    return end > start ? end - start : 0;
+}
+__device__ __forceinline__ PfRuns pf_runs(const PrefillArgs & a, int cls) {
+    const LK_GLOBAL int * nc = gptr(a.ncols);
+    const int c0 = a.col0, c1 = a.col1 > 0 ? a.col1 : nc[0];
+    PfRuns r;
+    r.na = pf_clip(cls == 0 ? 0 : nc[cls], nc[1 + cls], c0, c1, r.a0);
+    r.nb = pf_clip(nc[PF_NCLS + cls], nc[PF_NCLS + 1 + cls], c0, c1, r.b0);
+    return r;
+}
 hipError_t prefill_init();
 size_t prefill_table_bytes();
 hipError_t build_prefill_tables(uint4 * img, hipStream_t st);
-// columns of <= 64 slots (PF_TOK) of one expert: the shared expert's ceil(n / 64) first, then act order; cols sized
-// >= prefill_shared_cols(n) + P / 64 + NEXP_MAX + 2
-constexpr int PF_NCOLS = 4;   // the counts launch_prefill_cols writes (ncols[0] = all columns; the class boundaries)
-hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, int4 * cols, int * ncols, hipStream_t st);
-int prefill_shared_cols(int n);   // the shared expert's columns (the first ones) for n tokens
 hipError_t launch_q8_to_h(const int8_t * q, _Float16 * h, int64_t n, hipStream_t st);
+// every column of a.cols in [col0, col1), each on the kernel of its class
 hipError_t launch_prefill_gemm(const PrefillArgs & a, int grid, hipStream_t st);
+// the columns of few slots only (moe_few.hip)
+hipError_t few_init();
+hipError_t launch_few_gemm(const PrefillArgs & a, int grid, hipStream_t st);
 
 // K-quant matrices on the matrix cores (kq_gemm.hip), bit-identical to launch_kq_matvec: columns col0 .. col1 - 1 of
 // launch_prefill_cols (routed: expert e at w[0] + e * estride; the shared expert's: sh[0]), ggml's blocks read in

@@ -2,27 +2,27 @@
 //
 // Reference: fl_wide_moe (src/fused_layer.cu:540-561) runs tc_matvec<F_IQ2> (:178-202) per arena batch of <= 72 slots
 // of <= 8 rows each with mma.m16n8k32 s8 tiles, then swiglu_q8 (:334-341) and the down pass; the semantics are ggml's
-// mul_mat_id over IQ2_XXS x Q8_K (ggml_vec_dot_iq2_xxs_q8_K per output). Here one launch covers every expert of the
-// layer:
-//   * A column is up to 64 dispatch slots (PF_TOK) of one expert (the shared expert's slots P .. P + n - 1 included); an item is
-//     (column, 256 or 512 rows). The workgroups (one per CU: the tables fill most of the LDS) take the items round-robin.
-//   * The weights are dequantised once per item into fp16 MFMA operands: lane (r, g) of a wave owns row r of a 16-row
-//     tile and the 16-byte chunk g of each block (sub-blocks 2g, 2g + 1, both with their scale nibbles), so it builds
-//     w = sign * grid * (2 nibble + 1) from two replicated LDS tables (fp16 codebook words, fp16 sign masks) and one
-//     packed fp16 multiply per two weights. Every w is an integer of magnitude <= 43 * 31, exact in fp16.
-//   * The column's activations (the Q8_K integers as fp16, exact) are copied block by block into LDS with direct
-//     global->LDS loads, double-buffered; v_mfma_f32_16x16x32_f16 then forms, per 256-value block, the block sum
-//     bsum = sum_ib (2 s_ib + 1) sum_k g s q over a 16-token x 16-row tile, as two chains of four MFMA steps: steps
-//     0-3 cover sub-blocks 0, 2, 4, 6 (one per lane group) and steps 4-7 the odd ones. No codebook entry's 8 bytes
-//     sum above 203, so a chain's products and every partial sum are integers of magnitude at most
-//     16 * 203 * 31 * 127 = 12,787,376 < 2^24: each chain total is exact, whatever order the matrix core adds in. The
-//     block sum is then one fp32 addition of the two exact totals, i.e. the exact integer rounded to nearest even --
-//     exactly ggml's (float) of its int32 block sum, also where |bsum| exceeds 2^24 (up to 25.6 M).
+// mul_mat_id over IQ2_XXS x Q8_K (ggml_vec_dot_iq2_xxs_q8_K per output). Here one launch per class of columns covers
+// every expert of the layer:
+//   * A column is up to PF_TOK = 112 dispatch slots of one expert (the shared expert's slots P .. P + n - 1 included); an
+//     item is (column, row group). The workgroups (one per CU: the tables fill most of the LDS) take the items
+//     round-robin.
+//   * The weights are dequantised once per item into int8 MFMA operands. A scaled weight v = sign * grid * (2s + 1) is one
+//     of 6 values per sub-block (three magnitudes, two signs) and has at most 11 bits, so it is taken as two int8 digits,
+//     v = 64 h + l, |l| <= 32, |h| <= 21. The codebook table holds, per entry, 8 selector bytes (the magnitude's index
+//     0..2), the sign table 8 bytes of 0 or 4; or-ed they select, with one v_perm_b32 per 4 weights and digit, among the 8
+//     bytes of the sub-block's scale line (the digits of +-8, +-25, +-43 times 2s + 1, a 16-byte LDS line per scale
+//     nibble). Lane (r, g) of a wave owns row r of a 16-row tile and the 16-byte chunk g of each block (sub-blocks 2g,
+//     2g + 1), as the tiled layout stores them.
+//   * The column's activations (the Q8_K bytes) are copied block by block into LDS with direct global->LDS loads,
+//     double-buffered; v_mfma_i32_16x16x64_i8 forms, per 256-value block and digit, the exact int32 sum over a 16-token x
+//     16-row tile (4 steps), and the block sum is 64 h + l in int32, converted to fp32 once (rounded to nearest even):
+//     ggml's (float) of its int32 block sum.
 //   * Each output then advances in block order, y += (d_w * d_x) * bsum, and ends * 0.125: the fp32 operations and their
 //     order are those of ggml_vec_dot_iq2_xxs_q8_K, so every output is bit-identical to the CPU checker's.
 //   * Gate/up tiles write h = silu(g) * u per slot; down tiles write o per slot (the combine runs after).
-// The K index of an MFMA step is permuted consistently in both operands: step t of lane group g covers the 8 values
-// 64 g + 8 t .. + 7 of the block, i.e. entry t % 4 of sub-block 2 g + t / 4, which is what the lane's chunk holds.
+// The K index of an MFMA step is permuted consistently in both operands: step m of lane group g covers the 16 values
+// 64 g + 16 m .. + 15 of the block, i.e. entries 2 (m % 2), 2 (m % 2) + 1 of sub-block 2 g + m / 2.
 #include "moe_device.h"
 #include "moe_kernels.h"
 #include <type_traits>
@@ -30,74 +30,96 @@
 namespace lk {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef int i4 __attribute__((ext_vector_type(4)));
 
-constexpr int PF_NTM = 4;                    // 16-token MFMA tiles per column at most
-constexpr int PF_TOK = 16 * PF_NTM;          // slots per column: the dequantised weights of an item serve all of them
-// LDS: fp16 codebook (256 lines x 16 copies x 16 B), fp16 sign masks (128 lines, the 7 stored sign bits), then two
-// activation buffers (up to 64 token rows x 512 B, each row's 16-byte chunks XOR-swizzled by the row; the wide kernel's
-// fill the 160 KB exactly), then (narrow gate/up) the exchange of g. The tokens' block scales stay in registers (one per
-// lane, handed to the lanes that fold them by ds_bpermute).
-constexpr int L_PG = 0, L_PS = 65536, L_PB = L_PS + 128 * 256;
-constexpr int PB_TILE = 16 * 512;            // one 16-token tile of a buffer (512-byte aligned)
-constexpr int PTAB_BYTES = L_PB;             // the table image copied to LDS offset 0
+// Table image: selector lines (entry e: 32 copies of the 8 magnitude indices of grid[e]), sign lines (the 7 stored sign
+// bits: 32 copies of 8 bytes 0 / 4), then the 16 scale lines {l of + magnitudes, l of -, h of +, h of -} (bytes 0..2).
+// LDS: the tables, two buffers of the tokens' block scales, two activation buffers (16 NTM token rows of 256 bytes, each
+// row's 16-byte chunks XOR-swizzled by the row).
+constexpr int L_SEL = 0, L_SGN = 65536, L_SCL = TAB_BYTES, PTAB_BYTES = L_SCL + 256;
+constexpr int L_DX = PTAB_BYTES;
+static_assert(TAB_BYTES == L_SGN + 128 * 256, "the selector and sign lines have the decode image's geometry");
 
-// fp16 table image: line e of the codebook = 16 copies of the 8 fp16 values of grid[e]; line b of the signs = 16
-// copies of 8 fp16 sign masks (0x8000 for a negative weight) of the stored sign bits b (0..127) plus parity
 __global__ void k_ptab_image(uint32_t * img) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;   // dword index
     if (i >= PTAB_BYTES / 4) { return; }
-    const int line = (i * 4) >> 8, word = i & 3;            // 16 B entry copies: the dword inside the entry
-    uint32_t v;
-    if (i * 4 < L_PS) {
+    const int at = i * 4, line = at >> 8, half = i & 1;
+    uint32_t v = 0;
+    if (at < L_SGN) {
         const uint64_t gv = g_iq2xxs_grid[line];
-        const uint32_t b0 = (uint32_t) (gv >> (16 * word)) & 255u, b1 = (uint32_t) (gv >> (16 * word + 8)) & 255u;
-        v = (uint32_t) __half_as_ushort(__float2half((float) b0)) | ((uint32_t) __half_as_ushort(__float2half((float) b1)) << 16);
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t b = (uint32_t) (gv >> (32 * half + 8 * k)) & 255u;
+            v |= (b == 8 ? 0u : b == 25 ? 1u : 2u) << (8 * k);
+        }
+    } else if (at < L_SCL) {
+        const uint32_t s8 = ksigns8((uint32_t) (line - L_SGN / 256));
+        for (int k = 0; k < 4; ++k) { v |= ((s8 >> (4 * half + k)) & 1u) << (8 * k + 2); }
     } else {
-        const uint32_t s8 = ksigns8((uint32_t) (line - L_PS / 256));
-        v = (((s8 >> (2 * word)) & 1u) << 15) | (((s8 >> (2 * word + 1)) & 1u) << 31);
+        const int s = (at - L_SCL) >> 4, word = i & 3, mags[3] = { 8, 25, 43 };
+        for (int k = 0; k < 3; ++k) {
+            const int m = mags[k] * (2 * s + 1), h = (m + 32) >> 6, l = m - 64 * h;
+            const int d = word < 2 ? l : h;
+            v |= ((uint32_t) ((word & 1) ? -d : d) & 255u) << (8 * k);
+        }
     }
     img[i] = v;
 }
 hipError_t build_prefill_tables(uint4 * img, hipStream_t st) {
-    k_ptab_image<<<PTAB_BYTES / 4 / 256, 256, 0, st>>>(reinterpret_cast<uint32_t *>(img));
+    k_ptab_image<<<(PTAB_BYTES / 4 + 255) / 256, 256, 0, st>>>(reinterpret_cast<uint32_t *>(img));
     return hipGetLastError();
 }
 size_t prefill_table_bytes() { return PTAB_BYTES; }
 
-// Columns: the shared expert's slots first (P + 64 c ..), then every active expert's slots, 64 per column. A column of
-// at most 32 slots is narrow (the narrow GEMM takes it), every other one wide; only an expert's last column can be
-// narrow. Order: the shared expert's columns (its last one the only narrow one), then the routed wide columns in act
-// order, then the routed narrow columns in act order, so each class is at most two runs: ncols[0] = all columns,
-// ncols[1] = the shared wide columns, ncols[2] = the shared columns, ncols[3] = the end of the routed wide ones.
+// Columns: the shared expert's slots first, then every active expert's slots. An expert's slots go into the fewest columns
+// of at most tok slots, of equal size rounded up to 16 (the last one takes the rest). The routed columns are written class
+// by class, each in act order. Block b writes table b.
 __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, const int * __restrict__ nact_p, const int * __restrict__ offsets,
-                                                int n, int P, int4 * __restrict__ cols, int * __restrict__ ncols) {
-    __shared__ int scw[256], scn[256];
-    const int i = threadIdx.x, nact = *nact_p, nsh = (n + PF_TOK - 1) / PF_TOK;
-    int e = 0, s0 = 0, cnt = 0;
+                                                int n, int P, const PfTable t0, const PfTable t1) {
+    __shared__ int sc[PF_NCLS][256];
+    const PfTable T = blockIdx.x ? t1 : t0;
+    const int i = threadIdx.x, nact = *nact_p;
+    auto cls = [&](int slots) -> int { return slots > 64 ? PF_BROAD : slots > 32 ? PF_WIDE : slots > T.few ? PF_NARROW : PF_FEW; };
+    auto cut = [&](int cnt, int & cols, int & size) {   // cols columns of size slots, the last one the rest
+        cols = (cnt + T.tok - 1) / T.tok;
+        size = cols > 0 ? min(T.tok, ((cnt + cols - 1) / cols + 15) / 16 * 16) : 0;
+    };
+    int e = 0, s0 = 0, cnt = 0, cols, size;
     if (i < nact) { e = act[i]; s0 = offsets[e]; cnt = offsets[e + 1] - s0; }
-    const int rem = cnt % PF_TOK, nw = cnt / PF_TOK + (rem > PF_TOK / 2 ? 1 : 0), nn = rem > 0 && rem <= PF_TOK / 2 ? 1 : 0;
-    scw[i] = nw; scn[i] = nn;
+    cut(cnt, cols, size);
+    int nk[PF_NCLS] = { 0, 0, 0, 0 };                   // this expert's columns of each class
+    if (cols > 0) { nk[cls(size)] += cols - 1; nk[cls(cnt - size * (cols - 1))] += 1; }
+    for (int k = 0; k < PF_NCLS; ++k) { sc[k][i] = nk[k]; }
     __syncthreads();
     for (int off = 1; off < 256; off <<= 1) {   // inclusive scans
-        const int vw = i >= off ? scw[i - off] : 0, vn = i >= off ? scn[i - off] : 0;
+        int v[PF_NCLS];
+        for (int k = 0; k < PF_NCLS; ++k) { v[k] = i >= off ? sc[k][i - off] : 0; }
         __syncthreads();
-        scw[i] += vw; scn[i] += vn;
+        for (int k = 0; k < PF_NCLS; ++k) { sc[k][i] += v[k]; }
         __syncthreads();
     }
-    const int tw = scw[255], bw = nsh + scw[i] - nw, bn = nsh + tw + scn[i] - nn;
-    for (int c = 0; c < nw; ++c) { cols[bw + c] = make_int4(i, s0 + PF_TOK * c, min(PF_TOK, cnt - PF_TOK * c), e); }
-    if (nn) { cols[bn] = make_int4(i, s0 + cnt - rem, rem, e); }
-    for (int c = i; c < nsh; c += 256) { cols[c] = make_int4(-1, P + PF_TOK * c, min(PF_TOK, n - PF_TOK * c), 0); }
-    if (i == 255) {
-        const int rs = n % PF_TOK;
-        ncols[0] = nsh + tw + scn[255]; ncols[1] = nsh - (rs > 0 && rs <= PF_TOK / 2 ? 1 : 0); ncols[2] = nsh; ncols[3] = nsh + tw;
+    int nsh, ssize;
+    cut(n, nsh, ssize);
+    int at[PF_NCLS], end = nsh;
+    for (int k = 0; k < PF_NCLS; ++k) {
+        at[k] = end + sc[k][i] - nk[k];
+        end += sc[k][255];
+        if (i == 0) { T.ncols[PF_NCLS + 1 + k] = end; }
+    }
+    for (int c = 0; c < cols; ++c) {
+        const int m = c < cols - 1 ? size : cnt - size * c;
+        T.cols[at[cls(m)]++] = make_int4(i, s0 + size * c, m, e);
+    }
+    for (int c = i; c < nsh; c += 256) { T.cols[c] = make_int4(-1, P + ssize * c, min(ssize, n - ssize * c), 0); }
+    if (i == 0) {
+        T.ncols[0] = end;
+        int ns[PF_NCLS] = { 0, 0, 0, 0 }, at2 = 0;
+        if (nsh > 0) { ns[cls(ssize)] += nsh - 1; ns[cls(n - ssize * (nsh - 1))] += 1; }
+        for (int k = 0; k < PF_NCLS; ++k) { at2 += ns[k]; T.ncols[1 + k] = at2; }
     }
 }
-int prefill_shared_cols(int n) { return (n + PF_TOK - 1) / PF_TOK; }
-hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, int4 * cols, int * ncols, hipStream_t st) {
-    k_pf_cols<<<1, 256, 0, st>>>(act, nact, offsets, n, P, cols, ncols);
+hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, const PfTable & t0, const PfTable & t1, hipStream_t st) {
+    k_pf_cols<<<t1.cols ? 2 : 1, 256, 0, st>>>(act, nact, offsets, n, P, t0, t1);
     return hipGetLastError();
 }
 
@@ -120,35 +142,26 @@ hipError_t launch_q8_to_h(const int8_t * q, _Float16 * h, int64_t n, hipStream_t
 
 // ---------------------------------------------------------------- the grouped GEMM
 // NMAT = 2: gate/up (K = 7168, rows 2048, B rows = tokens, writes h); NMAT = 1: down (K = 2048, rows 7168, B rows =
-// slots, writes o). Two kernels take the columns of launch_prefill_cols by class:
-//   * wide (W = 8 waves, CPW = 2 16-row tiles per wave, columns of 33-64 slots, up to 4 token tiles): a wave's tiles
-//     are the gate and up rows of one 16-row tile (gate/up: h forms in registers) or two row tiles (down);
-//   * narrow (W = 16 waves, CPW = 1, columns of at most 32 slots, up to 2 token tiles): about half the registers per
-//     wave, so four waves share a SIMD and hide more of the LDS read -> dequantise -> MFMA chain; gate/up hands g to
-//     the up waves through LDS.
-// Either way an item is (column, row group) and every output is computed once, in the same arithmetic.
-template <int NMAT, int NB, int W, int CPW>
+// slots, writes o). W waves per workgroup, C 16-row tiles per wave, columns of at most 16 NTM slots:
+//   * narrow (W 16, C 2, NTM 2): columns of at most 32 slots, four waves per SIMD;
+//   * wide (W 8, C 2, NTM 4): 33..64 slots;
+//   * broad (W 8, C 1, NTM 7): 65..112 slots, the dequantised weights of a tile serve up to seven token tiles.
+// With C = 2 a wave's tiles are the gate and up rows of one 16-row tile (gate/up: h forms in registers) or two row tiles
+// (down); with C = 1 the gate waves hand g to the up waves through LDS. Every output is computed once, in the same
+// arithmetic.
+template <int NMAT, int NB, int W, int C, int NTM>
 struct PfGeo {
-    static constexpr bool NARROW = CPW == 1;
-    static constexpr int NTM = NARROW ? 2 : PF_NTM;             // token tiles per column at most
-    static constexpr int TPM = W * CPW / NMAT;                  // 16-row tiles per matrix in an item
-    static constexpr int ROWS = TPM * 16, K = NB * QK, NTH = W * 64;
-    static constexpr int BUF = NTM * PB_TILE;                   // one activation buffer
-    static constexpr int L_G = L_PB + 2 * BUF;                  // narrow gate/up: g of the gate waves [8][64 lanes][2 tiles][4]
-    static constexpr int LDS = L_G + (NARROW && NMAT == 2 ? 8 * 64 * NTM * 16 : 0);
-    static_assert(LDS <= 160 * 1024 && W * CPW % NMAT == 0, "prefill GEMM geometry");
+    static constexpr int TPM = W * C / NMAT;                    // 16-row tiles per matrix in an item
+    static constexpr int ROWS = TPM * 16, K = NB * QK;
+    static constexpr int BUF = NTM * 16 * QK;                   // one activation buffer
+    static constexpr int DXB = (NTM + 3) / 4 * 256;             // one buffer of block scales (64 tokens per copy)
+    static constexpr int L_X = (L_DX + 2 * DXB + 1023) / 1024 * 1024, LDS = L_X + 2 * BUF;
+    static constexpr bool XG = NMAT == 2 && C == 1;             // g goes through LDS (the second activation buffer)
+    static_assert(LDS <= 160 * 1024 && W * C % NMAT == 0 && C <= 2 && (!XG || W / 2 * 64 * NTM * 16 <= BUF), "prefill GEMM geometry");
     // the matrix and the 16-row tile (within the item) of combo c of wave w
-    __device__ static constexpr int mat(int w, int c) { return CPW == NMAT ? c : NMAT == 1 ? 0 : w / (W / NMAT); }
-    __device__ static constexpr int tile(int w, int c) { return CPW == NMAT ? w : NMAT == 1 ? w * CPW + c : w % (W / NMAT); }
+    __device__ static constexpr int mat(int w, int c) { return C == NMAT ? c : NMAT == 1 ? 0 : w / (W / NMAT); }
+    __device__ static constexpr int tile(int w, int c) { return C == NMAT ? w : NMAT == 1 ? w * C + c : w % (W / NMAT); }
 };
-
-struct PfLane {
-    int r, g;                 // row (token) in a 16-tile, chunk / lane group
-    uint32_t trg, trs;        // table addresses with this lane's copy
-};
-
-// activation rows in LDS: see pf_swz (moe_common.h); lane (r, g)'s chunk 8 g + t sits at slot (8 pf_swz2(g) + t) ^ r
-__device__ __forceinline__ int pf_swz2(int g) { return ((g & 1) << 1) | (g >> 1); }
 
 // one block of one 16-row tile: the tiled chunk g of row r (qs) and d
 struct PfW { u32x4 q; uint16_t d; };
@@ -165,48 +178,27 @@ __device__ __forceinline__ const uint8_t * pf_uniform(const uint8_t * p) {
     return (const uint8_t *) (((uint64_t) hi << 32) | (uint64_t) lo);
 }
 
-// 16 bytes per lane from a buffer straight into LDS (lane L at dst + 16 L); the builtin exists for the device pass only,
+// SZ bytes per lane from a buffer straight into LDS (lane L at dst + SZ L); the builtin exists for the device pass only,
 // so the host pass (which instantiates the kernel's launch stub) sees an empty body
-__device__ __forceinline__ void buf_lds16(__amdgpu_buffer_rsrc_t r, LK_LOCAL uint8_t * dst, uint32_t voff, uint32_t soff) {
+template <int SZ> __device__ __forceinline__ void buf_lds(__amdgpu_buffer_rsrc_t r, LK_LOCAL uint8_t * dst, uint32_t voff, uint32_t soff) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 16, voff, soff, 0, 0);
+    if constexpr (SZ == 16) { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 16, voff, soff, 0, 0); }
+    else { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 4, voff, soff, 0, 0); }
 #else
     (void) r; (void) dst; (void) voff; (void) soff;
 #endif
 }
-__device__ __forceinline__ void dma16(const void * src, LK_LOCAL uint8_t * dst) {
-    __builtin_amdgcn_global_load_lds((const LK_GLOBAL void *) src, (LK_LOCAL void *) dst, 16, 0, 0);
-}
 
-// the columns of one class inside [col0, col1): two runs [a0, a1) and [b0, b1) of the column table (k_pf_cols' order)
-struct PfRuns {
-    int a0, na, b0, nb;
-    __device__ int count() const { return na + nb; }
-    __device__ int col(int j) const { return j < na ? a0 + j : b0 + (j - na); }
-};
-__device__ __forceinline__ int pf_clip(int lo, int hi, int c0, int c1, int & start) {
-    start = lo > c0 ? lo : c0;
-    const int end = hi < c1 ? hi : c1;
-    return end > start ? end - start : 0;
-}
-template <bool NARROW>
-__device__ __forceinline__ PfRuns pf_runs(const PrefillArgs & a) {
-    const int total = gptr(a.ncols)[0], shw = gptr(a.ncols)[1], sh = gptr(a.ncols)[2], rw = gptr(a.ncols)[3];
-    const int c0 = a.col0, c1 = a.col1 > 0 ? a.col1 : total;
-    PfRuns r;
-    if (NARROW) { r.na = pf_clip(shw, sh, c0, c1, r.a0); r.nb = pf_clip(rw, total, c0, c1, r.b0); }
-    else { r.na = pf_clip(0, shw, c0, c1, r.a0); r.nb = pf_clip(sh, rw, c0, c1, r.b0); }
-    return r;
-}
-
-template <int NMAT, int NB, int W, int CPW>
+template <int NMAT, int NB, int W, int C, int NTM, int CLS>
 __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
 #pragma clang fp contract(off)
-    using Geo = PfGeo<NMAT, NB, W, CPW>;
-    constexpr int C = CPW;
+    using Geo = PfGeo<NMAT, NB, W, C, NTM>;
     extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
     LK_LOCAL uint8_t * lds = (LK_LOCAL uint8_t *) dyn_lds;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+    const PfRuns runs = pf_runs(a, CLS);
+    const int nrg = a.R / Geo::ROWS;
+    if ((int) blockIdx.x >= runs.count() * nrg) { return; }   // nothing to do: not even the tables
     if (lds_addr(dyn_lds) & 0xFFFFu) {   // table addressing needs a 64 KB aligned base
         if (threadIdx.x == 0) {
             __hip_atomic_fetch_or(gptr(a.err), 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -214,16 +206,11 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
         }
         return;
     }
-    // tables into LDS (direct loads), visible after vmcnt(0) + the first barrier
-    for (int c = wave; c < PTAB_BYTES / 1024; c += W) { dma16(a.ptab + c * 64 + lane, lds + c * 1024); }
-    PfLane ln;
-    ln.r = lane & 15; ln.g = lane >> 4;
-    ln.trg = (uint32_t) L_PG | ((uint32_t) ln.r << 4);
-    ln.trs = (uint32_t) L_PS | ((uint32_t) ln.r << 4);
-    const PfRuns runs = pf_runs<Geo::NARROW>(a);
-    const int nrg = a.R / Geo::ROWS;
+    tables_fill(reinterpret_cast<const uint8_t *>(a.ptab), lds, threadIdx.x, W * 64);
+    if (threadIdx.x < 16) { reinterpret_cast<LK_LOCAL u32x4 *>(lds + L_SCL)[threadIdx.x] = *(const LK_GLOBAL u32x4 *) (a.ptab + L_SCL / 16 + threadIdx.x); }
+    const int r = lane & 15, g = lane >> 4;
+    const uint32_t trg = (uint32_t) L_SEL | ((uint32_t) (lane & 31) << 3), trs = trg + (uint32_t) L_SGN;
     const size_t dreg = (size_t) (a.R / 64) * NB * 4096;   // d region offset of a tiled matrix
-    __builtin_amdgcn_s_waitcnt(0x0f70);
     __syncthreads();
 
     for (int it = blockIdx.x; it < runs.count() * nrg; it += gridDim.x) {
@@ -232,15 +219,13 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
         const int4 cd = make_int4((int) cv.x, (int) cv.y, (int) cv.z, (int) cv.w);
         const bool routed = cd.x >= 0;
         const int sb = cd.y, sc = cd.z;
-        // B rows of the copy instructions: instruction i copies rows 2 i and 2 i + 1 (lane half L >> 5)
-        auto brow = [&](int n32) -> int {
-            const int s = sb + (n32 < sc ? n32 : 0);
+        auto brow = [&](int t) -> int {   // activation row of token t of the column
+            const int s = sb + (t < sc ? t : 0);
             return NMAT == 2 ? (routed ? gptr(a.perm)[s] / a.topk : s - a.P) : s;
         };
         // Buffer loads: a scalar resource (base, no bounds that matter) + a 32-bit lane offset + a scalar block offset,
         // so no 64-bit per-lane address lives in vector registers.
-        const __amdgpu_buffer_rsrc_t rb = pf_rsrc(a.bh), rd = pf_rsrc(a.bd);
-        const uint32_t oX = (uint32_t) brow(lane) * (NB * 4);   // lane n loads the scale of token n of the column
+        const __amdgpu_buffer_rsrc_t rb = pf_rsrc(a.bq), rd = pf_rsrc(a.bd);
         // the wave's tiles: combo c = (matrix Geo::mat, 16-row tile Geo::tile): scalar resources at the tile's qs / d
         // bases, the lane's offset (chunk g of row r) in one vector register
         __amdgpu_buffer_rsrc_t uq[C], ud[C];
@@ -253,7 +238,7 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
             uq[c] = pf_rsrc(pf_uniform(Wm + (size_t) g64 * NB * 4096 + r0 * 16));
             ud[c] = pf_rsrc(pf_uniform(Wm + dreg + (size_t) g64 * NB * 128 + r0 * 2));
         }
-        const uint32_t lq = (uint32_t) ln.g * 1024 + (uint32_t) ln.r * 16, ldo = (uint32_t) ln.r * 2;
+        const uint32_t lq = (uint32_t) g * 1024 + (uint32_t) r * 16, ldo = (uint32_t) r * 2;
         auto load_w = [&](int j, PfW (&w)[C]) {
 #pragma unroll
             for (int c = 0; c < C; ++c) {
@@ -262,206 +247,174 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
             }
         };
         auto run_item = [&](auto ntc) {
-            constexpr int NT = decltype(ntc)::value;   // token tiles of the column (1, 2 or 4)
+            constexpr int NT = decltype(ntc)::value;   // token tiles of the column
             // the column's activations of block j go straight from memory into LDS buffer j % 2 (buffer loads to LDS:
             // lane L's 16 bytes land at L * 16 of the instruction's 1 KB, no registers): copy instruction i covers token
-            // rows 2 i + (lane / 32), i < 8 NT, taken by waves i % W; lane L < 32 of a row takes the row's chunk
-            // pf_swz(L ^ (row % 16)) -- the swizzle applied on the memory side. Lane n also loads token n's block scale
-            // into a register.
-            constexpr int NI = (8 * NT + W - 1) / W;   // copy instructions per wave (some waves of the narrow kernel none)
-            struct PfB { float dx; };
-            uint32_t ob[NI];
+            // rows 4 i .. 4 i + 3, i < 4 NT, taken by waves i % W; lane L of row (L / 16) takes the row's chunk
+            // (L % 16) ^ (row % 16) -- the swizzle applied on the memory side. gfx950 serves a ds_read_b128 in four passes
+            // of 16 lanes (equal bit 5, equal bit 4 ^ bit 3); lane (r, g) reads slot (4 g + m) ^ r of row r, so a pass holds
+            // 16 different slots. The tokens' block scales follow, 64 tokens per instruction (waves W - 1, W - 2).
+            constexpr int NI = (4 * NT + W - 1) / W, ND = (NT + 3) / 4;
+            uint32_t ob[NI], od = 0;
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
-                const int row = 2 * (wave + W * i) + (lane >> 5);
-                ob[i] = (uint32_t) brow(row < 16 * NT ? row : 0) * (Geo::K * 2) + pf_swz((uint32_t) ((lane & 31) ^ (row & 15))) * 16;
+                const int row = 4 * (wave + W * i) + (lane >> 4);
+                ob[i] = (uint32_t) brow(row < 16 * NT ? row : 0) * Geo::K + (uint32_t) (((lane & 15) ^ (row & 15)) << 4);
             }
-            auto load_b = [&](int j, PfB & bq, int buf) {
-                LK_LOCAL uint8_t * dst = lds + L_PB + buf * Geo::BUF;
+            const int dw0 = W - 1 - wave;   // which 64 tokens' scales this wave copies (0 .. ND - 1)
+            if (dw0 < ND) { od = (uint32_t) brow(64 * dw0 + lane) * (NB * 4); }
+            auto load_b = [&](int j, int buf) {
+                LK_LOCAL uint8_t * dst = lds + Geo::L_X + buf * Geo::BUF;
 #pragma unroll
                 for (int i = 0; i < NI; ++i) {
-                    if (wave + W * i < 8 * NT) { buf_lds16(rb, dst + 2 * (wave + W * i) * 512, ob[i], j * (QK * 2)); }
+                    if (wave + W * i < 4 * NT) { buf_lds<16>(rb, dst + (wave + W * i) * 1024, ob[i], j * QK); }
                 }
-                bq.dx = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, oX, j * 4, 0));
+                if (dw0 < ND) { buf_lds<4>(rd, lds + L_DX + buf * Geo::DXB + dw0 * 256, od, j * 4); }
             };
             f4 acc[C][NT];
 #pragma unroll
             for (int c = 0; c < C; ++c) { for (int tt = 0; tt < NT; ++tt) { acc[c][tt] = (f4) { 0.f, 0.f, 0.f, 0.f }; } }
 
             // one block: dequantise the C tiles step by step and run the MFMA chains of the token tiles
-            auto block = [&](int j, const PfW (&w)[C], int buf, float dxl) {
-                static_assert((L_PB % 512) == 0 && (Geo::BUF % 512) == 0, "XOR addressing inside 512-byte rows");
-                const uint32_t bx = ((uint32_t) (L_PB + buf * Geo::BUF) + (uint32_t) ln.r * 512) | ((uint32_t) ((8 * pf_swz2(ln.g)) ^ ln.r) << 4);
-                f4 cc[C][NT], cd[C][NT];   // the two exact chains: steps 0-3, steps 4-7
-                h2v sc[C][2];
+            auto block = [&](const PfW (&w)[C], int buf) {
+                const uint32_t bx = (uint32_t) (Geo::L_X + buf * Geo::BUF) + (uint32_t) r * QK + (uint32_t) (((4 * g) ^ r) << 4);
+                i4 D[C][NT][2];         // per tile pair: the sums of the low and of the high digits
+                u32x4 dig[C];           // the scale line of the lane's sub-block in use (2 g, then 2 g + 1)
                 uint32_t ms[C][2];
+                auto digits = [&](int c, int h) {
+                    const uint32_t sw = h ? w[c].q.w : w[c].q.y;
+                    dig[c] = *(const LK_LOCAL u32x4 *) (size_t) __builtin_amdgcn_udot4((sw >> 7) & 0x01010101u, 0x80402010u, (uint32_t) L_SCL, false);
+                };
 #pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    const _Float16 s0 = (_Float16) iq2_scale(w[c].q.y), s1 = (_Float16) iq2_scale(w[c].q.w);
-                    sc[c][0] = (h2v) { s0, s0 }; sc[c][1] = (h2v) { s1, s1 };
-                    ms[c][0] = w[c].q.y & 0x7f7f7f7fu; ms[c][1] = w[c].q.w & 0x7f7f7f7fu;
-                }
-                // step t's LDS reads (the activation chunks, per tile a codebook and a sign entry) are issued one step
-                // ahead of their use, into the other of two register sets
-                struct Lk { u32x4 g[C], s[C]; h8 x[NT]; };
-                auto lookup = [&](int t, Lk & k) {
-                    const uint32_t bo = bx ^ ((uint32_t) t << 4);   // chunk (8 g + t) ^ r of the lane's token row
+                for (int c = 0; c < C; ++c) { digits(c, 0); ms[c][0] = w[c].q.y & SIGN_BITS; ms[c][1] = w[c].q.w & SIGN_BITS; }
+                // Steps (m, c), m outer. The LDS reads of a step (the tile's two selector and sign entries; at the first
+                // tile of an m the activation chunks) are issued one step ahead of their use, into the other of two
+                // register sets, so their latency runs under the step's dequantisation and MFMAs.
+                struct Lk { uint2 g0, g1, s0, s1; };
+                auto operand = [&](int m, i4 (&x)[NT]) {
+                    const uint32_t bo = bx ^ ((uint32_t) m << 4);   // chunk (4 g + m) ^ r of the lane's token row
 #pragma unroll
-                    for (int tt = 0; tt < NT; ++tt) { k.x[tt] = __builtin_bit_cast(h8, *(const LK_LOCAL u32x4 *) (size_t) (bo + tt * PB_TILE)); }
-#pragma unroll
-                    for (int c = 0; c < C; ++c) {
-                        const uint32_t a0 = t < 4 ? w[c].q.x : w[c].q.z, a1 = ms[c][t >> 2];
-                        uint32_t ga, sa;
-                        switch (t & 3) {
-                        case 0: ga = tab_addr<0>(a0, ln.trg); sa = tab_addr<0>(a1, ln.trs); break;
-                        case 1: ga = tab_addr<1>(a0, ln.trg); sa = tab_addr<1>(a1, ln.trs); break;
-                        case 2: ga = tab_addr<2>(a0, ln.trg); sa = tab_addr<2>(a1, ln.trs); break;
-                        default: ga = tab_addr<3>(a0, ln.trg); sa = tab_addr<3>(a1, ln.trs); break;
-                        }
-                        k.g[c] = *(const LK_LOCAL u32x4 *) (size_t) ga;
-                        k.s[c] = *(const LK_LOCAL u32x4 *) (size_t) sa;
+                    for (int tt = 0; tt < NT; ++tt) { x[tt] = __builtin_bit_cast(i4, *(const LK_LOCAL u32x4 *) (size_t) (bo + tt * 16 * QK)); }
+                };
+                auto lookup = [&](int m, int c, Lk & k) {
+                    const uint32_t a0 = m < 2 ? w[c].q.x : w[c].q.z, a1 = ms[c][m >> 1];
+                    if (m & 1) {
+                        k.g0 = lload8(tab_addr<2>(a0, trg)); k.g1 = lload8(tab_addr<3>(a0, trg));
+                        k.s0 = lload8(tab_addr<2>(a1, trs)); k.s1 = lload8(tab_addr<3>(a1, trs));
+                    } else {
+                        k.g0 = lload8(tab_addr<0>(a0, trg)); k.g1 = lload8(tab_addr<1>(a0, trg));
+                        k.s0 = lload8(tab_addr<0>(a1, trs)); k.s1 = lload8(tab_addr<1>(a1, trs));
                     }
                 };
-                auto compute = [&](int t, const Lk & k) {
+                Lk k[2];
+                i4 x[2][NT];
+                operand(0, x[0]);
+                lookup(0, 0, k[0]);
 #pragma unroll
-                    for (int c = 0; c < C; ++c) {
-                        const h8 gs = __builtin_bit_cast(h8, k.g[c] ^ k.s[c]);
-                        const h2v s = sc[c][t >> 2];
-                        const h8 wv = gs * (h8) { s[0], s[1], s[0], s[1], s[0], s[1], s[0], s[1] };
-                        const f4 z = (f4) { 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-                        for (int tt = 0; tt < NT; ++tt) {
-                            if (t < 4) {
-                                cc[c][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k.x[tt], wv, t == 0 ? z : cc[c][tt], 0, 0, 0);
-                            } else {
-                                cd[c][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k.x[tt], wv, t == 4 ? z : cd[c][tt], 0, 0, 0);
-                            }
-                        }
+                for (int i = 0; i < 4 * C; ++i) {
+                    const int m = i / C, c = i % C;
+                    if (i + 1 < 4 * C) {
+                        if (c == C - 1) { operand(m + 1, x[(m + 1) & 1]); }
+                        lookup((i + 1) / C, (i + 1) % C, k[(i + 1) & 1]);
                     }
-                };
-                if constexpr (C * NT <= 4) {   // two register sets: step t + 1's reads issued before step t's MFMAs
-                    Lk ka, kb;
-                    lookup(0, ka);
+                    const Lk & u = k[i & 1];
+                    const uint32_t e[4] = { u.g0.x | u.s0.x, u.g0.y | u.s0.y, u.g1.x | u.s1.x, u.g1.y | u.s1.y };
+                    const u32x4 d = dig[c];
+                    i4 wl, wh;
 #pragma unroll
-                    for (int t = 0; t < 8; t += 2) {
-                        lookup(t + 1, kb);
-                        compute(t, ka);
-                        if (t + 2 < 8) { lookup(t + 2, ka); }
-                        compute(t + 1, kb);
+                    for (int q = 0; q < 4; ++q) {
+                        wl[q] = (int) __builtin_amdgcn_perm(d.y, d.x, e[q]);
+                        wh[q] = (int) __builtin_amdgcn_perm(d.w, d.z, e[q]);
                     }
-                } else {                       // more tiles: one set (the step's MFMAs cover the next reads' latency)
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        Lk k; lookup(t, k); compute(t, k);
-                        __builtin_amdgcn_sched_barrier(0);   // steps stay in order: reads of later steps are not hoisted
-                    }
-                }
-                // block fold, in block order: y += (d_w * d_x) * bsum, bsum = the two chains' exact totals added once; the
-                // scale of token 16 tt + 4 g + i comes from the lane that loaded it
-                float dx[NT][4];
-#pragma unroll
-                for (int tt = 0; tt < NT; ++tt) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        dx[tt][i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (16 * tt + 4 * ln.g + i), __builtin_bit_cast(int, dxl)));
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
-                    const float dw = h2f(w[c].d);
+                    if (m == 1) { digits(c, 1); }
+                    const i4 z = (i4) { 0, 0, 0, 0 };
 #pragma unroll
                     for (int tt = 0; tt < NT; ++tt) {
+                        D[c][tt][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[m & 1][tt], wl, m == 0 ? z : D[c][tt][0], 0, 0, 0);
+                        D[c][tt][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[m & 1][tt], wh, m == 0 ? z : D[c][tt][1], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // block fold, in block order: y += (d_w * d_x) * bsum; lane (r, g) holds tokens 4 g + i of each tile
+                float dw[C];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) { acc[c][tt][i] = acc[c][tt][i] + (dw * dx[tt][i]) * (cc[c][tt][i] + cd[c][tt][i]); }
+                for (int c = 0; c < C; ++c) { dw[c] = h2f(w[c].d); }
+#pragma unroll
+                for (int tt = 0; tt < NT; ++tt) {
+                    const f4 dx = *(const LK_LOCAL f4 *) (size_t) ((uint32_t) (L_DX + buf * Geo::DXB) + (uint32_t) (64 * tt + 16 * g));
+#pragma unroll
+                    for (int c = 0; c < C; ++c) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float b = (float) ((D[c][tt][1][i] << 6) + D[c][tt][0][i]);
+                            acc[c][tt][i] = acc[c][tt][i] + (dw[c] * dx[i]) * b;
+                        }
                     }
                 }
-                (void) j; (void) buf;
             };
 
-            // pipeline: weights two blocks ahead (three register stages), activations one block ahead (registers, then
-            // the other of two LDS buffers). Every step issues the same loads (indices clamped at the last blocks: those
-            // copies land in registers nobody reads any more), so the compiler's waits count them exactly.
-            // short rows (down, 8 blocks) and items of many tiles keep the weights one block ahead (two stages): their
-            // register budget is tighter
-            constexpr int WA = (NB <= 8 || C * NT > 4 || Geo::NARROW) ? 1 : 2;   // narrow: four waves per SIMD hide it instead
-            PfW w0[C], w1[C], w2[C];
-            PfB bq;
+            // pipeline: weights and activations one block ahead (registers; the other of two LDS buffers). Every step
+            // issues the same loads (the last one reloads its own block, which nobody reads any more).
+            PfW w0[C], w1[C];
             load_w(0, w0);
-            if (WA == 2) { load_w(1, w1); }
-            load_b(0, bq, 0);
+            load_b(0, 0);
             __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block 0's activations are in LDS
             __syncthreads();
-            auto step = [&](int j, PfW (&cur)[C], PfW (&ahead)[C]) {
-                const float dxl = bq.dx;             // block j's scale (loaded with its activations)
-                // buffer (j + 1) % 2 was last read in step j - 1, before its barrier
-                load_b(j + 1 < NB ? j + 1 : NB - 1, bq, (j + 1) & 1);
-                load_w(j + WA < NB ? j + WA : NB - 1, ahead);
+            auto step = [&](int j, const PfW (&cur)[C], PfW (&ahead)[C]) {
+                const int jn = j + 1 < NB ? j + 1 : NB - 1;
+                load_b(jn, (j + 1) & 1);             // buffer (j + 1) % 2 was last read in step j - 1, before its barrier
+                load_w(jn, ahead);
                 __builtin_amdgcn_sched_barrier(0);   // nothing of the block moves above the loads
-                block(j, cur, j & 1, dxl);
+                block(cur, j & 1);
                 __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): block j + 1's activations have landed in LDS (and the
-                __builtin_amdgcn_s_barrier();       // weights of the next block are in): the barrier publishes them
+                __builtin_amdgcn_s_barrier();        // weights of the next block are in): the barrier publishes them
             };
-            if constexpr (WA == 1) {   // step j uses stage j % 2 and refills the other with block j + 1
-                static_assert(NB % 2 == 0, "two steps per trip");
+            static_assert(NB % 2 == 0, "two steps per trip");
 #pragma unroll 1
-                for (int j = 0; j < NB; j += 2) { step(j, w0, w1); step(j + 1, w1, w0); }
-            } else {                   // step j uses stage j % 3 and refills the stage of block j - 1 with block j + 2
-                constexpr int NB3 = NB - NB % 3;
-                int j = 0;
-#pragma unroll 1
-                for (; j < NB3; j += 3) {
-                    step(j, w0, w2);
-                    step(j + 1, w1, w0);
-                    step(j + 2, w2, w1);
-                }
-                if (NB % 3 >= 1) { step(j, w0, w2); }
-                if (NB % 3 == 2) { step(j + 1, w1, w0); }
-            }
+            for (int j = 0; j < NB; j += 2) { step(j, w0, w1); step(j + 1, w1, w0); }
 
             // outputs: lane (r, g) holds tokens 4 g + i of each token tile for row r of each of its tiles
-            if constexpr (NMAT == 2 && C == 1) {
-                // narrow gate/up: the gate waves (0..7) leave 0.125 g in LDS, the up waves (8..15) form h for the same
-                // tile. The exchange area is last read in this item; the next item's first barrier orders its reuse.
-                LK_LOCAL float * xg = reinterpret_cast<LK_LOCAL float *>(lds + Geo::L_G);
+            if constexpr (Geo::XG) {
+                // the gate waves leave 0.125 g in the second activation buffer (last read before the last step's barrier,
+                // next filled after the next item's first one), the up waves form h for the same tile
+                LK_LOCAL f4 * xg = reinterpret_cast<LK_LOCAL f4 *>(lds + Geo::L_X + Geo::BUF);
                 const int ti = Geo::tile(wave, 0);
                 if (Geo::mat(wave, 0) == 0) {
 #pragma unroll
-                    for (int tt = 0; tt < NT; ++tt) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) { xg[((ti * 64 + lane) * Geo::NTM + tt) * 4 + i] = 0.125f * acc[0][tt][i]; }
-                    }
+                    for (int tt = 0; tt < NT; ++tt) { xg[(ti * NTM + tt) * 64 + lane] = 0.125f * acc[0][tt]; }
                 }
                 __syncthreads();
                 if (Geo::mat(wave, 0) == 1) {
-                    const int row = rg * Geo::ROWS + ti * 16 + ln.r;
+                    const int row = rg * Geo::ROWS + ti * 16 + r;
 #pragma unroll
                     for (int tt = 0; tt < NT; ++tt) {
+                        const f4 gt = xg[(ti * NTM + tt) * 64 + lane];
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const int n32 = 16 * tt + 4 * ln.g + i;
-                            if (n32 < sc) {
-                                const size_t o = (size_t) (sb + n32) * a.R + row;
-                                const float gv = xg[((ti * 64 + lane) * Geo::NTM + tt) * 4 + i], uv = 0.125f * acc[0][tt][i];
-                                a.out[o] = det_silu(gv) * uv;
-                                if (a.gdbg) { a.gdbg[o] = gv; a.udbg[o] = uv; }
+                            const int t = 16 * tt + 4 * g + i;
+                            if (t < sc) {
+                                const size_t o = (size_t) (sb + t) * a.R + row;
+                                const float uv = 0.125f * acc[0][tt][i];
+                                a.out[o] = det_silu(gt[i]) * uv;
+                                if (a.gdbg) { a.gdbg[o] = gt[i]; a.udbg[o] = uv; }
                             }
                         }
                     }
                 }
             } else {
-                constexpr int RT = NMAT == 2 ? 1 : C;   // row tiles of the wave (gate/up wide: one, both matrices)
+                constexpr int RT = NMAT == 2 ? 1 : C;   // row tiles of the wave (gate/up: one, both matrices)
 #pragma unroll
                 for (int c = 0; c < RT; ++c) {
-                    const int row = rg * Geo::ROWS + Geo::tile(wave, c) * 16 + ln.r;
+                    const int row = rg * Geo::ROWS + Geo::tile(wave, c) * 16 + r;
 #pragma unroll
                     for (int tt = 0; tt < NT; ++tt) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const int n32 = 16 * tt + 4 * ln.g + i;
-                            if (n32 < sc) {
-                                const size_t o = (size_t) (sb + n32) * a.R + row;
+                            const int t = 16 * tt + 4 * g + i;
+                            if (t < sc) {
+                                const size_t o = (size_t) (sb + t) * a.R + row;
                                 if (NMAT == 2) {
-                                    const float gv = 0.125f * acc[0][tt][i], uv = 0.125f * acc[1][tt][i];
+                                    const float gv = 0.125f * acc[0][tt][i], uv = 0.125f * acc[C - 1][tt][i];
                                     a.out[o] = det_silu(gv) * uv;
                                     if (a.gdbg) { a.gdbg[o] = gv; a.udbg[o] = uv; }
                                 } else {
@@ -473,45 +426,63 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
                 }
             }
         };
-        if constexpr (Geo::NARROW) {
+        if constexpr (NTM == 2) {
             if (sc > 16) { run_item(std::integral_constant<int, 2>{}); }
             else { run_item(std::integral_constant<int, 1>{}); }
+        } else if constexpr (NTM == 4) {
+            if (sc > 48) { run_item(std::integral_constant<int, 4>{}); }
+            else { run_item(std::integral_constant<int, 3>{}); }
         } else {
-            run_item(std::integral_constant<int, 4>{});   // a wide column: 33..64 slots
+            if (sc > 96) { run_item(std::integral_constant<int, 7>{}); }
+            else if (sc > 80) { run_item(std::integral_constant<int, 6>{}); }
+            else { run_item(std::integral_constant<int, 5>{}); }
         }
     }
 }
 
-template <int NMAT, int NB, int W, int CPW>
-static hipError_t pf_setup() {
-    return hipFuncSetAttribute((const void *) k_pf_gemm<NMAT, NB, W, CPW>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               PfGeo<NMAT, NB, W, CPW>::LDS);
-}
+template <int NMAT, int NB, int W, int C, int NTM, int CLS> struct PfKernel {
+    using Geo = PfGeo<NMAT, NB, W, C, NTM>;
+    static hipError_t setup() {
+        return hipFuncSetAttribute((const void *) k_pf_gemm<NMAT, NB, W, C, NTM, CLS>, hipFuncAttributeMaxDynamicSharedMemorySize, Geo::LDS);
+    }
+    static void go(const PrefillArgs & a, int grid, hipStream_t st) { k_pf_gemm<NMAT, NB, W, C, NTM, CLS><<<grid, W * 64, Geo::LDS, st>>>(a); }
+};
+template <int NMAT, int NB> struct PfKernels {
+    using Broad = PfKernel<NMAT, NB, 8, 1, 7, PF_BROAD>;
+    using Wide = PfKernel<NMAT, NB, 8, 2, 4, PF_WIDE>;
+    using Narrow = PfKernel<NMAT, NB, 16, 2, 2, PF_NARROW>;
+    static hipError_t setup() {
+        hipError_t e = Broad::setup();
+        if (e == hipSuccess) { e = Wide::setup(); }
+        return e == hipSuccess ? Narrow::setup() : e;
+    }
+    static bool rows_ok(int R) { return R % Broad::Geo::ROWS == 0 && R % Wide::Geo::ROWS == 0 && R % Narrow::Geo::ROWS == 0; }
+    static void go(const PrefillArgs & a, int grid, hipStream_t st) {   // classes that cannot occur are not launched
+        if (a.most > 64) { Broad::go(a, grid, st); }
+        if (a.most > 32) { Wide::go(a, grid, st); }
+        Narrow::go(a, grid, st);
+    }
+};
 hipError_t prefill_init() {
-    hipError_t e = pf_setup<2, 28, 8, 2>();
-    if (e == hipSuccess) { e = pf_setup<1, 8, 8, 2>(); }
-    if (e == hipSuccess) { e = pf_setup<2, 28, 16, 1>(); }
-    if (e == hipSuccess) { e = pf_setup<1, 8, 16, 1>(); }
-    return e;
+    hipError_t e = PfKernels<2, 28>::setup();
+    if (e == hipSuccess) { e = PfKernels<1, 8>::setup(); }
+    return e == hipSuccess ? few_init() : e;
 }
 
-// the wide kernel, then the narrow one, over the columns col0 .. col1 - 1 (each takes its class)
+// the broad, wide, narrow and few kernels over the columns col0 .. col1 - 1 (each takes its class)
 hipError_t launch_prefill_gemm(const PrefillArgs & a, int grid, hipStream_t st) {
-    if (grid < 1 || !a.ptab || !a.cols || !a.ncols || !a.bh || !a.bd || !a.out || !a.err) { return hipErrorInvalidValue; }
+    if (grid < 1 || !a.ptab || !a.cols || !a.ncols || !a.bq || !a.bd || !a.out || !a.err) { return hipErrorInvalidValue; }
     if (a.nmat == 2) {
-        if (a.K != 28 * QK || a.R % PfGeo<2, 28, 8, 2>::ROWS || a.R % PfGeo<2, 28, 16, 1>::ROWS || !a.w[0] || !a.w[1] || !a.sh[0] || !a.sh[1] || !a.perm) {
-            return hipErrorInvalidValue;
-        }
-        k_pf_gemm<2, 28, 8, 2><<<grid, 8 * 64, PfGeo<2, 28, 8, 2>::LDS, st>>>(a);
-        k_pf_gemm<2, 28, 16, 1><<<grid, 16 * 64, PfGeo<2, 28, 16, 1>::LDS, st>>>(a);
+        if (a.K != 28 * QK || !PfKernels<2, 28>::rows_ok(a.R) || !a.w[0] || !a.w[1] || !a.sh[0] || !a.sh[1] || !a.perm) { return hipErrorInvalidValue; }
+        PfKernels<2, 28>::go(a, grid, st);
     } else if (a.nmat == 1) {
-        if (a.K != 8 * QK || a.R % PfGeo<1, 8, 8, 2>::ROWS || a.R % PfGeo<1, 8, 16, 1>::ROWS || !a.w[0] || !a.sh[0]) { return hipErrorInvalidValue; }
-        k_pf_gemm<1, 8, 8, 2><<<grid, 8 * 64, PfGeo<1, 8, 8, 2>::LDS, st>>>(a);
-        k_pf_gemm<1, 8, 16, 1><<<grid, 16 * 64, PfGeo<1, 8, 16, 1>::LDS, st>>>(a);
+        if (a.K != 8 * QK || !PfKernels<1, 8>::rows_ok(a.R) || !a.w[0] || !a.sh[0]) { return hipErrorInvalidValue; }
+        PfKernels<1, 8>::go(a, grid, st);
     } else {
         return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? launch_few_gemm(a, grid, st) : e;
 }
 
 }  // namespace lk

@@ -882,3 +882,16 @@ def test_decode1_selection_crafted_logits(ctx, kind):
         assert np.array_equal(got["decode1"][1].view(np.uint32), wo.ravel().view(np.uint32)), (kind, case)
     del layer
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n,hot", [(9, True), (12, False), (17, True), (33, False), (64, True), (65, False), (72, True), (200, True)])
+def test_few_slot_columns_match_per_pass(ctx, n, hot):
+    """Columns of 1..8 slots on the int8 matrix-core kernel (every column up to 64 tokens, the small remainders above):
+    one and two sets of four tokens, partly filled ones, the shared expert's last column of 1..8, and hot experts whose
+    slots fill many columns. Bit for bit the per-pass kernels."""
+    layer = make_layer(ctx, seed=2100 + n, bias_sigma=0.05, hot=list(range(5, 256, 32)) if hot else None)
+    x = make_x(ctx, n, seed=61 + n)
+    ref = _prefill_state(ctx, layer, x, False)
+    got = _prefill_state(ctx, layer, x, True)
+    for k in ref:
+        assert np.array_equal(got[k].view(np.uint8), ref[k].view(np.uint8)), k
