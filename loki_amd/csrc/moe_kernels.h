@@ -144,7 +144,7 @@ hipError_t launch_prefill_cols(const int * act, const int * nact, const int * of
 constexpr int prefill_shared_cols(int n, int tok) { return (n + tok - 1) / tok; }   // the shared expert's columns (the first ones)
 // IQ2_XXS tables by batch size: up to PF_SPLIT_N tokens every column has at most 8 slots (launch_few_gemm alone), up to
 // PF_FEW_N the columns of at most 8 run on the few kernel, above on the narrow one
-constexpr int PF_SPLIT_N = 64, PF_FEW_N = 256;
+constexpr int PF_SPLIT_N = 128, PF_FEW_N = 256;
 constexpr int pf_tok(int n) { return n <= PF_SPLIT_N ? FEW_TOK : PF_TOK; }
 constexpr int pf_few(int n) { return n <= PF_FEW_N ? FEW_TOK : 0; }
 

@@ -155,9 +155,11 @@ struct PfGeo {
     static constexpr int ROWS = TPM * 16, K = NB * QK;
     static constexpr int BUF = NTM * 16 * QK;                   // one activation buffer
     static constexpr int DXB = (NTM + 3) / 4 * 256;             // one buffer of block scales (64 tokens per copy)
-    static constexpr int L_X = (L_DX + 2 * DXB + 1023) / 1024 * 1024, LDS = L_X + 2 * BUF;
-    static constexpr bool XG = NMAT == 2 && C == 1;             // g goes through LDS (the second activation buffer)
-    static_assert(LDS <= 160 * 1024 && W * C % NMAT == 0 && C <= 2 && (!XG || W / 2 * 64 * NTM * 16 <= BUF), "prefill GEMM geometry");
+    static constexpr int L_X = (L_DX + 2 * DXB + 1023) / 1024 * 1024;
+    static constexpr bool XG = NMAT == 2 && C == 1;             // g goes through LDS: an area of its own, or the second
+    static constexpr int XGB = XG ? W / 2 * 64 * NTM * 16 : 0;  // activation buffer when that is large enough
+    static constexpr int L_G = XGB <= BUF ? L_X + BUF : L_X + 2 * BUF, LDS = L_X + 2 * BUF + (XGB <= BUF ? 0 : XGB);
+    static_assert(LDS <= 160 * 1024 && W * C % NMAT == 0 && C <= 2 && W % 8 == 0, "prefill GEMM geometry");
     // the matrix and the 16-row tile (within the item) of combo c of wave w
     __device__ static constexpr int mat(int w, int c) { return C == NMAT ? c : NMAT == 1 ? 0 : w / (W / NMAT); }
     __device__ static constexpr int tile(int w, int c) { return C == NMAT ? w : NMAT == 1 ? w * C + c : w % (W / NMAT); }
@@ -275,27 +277,19 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
 #pragma unroll
             for (int c = 0; c < C; ++c) { for (int tt = 0; tt < NT; ++tt) { acc[c][tt] = (f4) { 0.f, 0.f, 0.f, 0.f }; } }
 
-            // one block: dequantise the C tiles step by step and run the MFMA chains of the token tiles
-            auto block = [&](const PfW (&w)[C], int buf) {
-                const uint32_t bx = (uint32_t) (Geo::L_X + buf * Geo::BUF) + (uint32_t) r * QK + (uint32_t) (((4 * g) ^ r) << 4);
-                i4 D[C][NT][2];         // per tile pair: the sums of the low and of the high digits
+            // A block's weights as MFMA operands: the low and the high digits of the C tiles (4 steps of 16 weights per lane)
+            // and their d. The LDS reads of a step (two selector and two sign entries) are issued one step ahead of their
+            // use, into the other of two register sets.
+            i4 wl[C][4], wh[C][4];
+            float dw[C];
+            auto dequant = [&](const PfW (&w)[C]) {
                 u32x4 dig[C];           // the scale line of the lane's sub-block in use (2 g, then 2 g + 1)
                 uint32_t ms[C][2];
                 auto digits = [&](int c, int h) {
                     const uint32_t sw = h ? w[c].q.w : w[c].q.y;
                     dig[c] = *(const LK_LOCAL u32x4 *) (size_t) __builtin_amdgcn_udot4((sw >> 7) & 0x01010101u, 0x80402010u, (uint32_t) L_SCL, false);
                 };
-#pragma unroll
-                for (int c = 0; c < C; ++c) { digits(c, 0); ms[c][0] = w[c].q.y & SIGN_BITS; ms[c][1] = w[c].q.w & SIGN_BITS; }
-                // Steps (m, c), m outer. The LDS reads of a step (the tile's two selector and sign entries; at the first
-                // tile of an m the activation chunks) are issued one step ahead of their use, into the other of two
-                // register sets, so their latency runs under the step's dequantisation and MFMAs.
                 struct Lk { uint2 g0, g1, s0, s1; };
-                auto operand = [&](int m, i4 (&x)[NT]) {
-                    const uint32_t bo = bx ^ ((uint32_t) m << 4);   // chunk (4 g + m) ^ r of the lane's token row
-#pragma unroll
-                    for (int tt = 0; tt < NT; ++tt) { x[tt] = __builtin_bit_cast(i4, *(const LK_LOCAL u32x4 *) (size_t) (bo + tt * 16 * QK)); }
-                };
                 auto lookup = [&](int m, int c, Lk & k) {
                     const uint32_t a0 = m < 2 ? w[c].q.x : w[c].q.z, a1 = ms[c][m >> 1];
                     if (m & 1) {
@@ -306,51 +300,68 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
                         k.s0 = lload8(tab_addr<0>(a1, trs)); k.s1 = lload8(tab_addr<1>(a1, trs));
                     }
                 };
+#pragma unroll
+                for (int c = 0; c < C; ++c) { digits(c, 0); ms[c][0] = w[c].q.y & SIGN_BITS; ms[c][1] = w[c].q.w & SIGN_BITS; dw[c] = h2f(w[c].d); }
                 Lk k[2];
-                i4 x[2][NT];
-                operand(0, x[0]);
                 lookup(0, 0, k[0]);
 #pragma unroll
                 for (int i = 0; i < 4 * C; ++i) {
                     const int m = i / C, c = i % C;
-                    if (i + 1 < 4 * C) {
-                        if (c == C - 1) { operand(m + 1, x[(m + 1) & 1]); }
-                        lookup((i + 1) / C, (i + 1) % C, k[(i + 1) & 1]);
-                    }
+                    if (i + 1 < 4 * C) { lookup((i + 1) / C, (i + 1) % C, k[(i + 1) & 1]); }
                     const Lk & u = k[i & 1];
                     const uint32_t e[4] = { u.g0.x | u.s0.x, u.g0.y | u.s0.y, u.g1.x | u.s1.x, u.g1.y | u.s1.y };
                     const u32x4 d = dig[c];
-                    i4 wl, wh;
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        wl[q] = (int) __builtin_amdgcn_perm(d.y, d.x, e[q]);
-                        wh[q] = (int) __builtin_amdgcn_perm(d.w, d.z, e[q]);
+                        wl[c][m][q] = (int) __builtin_amdgcn_perm(d.y, d.x, e[q]);
+                        wh[c][m][q] = (int) __builtin_amdgcn_perm(d.w, d.z, e[q]);
                     }
                     if (m == 1) { digits(c, 1); }
-                    const i4 z = (i4) { 0, 0, 0, 0 };
-#pragma unroll
-                    for (int tt = 0; tt < NT; ++tt) {
-                        D[c][tt][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[m & 1][tt], wl, m == 0 ? z : D[c][tt][0], 0, 0, 0);
-                        D[c][tt][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[m & 1][tt], wh, m == 0 ? z : D[c][tt][1], 0, 0, 0);
-                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                // block fold, in block order: y += (d_w * d_x) * bsum; lane (r, g) holds tokens 4 g + i of each tile
-                float dw[C];
+            };
+            // The block's products with one token tile after the other: the next tile's activations are read and the
+            // previous tile's sums folded while this one's MFMAs run. Fold, in block order: y += (d_w * d_x) * bsum; lane
+            // (r, g) holds tokens 4 g + i of a tile.
+            auto products = [&](int buf) {
+                const uint32_t bx = (uint32_t) (Geo::L_X + buf * Geo::BUF) + (uint32_t) r * QK + (uint32_t) (((4 * g) ^ r) << 4);
+                i4 x[2][4], D[2][C][2];
+                f4 dx[2];
+                auto operand = [&](int tt) {   // chunks (4 g + m) ^ r of the lane's token row
 #pragma unroll
-                for (int c = 0; c < C; ++c) { dw[c] = h2f(w[c].d); }
-#pragma unroll
-                for (int tt = 0; tt < NT; ++tt) {
-                    const f4 dx = *(const LK_LOCAL f4 *) (size_t) ((uint32_t) (L_DX + buf * Geo::DXB) + (uint32_t) (64 * tt + 16 * g));
+                    for (int m = 0; m < 4; ++m) { x[tt & 1][m] = __builtin_bit_cast(i4, *(const LK_LOCAL u32x4 *) (size_t) ((bx ^ (uint32_t) (m << 4)) + tt * 16 * QK)); }
+                    dx[tt & 1] = *(const LK_LOCAL f4 *) (size_t) ((uint32_t) (L_DX + buf * Geo::DXB) + (uint32_t) (64 * tt + 16 * g));
+                };
+                auto fold = [&](int tt, int i, float dxi) {
 #pragma unroll
                     for (int c = 0; c < C; ++c) {
+                        const float b = (float) ((D[tt & 1][c][1][i] << 6) + D[tt & 1][c][0][i]);
+                        acc[c][tt][i] = acc[c][tt][i] + (dw[c] * dxi) * b;
+                    }
+                };
+                operand(0);
+                f4 dp;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float b = (float) ((D[c][tt][1][i] << 6) + D[c][tt][0][i]);
-                            acc[c][tt][i] = acc[c][tt][i] + (dw[c] * dx[i]) * b;
+                for (int tt = 0; tt < NT; ++tt) {
+                    if (tt > 0) { dp = dx[(tt - 1) & 1]; }
+                    if (tt + 1 < NT) { operand(tt + 1); }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        const i4 z = (i4) { 0, 0, 0, 0 };
+#pragma unroll
+                        for (int c = 0; c < C; ++c) {
+                            i4 (&d)[2] = D[tt & 1][c];
+                            d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[tt & 1][m], wl[c][m], m == 0 ? z : d[0], 0, 0, 0);
+                            d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[tt & 1][m], wh[c][m], m == 0 ? z : d[1], 0, 0, 0);
                         }
+                        if (tt > 0) { fold(tt - 1, m, dp[m]); }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 }
+                dp = dx[(NT - 1) & 1];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { fold(NT - 1, i, dp[i]); }
             };
 
             // pipeline: weights and activations one block ahead (registers; the other of two LDS buffers). Every step
@@ -365,7 +376,8 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
                 load_b(jn, (j + 1) & 1);             // buffer (j + 1) % 2 was last read in step j - 1, before its barrier
                 load_w(jn, ahead);
                 __builtin_amdgcn_sched_barrier(0);   // nothing of the block moves above the loads
-                block(cur, j & 1);
+                dequant(cur);
+                products(j & 1);
                 __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): block j + 1's activations have landed in LDS (and the
                 __builtin_amdgcn_s_barrier();        // weights of the next block are in): the barrier publishes them
             };
@@ -377,7 +389,7 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
             if constexpr (Geo::XG) {
                 // the gate waves leave 0.125 g in the second activation buffer (last read before the last step's barrier,
                 // next filled after the next item's first one), the up waves form h for the same tile
-                LK_LOCAL f4 * xg = reinterpret_cast<LK_LOCAL f4 *>(lds + Geo::L_X + Geo::BUF);
+                LK_LOCAL f4 * xg = reinterpret_cast<LK_LOCAL f4 *>(lds + Geo::L_G);
                 const int ti = Geo::tile(wave, 0);
                 if (Geo::mat(wave, 0) == 0) {
 #pragma unroll
@@ -450,7 +462,7 @@ template <int NMAT, int NB, int W, int C, int NTM, int CLS> struct PfKernel {
 template <int NMAT, int NB> struct PfKernels {
     using Broad = PfKernel<NMAT, NB, 8, 1, 7, PF_BROAD>;
     using Wide = PfKernel<NMAT, NB, 8, 2, 4, PF_WIDE>;
-    using Narrow = PfKernel<NMAT, NB, 16, 2, 2, PF_NARROW>;
+    using Narrow = PfKernel<NMAT, NB, 16, 1, 2, PF_NARROW>;
     static hipError_t setup() {
         hipError_t e = Broad::setup();
         if (e == hipSuccess) { e = Wide::setup(); }
