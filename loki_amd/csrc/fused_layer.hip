@@ -244,10 +244,10 @@ int route_dev(FLCtx * c, const float * W, const float * bias, const float * x, i
                                    c->epoch, c->rcnt.p, done, c->derr.p, c->herr ? c->herr_dev : nullptr, c->st));
         return FL_OK;
     }
-    double * rp = nullptr;   // the K-split tiles' parts (n from RL_SPLIT_MIN to RL_SPLIT_MAX)
-    if (const size_t nd = router_split_doubles(n, n_exp, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
+    double * rp = nullptr;   // the matrix-core kernel's parts
+    if (const size_t nd = router_part_doubles(n, n_exp, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
     TRY(c, launch_router_logits(W, x, n, n_exp, E, logits, rp, c->st));
-    TRY(c, launch_router_select(logits, bias, n, n_exp, c->n_group, c->topk_group, c->topk, c->scale, probs, sel, w, c->st));
+    TRY(c, launch_router_select(logits, rp, E, bias, n, n_exp, c->n_group, c->topk_group, c->topk, c->scale, probs, sel, w, c->st));
     return FL_OK;
 }
 extern "C" int fl_route_dev(FLCtx * c, const float * W, const float * bias, const float * x, int n, int n_exp, int E,
@@ -604,16 +604,16 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     TRY(c, launch_quant_q8k(x, n, E, c->xq.p, c->xd.p, st));
     if (mfma && kq) { TRY(c, launch_q8_to_h(c->xq.p, c->xh.p, (int64_t) n * E, st)); }
     prof_mark(c, ev, 1);
-    double * rp = nullptr;   // the K-split tiles' parts (n from RL_SPLIT_MIN to RL_SPLIT_MAX)
-    if (const size_t nd = router_split_doubles(n, ne, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
+    double * rp = nullptr;   // the matrix-core kernel's parts
+    if (const size_t nd = router_part_doubles(n, ne, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
     TRY(c, launch_router_logits(L->gate_inp, x, n, ne, E, c->logits.p, rp, st));
     prof_mark(c, ev, 2);
     if (share) {   // every row's topk picks, then the keep across the rows
         ALLOC(c, c->sel8, (size_t) n * tsel); ALLOC(c, c->w8, (size_t) n * tsel);
-        TRY(c, launch_router_select(c->logits.p, L->probs_b, n, ne, c->n_group, c->topk_group, tsel, c->scale, c->probs.p, c->sel8.p, c->w8.p, st, tsel, 0.f));
+        TRY(c, launch_router_select(c->logits.p, rp, E, L->probs_b, n, ne, c->n_group, c->topk_group, tsel, c->scale, c->probs.p, c->sel8.p, c->w8.p, st, tsel, 0.f));
         TRY(c, launch_keep_share(c->sel8.p, c->w8.p, n, tsel, tk, renorm, c->sel.p, c->wts.p, st));
     } else {
-        TRY(c, launch_router_select(c->logits.p, L->probs_b, n, ne, c->n_group, c->topk_group, tsel, c->scale, c->probs.p, c->sel.p, c->wts.p, st, tk, renorm));
+        TRY(c, launch_router_select(c->logits.p, rp, E, L->probs_b, n, ne, c->n_group, c->topk_group, tsel, c->scale, c->probs.p, c->sel.p, c->wts.p, st, tk, renorm));
     }
     prof_mark(c, ev, 3);
     int * dsc = nullptr;

@@ -12,15 +12,15 @@ namespace lk {
 hipError_t launch_quant_q8k(const float * x, int64_t nrows, int K, int8_t * q, float * d, hipStream_t st);
 
 // router logits [n][n_exp] under the fp64 chunk contract (K % 256 == 0)
-// part2: fp64 scratch of router_split_doubles(n, n_exp, K) for the K-split tiles (RL_SPLIT_MIN <= n <= RL_SPLIT_MAX,
-// K 7168); may be null (then the split is not used)
-constexpr int RL_SPLIT_MIN = 40;     // below it one workgroup per expert (k_router_wg) is as fast or faster
-constexpr int RL_SPLIT_MAX = 2048;   // above it the whole LDS tiles (scratch 16 x n x n_exp doubles at most 64 MiB)
-size_t router_split_doubles(int n, int n_exp, int K);
+// part2: fp64 scratch of router_part_doubles(n, n_exp, K) for the matrix-core kernel (k_router_mfma), which then leaves the
+// logits as parts [router_parts][n][n_exp] for launch_router_select to add up, round and write (null or no parts: written
+// here)
+int router_parts(int n, int n_exp, int K);
+size_t router_part_doubles(int n, int n_exp, int K);
 hipError_t launch_router_logits(const float * W, const float * x, int n, int n_exp, int K, float * logits, double * part2, hipStream_t st);
 // sigmoid, bias, grouped top-k, normalised weights; probs [n][n_exp], sel/wts [n][keep]: with 0 < keep < topk each
 // row keeps its keep heaviest picks (rescaled to sum to renorm when renorm > 0), else all topk
-hipError_t launch_router_select(const float * logits, const float * bias, int n, int n_exp, int n_group, int topk_group,
+hipError_t launch_router_select(float * logits, const double * part2, int K, const float * bias, int n, int n_exp, int n_group, int topk_group,
                                 int topk, float scale, float * probs, int * sel, float * wts, hipStream_t st, int keep = 0,
                                 float renorm = 0.f);
 

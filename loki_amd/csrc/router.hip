@@ -31,11 +31,11 @@ __global__ void __launch_bounds__(64) k_router_logits(const float * __restrict__
     }
 }
 
-// Batches below 256 tokens (K = 7168): one workgroup (4 waves) per expert; thread c owns chunk c (28 values) of every
+// A few tokens (K = 7168, n < RM_MIN): one workgroup (4 waves) per expert; thread c owns chunk c (28 values) of every
 // token and keeps its 28 weights in registers. Per token the chunk sum runs in element order with v_fma_f64 (exact
 // products, one rounding each), tree levels 1-6 are lane butterflies inside the wave (chunks 64 q .. 64 q + 63 of wave
 // q), and levels 7-8 add the four waves' totals as (q0 + q1) + (q2 + q3) through LDS. Four tokens per pass.
-constexpr int RW_MAXN = 256;
+constexpr int RW_MAXN = 16;
 __device__ __forceinline__ void router_wg_logits(const float * __restrict__ W, const float * __restrict__ x, int n, int n_exp,
                                                  float * __restrict__ logits, double (*part)[4]) {
 #pragma clang fp contract(off)
@@ -153,321 +153,158 @@ __global__ void __launch_bounds__(256) k_router_wg_sel(const float * __restrict_
     }
 }
 
-// Large batches (K = 7168): register tiles. Lane (tg, eg) = (lane / 8, lane % 8) owns the logits of TT tokens x EE
-// experts of the workgroup's (8 TT) x (8 EE) tile; wave q computes slice q of the contract (chunks q * 256 / NQ ..) with the
-// same in-order fp64 chunk sums and pairwise tree as k_router_wg, and the slices are combined by the tree's top levels
-// through LDS. Each 16-byte load of x or W feeds EE or TT fused multiply-adds, so x and W are read once per tile.
-template <int TT, int EE> struct RgAcc { double v[TT][EE]; };
-// one chunk's in-order sums (28 products each) for the lane's TT x EE logits; the loads of step i + 1 are in flight
-// while step i computes, and nothing is hoisted further (register budget)
-template <int TT, int EE>
-__device__ __forceinline__ void rg_chunk(const float * const (&xr)[TT], const float * const (&wr)[EE], int c, RgAcc<TT, EE> & s) {
+// Prefill batches (K = 7168): the chunk sums on the fp64 matrix cores. v_mfma_f64_16x16x4_f64 adds its four products to
+// the accumulator one after the other in K order, each by one fma (checked on the device against a sequential fma chain
+// over random and cancelling data: no bit differs), and an fp32 x fp32 product is exact in fp64: seven of them are one
+// chunk of the contract. Bound by the matrix cores' fp64 rate (64 clocks per product and SIMD, the VALU's fma rate,
+// without its operand traffic): the VALU tiles this replaces took 338 us at 2048 tokens and 102 at 512.
+//   * A workgroup (8 waves) owns 32 tokens x 32 experts and 1 / KS of the chunks (blockIdx.z); wave w takes CPW = 256 / (8
+//     KS) consecutive chunks for the whole tile (2 x 2 tiles of 16 x 16).
+//   * Operands come straight from memory: lane (r, g) loads 16 bytes of row r, piece 4 q + g of the row's 4-value pieces,
+//     so an instruction covers 16 rows x 64 bytes; a 4 x 4 transpose over the lane groups (two v_permlane32_swap, two
+//     v_permlane16_swap) gives the operands of products 4 q .. 4 q + 3. Four chunks are seven such loads per operand
+//     tile; the next one is in flight while one is used.
+//   * The contract's pairwise tree runs in registers as the chunks arrive, its next three levels over the workgroup's
+//     waves through LDS, the levels over the KS parts in the selection (launch_router_select), which rounds to fp32.
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef float rf4 __attribute__((ext_vector_type(4)));
+constexpr int RM_W = 8, RM_LDS = RM_W * 16 * 64 * 8;
+struct RmAcc { d4 v[2][2]; };   // [token tile][expert tile]: lane (r, g) holds expert r, tokens g + 4 i
+__device__ __forceinline__ void rm_add(RmAcc & d, const RmAcc & l, const RmAcc & r) {
 #pragma clang fp contract(off)
-    constexpr int CL = 28, NS = CL / 4;
-    float4 xv[2][TT], wv[2][EE];
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
+    for (int i = 0; i < 2; ++i) { for (int j = 0; j < 2; ++j) { d.v[i][j] = l.v[i][j] + r.v[i][j]; } }
+}
+__device__ __forceinline__ void rm_transpose(float & a0, float & a1, float & a2, float & a3) {
+    __asm__ volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1\n\t"
+                     "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1" : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3));
+}
+template <int KS>
+__global__ void __launch_bounds__(RM_W * 64, 1) k_router_mfma(const float * __restrict__ W, const float * __restrict__ x, int n, int n_exp,
+                                                              double * __restrict__ part2, float * __restrict__ logits) {
+#pragma clang fp contract(off)
+    constexpr int K = 7168, CPW = 256 / (RM_W * KS), G4 = CPW / 4, LG = G4 == 8 ? 3 : G4 == 4 ? 2 : G4 == 2 ? 1 : 0;
+    static_assert(G4 >= 1 && G4 == (1 << LG), "slices of 4, 8, 16 or 32 chunks");
+    extern __shared__ __attribute__((aligned(16))) uint8_t rm_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), r = lane & 15, g = lane >> 4;
+    // consecutive workgroups go to the 8 XCDs in turn: with 8 expert tiles, those of one token tile are put on one XCD, so
+    // its L2 serves the tokens to all of them (token tiles past a multiple of 8 keep the plain order)
+    int tt = blockIdx.y, et = blockIdx.x;
+    if (gridDim.x == 8 && tt < (int) gridDim.y / 8 * 8) { et = blockIdx.y & 7; tt = (int) (blockIdx.y & ~7u) + (int) blockIdx.x; }
+    const int tb = tt * 32, eb = et * 32;
+    const int c0 = ((int) blockIdx.z * RM_W + wave) * CPW;
+    const float * src[4];   // x rows of the two token tiles, W rows of the two expert tiles (rows past the end repeat row 0)
 #pragma unroll
-        for (int e = 0; e < EE; ++e) { s.v[t][e] = 0.0; }
+    for (int k = 0; k < 2; ++k) {
+        const int t = tb + 16 * k + r, e = eb + 16 * k + r;
+        src[k] = x + (size_t) (t < n ? t : 0) * K + 28 * c0 + 4 * g;
+        src[2 + k] = W + (size_t) (e < n_exp ? e : 0) * K + 28 * c0 + 4 * g;
     }
-    auto load = [&](int i, int b) {
+    rf4 raw[2][4];
+    auto fetch = [&](int q, int b) {   // quad q of 16 values: the lane's piece of each operand row
 #pragma unroll
-        for (int t = 0; t < TT; ++t) { xv[b][t] = gloadf4(xr[t] + CL * c + 4 * i); }
-#pragma unroll
-        for (int e = 0; e < EE; ++e) { wv[b][e] = gloadf4(wr[e] + CL * c + 4 * i); }
+        for (int k = 0; k < 4; ++k) { raw[b][k] = *(const LK_GLOBAL rf4 *) (src[k] + 16 * q); }
     };
-    load(0, 0);
+    RmAcc pend[LG + 1], node, ev, l1;
+    fetch(0, 0);
+#pragma unroll 1
+    for (int g4 = 0; g4 < G4; ++g4) {   // four chunks: 28 products, 7 quads
+        RmAcc acc;
 #pragma unroll
-    for (int i = 0; i < NS; ++i) {
-        const int b = i & 1;
-        if (i + 1 < NS) { load(i + 1, b ^ 1); }
+        for (int q = 0; q < 7; ++q) {
+            // the quads of a trip are 7: the buffer parity runs over q, the first quad of the next trip goes to buffer 1
+            // (q = 6 is in buffer 0) and is moved to 0 at the end of the trip
+            fetch(min(7 * g4 + q + 1, 7 * G4 - 1), (q + 1) & 1);
+            rf4 (&c)[4] = raw[q & 1];
+            float p[4][4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            double xd[TT], wd[EE];
-#pragma unroll
-            for (int t = 0; t < TT; ++t) { xd[t] = (double) (q == 0 ? xv[b][t].x : q == 1 ? xv[b][t].y : q == 2 ? xv[b][t].z : xv[b][t].w); }
-#pragma unroll
-            for (int e = 0; e < EE; ++e) { wd[e] = (double) (q == 0 ? wv[b][e].x : q == 1 ? wv[b][e].y : q == 2 ? wv[b][e].z : wv[b][e].w); }
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-#pragma unroll
-                for (int e = 0; e < EE; ++e) { s.v[t][e] = __builtin_fma(xd[t], wd[e], s.v[t][e]); }
+            for (int k = 0; k < 4; ++k) {
+                p[k][0] = c[k][0]; p[k][1] = c[k][1]; p[k][2] = c[k][2]; p[k][3] = c[k][3];
+                rm_transpose(p[k][0], p[k][1], p[k][2], p[k][3]);
             }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-template <int TT, int EE>
-__device__ __forceinline__ void rg_add(RgAcc<TT, EE> & d, const RgAcc<TT, EE> & l, const RgAcc<TT, EE> & r) {
-#pragma clang fp contract(off)
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
+            for (int s = 0; s < 4; ++s) {
+                const int st = 4 * q + s, ch = st / 7;
+                const d4 z = (d4) { 0.0, 0.0, 0.0, 0.0 };
 #pragma unroll
-        for (int e = 0; e < EE; ++e) { d.v[t][e] = l.v[t][e] + r.v[t][e]; }
-    }
-}
-// the level-4 node over chunks c0 .. c0 + 15: the pairwise tree built as the chunks arrive (binary counter; pend[l]
-// holds the pending left node of level l)
-template <int TT, int EE>
-__device__ __forceinline__ RgAcc<TT, EE> rg_tile16(const float * const (&xr)[TT], const float * const (&wr)[EE], int c0) {
-    RgAcc<TT, EE> pend[4], v;
-#pragma unroll 1
-    for (int c = 0; c < 16; ++c) {
-        rg_chunk<TT, EE>(xr, wr, c0 + c, v);
-        if (!(c & 1)) { pend[0] = v; continue; }
-        rg_add(v, pend[0], v);
-        if (!(c & 2)) { pend[1] = v; continue; }
-        rg_add(v, pend[1], v);
-        if (!(c & 4)) { pend[2] = v; continue; }
-        rg_add(v, pend[2], v);
-        if (!(c & 8)) { pend[3] = v; continue; }
-        rg_add(v, pend[3], v);
-    }
-    return v;
-}
-template <int TT, int EE, int NQ>
-__global__ void __launch_bounds__(64 * NQ) k_router_tile(const float * __restrict__ W, const float * __restrict__ x, int n, int n_exp,
-                                                       float * __restrict__ logits) {
-#pragma clang fp contract(off)
-    constexpr int K = 7168, CPW = 256 / NQ, LW = CPW == 64 ? 6 : CPW == 32 ? 5 : 4;   // chunks per wave, tree levels
-    static_assert(CPW == (1 << LW) && LW >= 4, "slices of 16, 32 or 64 chunks");
-    __shared__ double part[NQ][TT * EE][64];
-    const int q = threadIdx.x >> 6, lane = lane_id(), tg = lane >> 3, eg = lane & 7;
-    const int tb = blockIdx.y * 8 * TT + tg * TT, eb = blockIdx.x * 8 * EE + eg * EE;
-    const float * xr[TT]; const float * wr[EE];
+                for (int i = 0; i < 2; ++i) {
 #pragma unroll
-    for (int t = 0; t < TT; ++t) { xr[t] = x + (size_t) (tb + t < n ? tb + t : 0) * K; }
-#pragma unroll
-    for (int e = 0; e < EE; ++e) { wr[e] = W + (size_t) (eb + e < n_exp ? eb + e : 0) * K; }
-    // the wave's slice as 16-chunk groups (level-4 nodes), combined pairwise in order (levels 5, 6)
-    RgAcc<TT, EE> tot, l4, l5;
-#pragma unroll 1
-    for (int g = 0; g < CPW / 16; ++g) {
-        RgAcc<TT, EE> v = rg_tile16<TT, EE>(xr, wr, q * CPW + 16 * g);
-        if (LW == 4) { tot = v; break; }
-        if (!(g & 1)) { l4 = v; continue; }
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-#pragma unroll
-            for (int e = 0; e < EE; ++e) { v.v[t][e] = l4.v[t][e] + v.v[t][e]; }
-        }
-        if (LW == 5) { tot = v; break; }
-        if (!(g & 2)) { l5 = v; continue; }
-#pragma unroll
-        for (int t = 0; t < TT; ++t) {
-#pragma unroll
-            for (int e = 0; e < EE; ++e) { tot.v[t][e] = l5.v[t][e] + v.v[t][e]; }
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-#pragma unroll
-        for (int e = 0; e < EE; ++e) { part[q][t * EE + e][lane] = tot.v[t][e]; }
-    }
-    __syncthreads();
-    // the tree's top levels over the NQ slices, pairwise in slice order; output o of the lane by wave o % NQ
-    for (int o = q; o < TT * EE; o += NQ) {
-        const int t = tb + o / EE, e = eb + o % EE;
-        double v[NQ];
-#pragma unroll
-        for (int j = 0; j < NQ; ++j) { v[j] = part[j][o][lane]; }
-#pragma unroll
-        for (int w = 1; w < NQ; w *= 2) {
-#pragma unroll
-            for (int j = 0; j + w < NQ; j += 2 * w) { v[j] = v[j] + v[j + w]; }
-        }
-        if (t < n && e < n_exp) { logits[(size_t) t * n_exp + e] = (float) v[0]; }
-    }
-}
-
-// Large batches (K = 7168), LDS-staged: the tiles, lanes and contract of k_router_tile<4, 4, NQ> (32 tokens x 32 experts
-// per workgroup, lane (tg, eg) owns tokens 4 tg .. + 3 x experts 4 eg .. + 3, wave q the chunks q * 256 / NQ ..), but a
-// chunk's 32 x rows and 32 W rows (28 values each) are loaded once per wave with coalesced 16-byte loads, converted to
-// fp64 once and staged in the wave's own LDS buffer, where the lanes read them back (8 lanes share each row: a broadcast).
-// Without the staging every lane loads and converts its 8 rows itself: 8x the load instructions and the conversions, and
-// the texture unit's load rate bounds the kernel. The next chunk's raw values are in registers while a chunk computes.
-// With KS > 1 the chunks are split over KS workgroups (blockIdx.z takes chunks z * 256 / KS ..), each forming its
-// part's subtree into part2[z]; k_router_join adds the parts pairwise in order, the tree's top log2(KS) levels. The
-// split that is launched, <2, 16>, gives each wave 8 chunks and needs 250 VGPRs, so two waves share a SIMD: the chunks'
-// load latencies, which bound the whole tiles (64 chunks per wave, one wave per SIMD), overlap.
-// Buffer layout, per operand: [block i (4 values)][row r % 4][half h][row r / 4] of 16 bytes (2 doubles), so a read of
-// one (i, r % 4, h) by the wave touches 8 consecutive 16-byte slots: every bank once.
-constexpr int RL_SLOTS = 7 * 4 * 2 * 8;   // 16-byte slots per operand and chunk
-template <int NQ, int KS>
-__global__ void __launch_bounds__(64 * NQ) k_router_lds(const float * __restrict__ W, const float * __restrict__ x, int n, int n_exp,
-                                                         float * __restrict__ logits, double * __restrict__ part2) {
-#pragma clang fp contract(off)
-    constexpr int K = 7168, CL = 28, CPW = 256 / (NQ * KS), LW = CPW == 64 ? 6 : CPW == 32 ? 5 : CPW == 16 ? 4 : 3;
-    constexpr int GN = CPW < 16 ? CPW : 16;   // chunks per tree group (the group's levels run as the chunks arrive)
-    static_assert(CPW == (1 << LW) && LW >= 3, "slices of 8, 16, 32 or 64 chunks");
-    static_assert(NQ * 16 * 64 * 8 <= NQ * 2 * RL_SLOTS * 16, "the slices' totals fit the staging buffers");
-    __shared__ __attribute__((aligned(16))) double2 buf[NQ][2][RL_SLOTS];   // [wave][x, W][slot]; then the slices' totals
-    const int q = threadIdx.x >> 6, lane = lane_id(), tg = lane >> 3, eg = lane & 7;
-    const int tb = blockIdx.y * 32, eb = blockIdx.x * 32;
-    // the lane's staging share: 16-byte pieces f = lane + 64 k (k < 7) of the chunk's 448 (x rows first, then W rows)
-    const float * src[7]; int dst[7];
-#pragma unroll
-    for (int k = 0; k < 7; ++k) {
-        const int f = lane + 64 * k, op = f >= 224, g = f - 224 * op, r = g / 7, i = g % 7;
-        const int row = op ? (eb + r < n_exp ? eb + r : 0) : (tb + r < n ? tb + r : 0);
-        src[k] = (op ? W : x) + (size_t) row * K + 4 * i;
-        dst[k] = op * RL_SLOTS + ((i * 4 + (r & 3)) * 2) * 8 + (r >> 2);   // half 0; half 1 is 8 slots on
-    }
-    double2 * wb = &buf[q][0][0];
-    float4 nv[7];
-    auto fetch = [&](int c) {
-#pragma unroll
-        for (int k = 0; k < 7; ++k) { nv[k] = gloadf4(src[k] + CL * c); }
-    };
-    auto stage = [&]() {
-#pragma unroll
-        for (int k = 0; k < 7; ++k) {
-            wb[dst[k]] = make_double2((double) nv[k].x, (double) nv[k].y);
-            wb[dst[k] + 8] = make_double2((double) nv[k].z, (double) nv[k].w);
-        }
-    };
-    // chunk c's in-order sums for the lane's 4 x 4 logits, from the staged buffer
-    auto chunk = [&](RgAcc<4, 4> & s) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) { s.v[t][e] = 0.0; }
-        }
-#pragma unroll
-        for (int i = 0; i < 7; ++i) {
-            double xa[4][4], wa[4][4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const double2 v = wb[((i * 4 + t) * 2 + h) * 8 + tg];
-                    xa[t][2 * h] = v.x; xa[t][2 * h + 1] = v.y;
-                    const double2 u = wb[RL_SLOTS + ((i * 4 + t) * 2 + h) * 8 + eg];
-                    wa[t][2 * h] = u.x; wa[t][2 * h + 1] = u.y;
+                    for (int j = 0; j < 2; ++j) {
+                        acc.v[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double) p[i][s], (double) p[2 + j][s], st % 7 == 0 ? z : acc.v[i][j], 0, 0, 0);
+                    }
                 }
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) { s.v[t][e] = __builtin_fma(xa[t][j], wa[e][j], s.v[t][e]); }
+                if (st % 7 == 6) {
+                    if (ch == 0) { ev = acc; }
+                    else if (ch == 1) { rm_add(l1, ev, acc); }
+                    else if (ch == 2) { ev = acc; }
+                    else { rm_add(node, ev, acc); rm_add(node, l1, node); }
                 }
             }
         }
-    };
-    const int c0 = (KS == 1 ? 0 : (int) blockIdx.z * (256 / KS)) + q * CPW;
-    fetch(c0);
-    int cn = 0;   // chunks of the slice consumed
-    // one chunk: stage the fetched values, fetch the next chunk's, compute (a wave's LDS operations run in order, so the
-    // staging writes follow the previous chunk's reads)
-    auto next_chunk = [&](RgAcc<4, 4> & v) {
-        stage();
-        if (cn + 1 < CPW) { fetch(c0 + cn + 1); }
-        chunk(v);
-        ++cn;
-    };
-    // the slice's pairwise tree: 16-chunk groups built as the chunks arrive (binary counter), then levels 5 and 6
-    auto tile16 = [&]() {   // GN chunks (16; for 8-chunk slices the loop ends at c = 7 with v the group's total)
-        RgAcc<4, 4> pend[4], v;
-#pragma unroll 1
-        for (int c = 0; c < GN; ++c) {
-            next_chunk(v);
-            if (!(c & 1)) { pend[0] = v; continue; }
-            rg_add(v, pend[0], v);
-            if (!(c & 2)) { pend[1] = v; continue; }
-            rg_add(v, pend[1], v);
-            if (!(c & 4)) { pend[2] = v; continue; }
-            rg_add(v, pend[2], v);
-            if (!(c & 8)) { pend[3] = v; continue; }
-            rg_add(v, pend[3], v);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { raw[0][k] = raw[1][k]; }
+        // levels above 4 chunks: binary counter over the groups
+#pragma unroll
+        for (int l = 0; l < LG; ++l) {
+            if (!((g4 >> l) & 1)) { pend[l] = node; break; }
+            rm_add(node, pend[l], node);
         }
-        return v;
-    };
-    RgAcc<4, 4> tot, l4, l5;
-#pragma unroll 1
-    for (int g = 0; g < CPW / GN; ++g) {
-        RgAcc<4, 4> v = tile16();
-        if (LW <= 4) { tot = v; break; }
-        if (!(g & 1)) { l4 = v; continue; }
-        rg_add(v, l4, v);
-        if (LW == 5) { tot = v; break; }
-        if (!(g & 2)) { l5 = v; continue; }
-        rg_add(tot, l5, v);
     }
-    __syncthreads();   // every wave is done with its staging buffer: it now holds the slices' totals
-    double * part = reinterpret_cast<double *>(&buf[0][0][0]);   // [NQ][16][64]
+    // the next three levels over the workgroup's waves, pairwise in slice order: output o of the lane by wave o % 8
+    double * part = reinterpret_cast<double *>(rm_lds);   // [8 waves][16][64]
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int i = 0; i < 2; ++i) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) { part[(q * 16 + t * 4 + e) * 64 + lane] = tot.v[t][e]; }
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { part[(wave * 16 + (2 * i + j) * 4 + k) * 64 + lane] = node.v[i][j][k]; }
+        }
     }
     __syncthreads();
-    // the tree's top levels over the NQ slices, pairwise in slice order; output o of the lane by wave o % NQ
-    for (int o = q; o < 16; o += NQ) {
-        const int t = tb + tg * 4 + o / 4, e = eb + eg * 4 + o % 4;
-        double v[NQ];
+    for (int o = wave; o < 16; o += RM_W) {
+        double v[RM_W];
 #pragma unroll
-        for (int j = 0; j < NQ; ++j) { v[j] = part[(j * 16 + o) * 64 + lane]; }
+        for (int w = 0; w < RM_W; ++w) { v[w] = part[(w * 16 + o) * 64 + lane]; }
 #pragma unroll
-        for (int w = 1; w < NQ; w *= 2) {
+        for (int w = 1; w < RM_W; w *= 2) {
 #pragma unroll
-            for (int j = 0; j + w < NQ; j += 2 * w) { v[j] = v[j] + v[j + w]; }
+            for (int j = 0; j + w < RM_W; j += 2 * w) { v[j] = v[j] + v[j + w]; }
         }
+        const int t = tb + 16 * (o >> 3) + g + 4 * (o & 3), e = eb + 16 * ((o >> 2) & 1) + r;
         if (t < n && e < n_exp) {
             if constexpr (KS == 1) { logits[(size_t) t * n_exp + e] = (float) v[0]; }
             else { part2[((size_t) blockIdx.z * n + t) * n_exp + e] = v[0]; }
         }
     }
 }
-// the top levels of the K-split tree: the KS parts added pairwise in order, then rounded to fp32
-template <int KS>
-__global__ void __launch_bounds__(256) k_router_join(const double * __restrict__ part2, int total, float * __restrict__ logits) {
-#pragma clang fp contract(off)
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= total) { return; }
-    double v[KS];
-#pragma unroll
-    for (int j = 0; j < KS; ++j) { v[j] = part2[(size_t) j * total + i]; }
-#pragma unroll
-    for (int w = 1; w < KS; w *= 2) {
-#pragma unroll
-        for (int j = 0; j + w < KS; j += 2 * w) { v[j] = v[j] + v[j + w]; }
-    }
-    logits[i] = (float) v[0];
-}
 
-// the K split for n tokens: 16 parts from RL_SPLIT_MIN to RL_SPLIT_MAX tokens, else none
-static int router_split(int n, int n_exp, int K) {
+// parts of the chunks for n tokens: enough workgroups of a 32 x 32 tile for the CUs (0: the logits are written whole, by
+// k_router_mfma<1> above RM_MAX, which keeps the parts' scratch at 8 MiB)
+constexpr int RM_MIN = 17, RM_MAX = 2048;
+int router_parts(int n, int n_exp, int K) {
     (void) n_exp;
-    return K == 7168 && n >= RL_SPLIT_MIN && n <= RL_SPLIT_MAX ? 16 : 1;
+    return K != 7168 || n < RM_MIN || n > RM_MAX ? 0 : n <= 128 ? 8 : n <= 256 ? 4 : 2;
 }
-size_t router_split_doubles(int n, int n_exp, int K) {
-    const int ks = router_split(n, n_exp, K);
-    return ks > 1 ? (size_t) ks * n * n_exp : 0;
-}
+size_t router_part_doubles(int n, int n_exp, int K) { return (size_t) router_parts(n, n_exp, K) * n * n_exp; }
 
 hipError_t launch_router_logits(const float * W, const float * x, int n, int n_exp, int K, float * logits, double * part2, hipStream_t st) {
     if (n <= 0) { return hipSuccess; }
     if (K % 1024 != 0) { return hipErrorInvalidValue; }
-    // measured on MI355X (route call wall time): k_router_wg costs ~0.6 us per token (every workgroup reads all of x),
-    // 25 us at 32 tokens, 33 at 48; the split tiles 28 us to 64 tokens, 35 at 96, 53 at 255, 72 at 300, 103 at 512,
-    // 180 at 1024, 343 at 2048 (the whole tiles 375)
-    if (router_split(n, n_exp, K) > 1 && part2) {   // 32 x 32 tiles, the chunks split over 16 workgroups, then the join
-        const int total = n * n_exp;
-        k_router_lds<2, 16><<<dim3((n_exp + 31) / 32, (n + 31) / 32, 16), 128, 0, st>>>(W, x, n, n_exp, nullptr, part2);
-        k_router_join<16><<<dim3((total + 255) / 256), 256, 0, st>>>(part2, total, logits);
+    if (part2) {
+        const dim3 grid((n_exp + 31) / 32, (n + 31) / 32, router_parts(n, n_exp, K));
+        switch (grid.z) {
+        case 8: k_router_mfma<8><<<grid, RM_W * 64, RM_LDS, st>>>(W, x, n, n_exp, part2, logits); break;
+        case 4: k_router_mfma<4><<<grid, RM_W * 64, RM_LDS, st>>>(W, x, n, n_exp, part2, logits); break;
+        case 2: k_router_mfma<2><<<grid, RM_W * 64, RM_LDS, st>>>(W, x, n, n_exp, part2, logits); break;
+        default: return hipErrorInvalidValue;
+        }
         return hipGetLastError();
     }
-    if (K == 7168 && n >= 1024) {   // 32 x 32 tiles (4 x 4 per lane), staged in LDS
-        k_router_lds<4, 1><<<dim3((n_exp + 31) / 32, (n + 31) / 32), 256, 0, st>>>(W, x, n, n_exp, logits, nullptr);
+    if (K == 7168 && n > RM_MAX) {
+        k_router_mfma<1><<<dim3((n_exp + 31) / 32, (n + 31) / 32), RM_W * 64, RM_LDS, st>>>(W, x, n, n_exp, nullptr, logits);
         return hipGetLastError();
     }
-    if (K == 7168 && n >= RW_MAXN) {   // 32 x 16 tiles (4 x 2 per lane)
-        k_router_tile<4, 2, 4><<<dim3((n_exp + 15) / 16, (n + 31) / 32), 256, 0, st>>>(W, x, n, n_exp, logits);
-        return hipGetLastError();
-    }
-    if (K == 7168) {
+    if (K == 7168 && n <= RW_MAXN) {
         k_router_wg<<<dim3(n_exp), 256, 0, st>>>(W, x, n, n_exp, logits);
         return hipGetLastError();
     }
@@ -476,8 +313,10 @@ hipError_t launch_router_logits(const float * W, const float * x, int n, int n_e
 }
 
 // one wave per token; lane l holds experts 4l..4l+3 (n_exp <= 256); the rule is select_token's (moe_device.h), with
-// keep entries per token written (keep = topk: all of them)
-__global__ void __launch_bounds__(64) k_router_select(const float * __restrict__ logits, const float * __restrict__ bias, int n, int n_exp,
+// keep entries per token written (keep = topk: all of them). KS > 0: the logits arrive as KS parts of the contract's tree
+// (k_router_mfma), added pairwise in order and rounded here, and are written out too.
+template <int KS>
+__global__ void __launch_bounds__(64) k_router_select(float * __restrict__ logits, const double * __restrict__ part2, const float * __restrict__ bias, int n, int n_exp,
                                                       int n_group, int topk_group, int topk, float scale, int keep, float renorm,
                                                       float * __restrict__ probs, int * __restrict__ sel, float * __restrict__ wts) {
     __shared__ float scr[NEXP_MAX + 2 * 64];
@@ -486,7 +325,22 @@ __global__ void __launch_bounds__(64) k_router_select(const float * __restrict__
     float lg[4], bv[4];
     load_bias(bias, n_exp, bv);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) { const int e = 4 * lane + j; lg[j] = e < n_exp ? logits[(size_t) t * n_exp + e] : 0.f; }
+    for (int j = 0; j < 4; ++j) {
+        const int e = 4 * lane + j;
+        if constexpr (KS == 0) { lg[j] = e < n_exp ? logits[(size_t) t * n_exp + e] : 0.f; }
+        else {
+            double v[KS];
+#pragma unroll
+            for (int k = 0; k < KS; ++k) { v[k] = e < n_exp ? part2[((size_t) k * n + t) * n_exp + e] : 0.0; }
+#pragma unroll
+            for (int w = 1; w < KS; w *= 2) {
+#pragma unroll
+                for (int k = 0; k + w < KS; k += 2 * w) { v[k] = v[k] + v[k + w]; }
+            }
+            lg[j] = (float) v[0];
+            if (e < n_exp) { logits[(size_t) t * n_exp + e] = lg[j]; }
+        }
+    }
     select_token(lg, bv, n_exp, n_group, topk_group, topk, scale, scr, so, wo, probs ? probs + (size_t) t * n_exp : nullptr, keep, renorm);
     lds_visible();
     if (lane < keep) { sel[(size_t) t * keep + lane] = so[lane]; wts[(size_t) t * keep + lane] = wo[lane]; }
@@ -540,12 +394,19 @@ hipError_t launch_keep_share(const int * sel8, const float * w8, int n, int topk
     return hipGetLastError();
 }
 
-hipError_t launch_router_select(const float * logits, const float * bias, int n, int n_exp, int n_group, int topk_group,
+hipError_t launch_router_select(float * logits, const double * part2, int K, const float * bias, int n, int n_exp, int n_group, int topk_group,
                                 int topk, float scale, float * probs, int * sel, float * wts, hipStream_t st, int keep, float renorm) {
     if (n <= 0) { return hipSuccess; }
     if (keep <= 0) { keep = topk; }
     if (!select_rule_ok(n_exp, n_group, topk_group, topk, keep)) { return hipErrorInvalidValue; }
-    k_router_select<<<n, 64, 0, st>>>(logits, bias, n, n_exp, n_group, topk_group, topk, scale, keep, renorm, probs, sel, wts);
+    auto go = [&](auto kernel) { kernel<<<n, 64, 0, st>>>(logits, part2, bias, n, n_exp, n_group, topk_group, topk, scale, keep, renorm, probs, sel, wts); };
+    switch (part2 ? router_parts(n, n_exp, K) : 0) {
+    case 0: go(k_router_select<0>); break;
+    case 2: go(k_router_select<2>); break;
+    case 4: go(k_router_select<4>); break;
+    case 8: go(k_router_select<8>); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 

@@ -895,3 +895,24 @@ def test_few_slot_columns_match_per_pass(ctx, n, hot):
     got = _prefill_state(ctx, layer, x, True)
     for k in ref:
         assert np.array_equal(got[k].view(np.uint8), ref[k].view(np.uint8)), k
+
+
+@pytest.mark.parametrize("n", [9, 16, 31, 32, 33, 128, 129, 256, 257, 2049])
+def test_router_parts_bitwise(ctx, n):
+    """The router on the fp64 matrix cores (from 9 tokens): the edges of its 32-token tiles and of the chunk split (8, 4,
+    2 parts and whole logits), with rows of very different sizes and rows that cancel almost completely. Logits bit for
+    bit the checker's."""
+    import torch
+    rng = np.random.default_rng(n)
+    W = (rng.standard_normal((NEXP, E)) * 0.02).astype(np.float32)
+    x = (rng.standard_normal((n, E)) * np.exp2(rng.integers(-12, 12, (n, 1)))).astype(np.float32)
+    x[0, 1::2] = -x[0, ::2]
+    W[::7, 1::2] = W[::7, ::2]
+    b = (rng.standard_normal(NEXP) * 0.05).astype(np.float32)
+    lg, pr, sel, w = ctx.route(torch.from_numpy(W).cuda(), torch.from_numpy(b).cuda(), torch.from_numpy(x).cuda())
+    ctx.sync()
+    rows = np.arange(n) if n <= 257 else np.r_[0:64, n - 64:n]
+    l0, p0, s0, w0 = orc.router(W, b, x[rows])
+    assert np.array_equal(lg.cpu().numpy()[rows].view(np.uint32), l0.view(np.uint32))
+    assert np.array_equal(pr.cpu().numpy()[rows].view(np.uint32), p0.view(np.uint32))
+    assert np.array_equal(sel.cpu().numpy()[rows], s0) and np.array_equal(w.cpu().numpy()[rows].view(np.uint32), w0.view(np.uint32))
