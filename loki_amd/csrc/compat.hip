@@ -341,9 +341,9 @@ static void shared_expert(FLCtx * c, Compat * s, const int8_t * xq, const float 
         CK(prefill_ready(c) == FL_OK ? hipSuccess : hipErrorOutOfMemory);
         // shared columns only (wide_base runs every row of a wide pass here, so N is not bounded by 64): one table for the
         // IQ2_XXS GEMMs, one for the K-quant GEMM
-        FALLOC(s->pcols, (size_t) prefill_shared_cols(N, FEW_TOK) + prefill_shared_cols(N, KQ_TOK)); FALLOC(s->pncols, 2 * PF_NCOLS);
-        iq = { s->pcols.p, s->pncols.p, pf_tok(N), pf_few(N) };
-        kt = { s->pcols.p + prefill_shared_cols(N, FEW_TOK), s->pncols.p + PF_NCOLS, KQ_TOK, 0 };
+        FALLOC(s->pcols, (size_t) prefill_shared_cols(N, FEW_TOK) + prefill_shared_cols(N, 16)); FALLOC(s->pncols, 2 * PF_NCOLS);
+        iq = { s->pcols.p, s->pncols.p, pf_tok(N), pf_few(N), pf_tok(N) };
+        kt = { s->pcols.p + prefill_shared_cols(N, FEW_TOK), s->pncols.p + PF_NCOLS, KQ_TOK, 0, kq_shared_tok(N) };
         FCK(launch_prefill_cols(zero_int(c), zero_int(c), zero_int(c), N, 0, iq, kt, c->st));
         g.ptab = c->ptab.p; g.tab = c->tab.p; g.perm = zero_int(c); g.topk = 1; g.P = 0; g.most = N;
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
@@ -362,10 +362,9 @@ static void shared_expert(FLCtx * c, Compat * s, const int8_t * xq, const float 
             FCK(launch_q8_to_h(xq, s->xh.p, (int64_t) N * E_, c->st));
             k.cols = kt.cols; k.ncols = kt.ncols; k.bh = s->xh.p;
             FALLOC(s->sg, (size_t) N * H_); FALLOC(s->su, (size_t) N * H_);
-            for (int m = 0; m < 2; ++m) {
-                k.sh[0] = k.w[0] = (const uint8_t *) s->sh_key[m]; k.nmat = 1; k.out = m ? s->su.p : s->sg.p;
-                FCK(launch_kq_gemm(k, FL_Q5K, c->ncu, c->st));
-            }
+            k.sh[0] = k.w[0] = (const uint8_t *) s->sh_key[0]; k.sh[1] = (const uint8_t *) s->sh_key[1];
+            k.nmat = 1; k.out = s->sg.p; k.udbg = s->su.p;
+            FCK(launch_kq_gemm(k, FL_Q5K, c->ncu, c->st));
             FCK(launch_swiglu(s->sg.p, s->su.p, (int64_t) N * H_, s->h.p, c->st));
         }
         FCK(launch_quant_q8k(s->h.p, N, H_, s->hq.p, s->hd.p, c->st));
@@ -395,8 +394,7 @@ static void shared_expert(FLCtx * c, Compat * s, const int8_t * xq, const float 
             k.w[0] = k.sh[0] = tm[2]; k.cols = iq.cols; k.ncols = iq.ncols;
             FCK(iq2_gemm(k, c->ncu, c->st));
         } else {
-            FALLOC(s->hh, (size_t) N * H_);
-            FCK(launch_q8_to_h(s->hq.p, s->hh.p, (int64_t) N * H_, c->st));
+            if (s->shf[2] == FL_Q6K) { FALLOC(s->hh, (size_t) N * H_); FCK(launch_q8_to_h(s->hq.p, s->hh.p, (int64_t) N * H_, c->st)); }
             k.cols = kt.cols; k.ncols = kt.ncols; k.bh = s->hh.p;
             k.w[0] = k.sh[0] = (const uint8_t *) s->sh_key[2];
             FCK(launch_kq_gemm(k, s->shf[2], c->ncu, c->st));
@@ -444,8 +442,8 @@ static void routed_experts(FLCtx * c, Compat * s, const Arena & ar, const int8_t
         hipStream_t st = c->st;
         const size_t nc = (size_t) P / pf_tok(n) + NEXP_MAX + 4;   // entries of the first table
         FALLOC(s->pcols, nc + (size_t) P / KQ_TOK + NEXP_MAX + 4); FALLOC(s->pncols, 2 * PF_NCOLS);
-        const PfTable iq = { s->pcols.p, s->pncols.p, pf_tok(n), pf_few(n) };
-        const PfTable kt = { down_fmt == FL_IQ2 ? nullptr : s->pcols.p + nc, s->pncols.p + PF_NCOLS, KQ_TOK, 0 };
+        const PfTable iq = { s->pcols.p, s->pncols.p, pf_tok(n), pf_few(n), pf_tok(n) };
+        const PfTable kt = { down_fmt == FL_IQ2 ? nullptr : s->pcols.p + nc, s->pncols.p + PF_NCOLS, KQ_TOK, 0, KQ_TOK };
         const auto iq2_gemm = iq.tok == FEW_TOK ? launch_few_gemm : launch_prefill_gemm;
         FCK(launch_prefill_cols(act, nact, offsets, 0, P, iq, kt, st));
         PrefillArgs g{};
@@ -460,10 +458,8 @@ static void routed_experts(FLCtx * c, Compat * s, const Arena & ar, const int8_t
             d.w[0] = ar.d; d.sh[0] = ar.d; d.estride = mat_bytes(E_, H_);
             FCK(iq2_gemm(d, c->ncu, st));
         } else {   // src/fused_layer.cu:607-608 (tc_matvec<F_Q2K / F_Q3K>)
-            FALLOC(s->hh, (size_t) P * H_);
-            FCK(launch_q8_to_h(s->hq.p, s->hh.p, (int64_t) P * H_, st));
             d.w[0] = (const uint8_t *) down; d.sh[0] = (const uint8_t *) down; d.estride = fmt_bytes(down_fmt, E_, H_);
-            d.cols = kt.cols; d.ncols = kt.ncols; d.bh = s->hh.p;
+            d.cols = kt.cols; d.ncols = kt.ncols;
             FCK(launch_kq_gemm(d, down_fmt, c->ncu, st));
         }
         return;

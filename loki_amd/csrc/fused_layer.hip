@@ -559,6 +559,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     const bool kq1 = kq && kd1 != 0 && n == 1 && tsel == MAXK && tk == MAXK && decode1_ready(c);
     const bool fused = (!kq || kq1) && c->fused && n <= 8 && E == 7168 && H == 2048 && decode_rule_ok(ne, c->n_group) && decode_ready(c);
     const bool mfma = !fused && c->pf_mfma && n > 8 && E == 7168 && H == 2048;
+    const bool q5 = lf[1] == FL_Q5K && lf[2] == FL_Q5K, q6 = lf[3] == FL_Q6K;   // shared matrices on fp16 activations
     ALLOC(c, c->xq, (size_t) n * E); ALLOC(c, c->xd, (size_t) n * (E / 256));
     ALLOC(c, c->logits, (size_t) n * ne); ALLOC(c, c->probs, (size_t) n * ne);
     ALLOC(c, c->sel, P); ALLOC(c, c->wts, P); ALLOC(c, c->perm, P); ALLOC(c, c->inv, P);
@@ -593,7 +594,9 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     if (mfma) {
         if (int rc = prefill_ready(c)) { return rc; }
         ALLOC(c, c->pcols, rows / pf_tok(n) + NEXP_MAX + 4); ALLOC(c, c->pncols, 2 * PF_NCOLS);
-        if (kq) { ALLOC(c, c->xh, (size_t) n * E); ALLOC(c, c->hh, rows * H); ALLOC(c, c->pcolsk, rows / KQ_TOK + NEXP_MAX + 4); }
+        if (kq) { ALLOC(c, c->pcolsk, P / KQ_TOK + n / 16 + NEXP_MAX + 4); }
+        if (q5) { ALLOC(c, c->xh, (size_t) n * E); }
+        if (q6) { ALLOC(c, c->hh, (size_t) n * H); }
     }
     prof_mark(c, ev, 0);
     if (prenorm) {   // the per-pass path normalises into a context buffer first (k_rmsnorm: the same arithmetic)
@@ -602,7 +605,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         x = c->xn.p;
     }
     TRY(c, launch_quant_q8k(x, n, E, c->xq.p, c->xd.p, st));
-    if (mfma && kq) { TRY(c, launch_q8_to_h(c->xq.p, c->xh.p, (int64_t) n * E, st)); }
+    if (mfma && q5) { TRY(c, launch_q8_to_h(c->xq.p, c->xh.p, (int64_t) n * E, st)); }
     prof_mark(c, ev, 1);
     double * rp = nullptr;   // the matrix-core kernel's parts
     if (const size_t nd = router_part_doubles(n, ne, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
@@ -620,14 +623,14 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     if (const size_t nd = dispatch_scratch_ints(P)) { ALLOC(c, c->dscr, nd); dsc = c->dscr.p; }
     TRY(c, launch_dispatch(c->sel.p, P, ne, c->counts.p, c->offsets.p, c->perm.p, c->inv.p, c->act.p, c->nact.p, st, dsc));
     if (mfma) {
-        const PfTable iq = { c->pcols.p, c->pncols.p, pf_tok(n), pf_few(n) };
-        const PfTable kt = { kq ? c->pcolsk.p : nullptr, c->pncols.p + PF_NCOLS, KQ_TOK, 0 };
+        const PfTable iq = { c->pcols.p, c->pncols.p, pf_tok(n), pf_few(n), pf_tok(n) };
+        const PfTable kt = { kq ? c->pcolsk.p : nullptr, c->pncols.p + PF_NCOLS, KQ_TOK, 0, kq_shared_tok(n) };
         TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, n, P, iq, kt, st));
         prof_mark(c, ev, 4);
         // Columns: the shared expert's first (nsh of them), then the routed experts'. Each matrix runs where its format
         // does: IQ2_XXS on the IQ2_XXS GEMM, Q2_K / Q3_K / Q6_K downs and a Q5_K shared gate / up on the K-quant GEMM,
         // any other K-quant on the mat-vecs.
-        const int nsh = prefill_shared_cols(n, KQ_TOK), nshi = prefill_shared_cols(n, iq.tok);   // K-quant, IQ2_XXS tables
+        const int nsh = prefill_shared_cols(n, kt.stok), nshi = prefill_shared_cols(n, iq.tok);   // K-quant, IQ2_XXS tables
         const auto iq2_gemm = iq.tok == FEW_TOK ? launch_few_gemm : launch_prefill_gemm;
         PrefillArgs g{};
         g.ptab = c->ptab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
@@ -638,25 +641,23 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
         g.col0 = lf[1] == FL_IQ2 ? 0 : nshi;
         TRY(c, iq2_gemm(g, c->ncu, st));
-        if (lf[1] == FL_Q5K && lf[2] == FL_Q5K) {   // the real shards' shared gate / up: ksg / ksu rows 0 .. n - 1
+        if (q5) {   // the real shards' shared gate / up: ksg / ksu rows 0 .. n - 1
             ALLOC(c, c->ksg, (size_t) n * H); ALLOC(c, c->ksu, (size_t) n * H);
-            for (int m = 0; m < 2; ++m) {
-                PrefillArgs k{};
-                k.sh[0] = (const uint8_t *) (m ? L->sh_up : L->sh_gate); k.w[0] = k.sh[0];
-                k.R = H; k.K = E; k.cols = kt.cols; k.ncols = kt.ncols; k.col0 = 0; k.col1 = nsh;
-                k.bh = c->xh.p; k.bd = c->xd.p; k.arow0 = P; k.orow0 = P; k.out = m ? c->ksu.p : c->ksg.p;
-                TRY(c, launch_kq_gemm(k, FL_Q5K, c->ncu, st));
-            }
+            PrefillArgs k{};
+            k.sh[0] = k.w[0] = (const uint8_t *) L->sh_gate; k.sh[1] = (const uint8_t *) L->sh_up;
+            k.R = H; k.K = E; k.cols = kt.cols; k.ncols = kt.ncols; k.col0 = 0; k.col1 = nsh;
+            k.bh = c->xh.p; k.bd = c->xd.p; k.arow0 = P; k.orow0 = P; k.out = c->ksg.p; k.udbg = c->ksu.p;
+            TRY(c, launch_kq_gemm(k, FL_Q5K, c->ncu, st));
             if (int rc = shared_swiglu(c, n, P, H, st)) { return rc; }
         } else if (lf[1] != FL_IQ2) {
             if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, st)) { return rc; }
         }
         TRY(c, launch_quant_q8k(c->h.p, (int64_t) rows, H, c->hq.p, c->hd.p, st));
-        if (kq) { TRY(c, launch_q8_to_h(c->hq.p, c->hh.p, (int64_t) rows * H, st)); }
+        if (q6) { TRY(c, launch_q8_to_h(c->hq.p + (size_t) P * H, c->hh.p, (int64_t) n * H, st)); }
         prof_mark(c, ev, 5);
         PrefillArgs d = g;   // the down pass: activations Q8_K(h) of every slot, o rows by slot
         d.w[0] = (const uint8_t *) L->down_exps; d.w[1] = nullptr; d.sh[0] = (const uint8_t *) L->sh_down; d.sh[1] = nullptr;
-        d.R = E; d.K = H; d.nmat = 1; d.bq = c->hq.p; d.bh = c->hh.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr;
+        d.R = E; d.K = H; d.nmat = 1; d.bq = c->hq.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr;
         const bool sh_iq = lf[3] == FL_IQ2, sh_kg = lf[3] == FL_Q2K || lf[3] == FL_Q3K || lf[3] == FL_Q6K;
         if (lf[0] == FL_IQ2) {   // routed (+ the shared expert when it is IQ2_XXS)
             d.col0 = sh_iq ? 0 : nshi;
@@ -670,6 +671,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         if (sh_kg) {
             PrefillArgs k = d;
             k.cols = kt.cols; k.ncols = kt.ncols; k.col0 = 0; k.col1 = nsh;
+            if (q6) { k.bh = c->hh.p; k.bd = c->hd.p + (size_t) P * (H / 256); k.arow0 = P; }   // (the shared rows alone)
             TRY(c, launch_kq_gemm(k, lf[3], c->ncu, st));
         } else if (!sh_iq) {
             if (int rc = shared_down_sep(c, L, n, P, E, H, tk, st)) { return rc; }

@@ -1,14 +1,12 @@
-// kq_gemm.hip -- K-quant matrices (the real shards' formats: routed down Q2_K / Q3_K, shared expert Q5_K / Q5_K /
-// Q6_K) on the matrix cores at prefill sizes.
+// kq_gemm.hip -- the shared expert's K-quant matrices (the real shards' Q5_K gate / up and Q6_K down) on the matrix cores
+// at prefill sizes; the routed downs' formats (Q2_K, Q3_K) are kq8_gemm.hip's.
 //
-// Reference: the K-quant mat-vecs of the wide pass (tc_matvec<F_Q2K/F_Q3K/F_Q5K/F_Q6K>, src/fused_layer.cu:102-158,
-// 203-254, launched at 520-524 and 541-550). The arithmetic is ggml_vec_dot_q{2,3,5,6}_K_q8_K's as the K-quant
-// mat-vec (kquant.hip) restates it, and the outputs are bit-identical to that kernel's: per block the exact integer
-// sums isum = sum_j sc_j sum_i q_i x_i (q the stored value minus its offset: Q3_K 4, Q6_K 32) and, for Q2_K / Q5_K,
-// summ = sum_j mn_j bsum_j; then over the blocks in order
-//   Q2_K         acc += (d8 * d) * isum - (d8 * dmin) * summ
-//   Q3_K, Q6_K   acc += (d * d8) * isum
-//   Q5_K         acc_s += (d * d8) * isum, acc_m -= (dmin * d8) * summ, result acc_m + acc_s
+// Reference: the K-quant mat-vecs of the wide pass (tc_matvec<F_Q5K/F_Q6K>, src/fused_layer.cu:102-158, launched at
+// 520-524). The arithmetic is ggml_vec_dot_q{5,6}_K_q8_K's as the K-quant mat-vec (kquant.hip) restates it, and the outputs
+// are bit-identical to that kernel's: per block the exact integer sums isum = sum_j sc_j sum_i q_i x_i (q the stored value
+// minus its offset: Q6_K 32) and, for Q5_K, summ = sum_j mn_j bsum_j; then over the blocks in order
+//   Q6_K   acc += (d * d8) * isum
+//   Q5_K   acc_s += (d * d8) * isum, acc_m -= (dmin * d8) * summ, result acc_m + acc_s
 // with isum and summ rounded to fp32 once.
 //
 // The integer sums come from v_mfma_f32_16x16x32_f16 chains per 16 x 16 (token, row) tile, the activations being the
@@ -16,20 +14,18 @@
 // 1024 + u by one byte permute, and fma(1024 + u, sc, -1024 sc) = u * sc is exact whenever |u * sc| <= 2048 (the fma
 // rounds once and fp16 holds every integer up to 2048; Q6_K, whose 8-bit scales make -1024 sc overflow fp16, takes
 // (1024 + u - 1024) * sc instead). The chains:
-//   A    sum u * sc * x   (Q6_K: u's low 4 bits; |u * sc| <= 7 * 32 (Q3_K), 3 * 15 (Q2_K), 31 * 63 (Q5_K), 15 * 128)
+//   A    sum u * sc * x   (Q6_K: u's low 4 bits; |u * sc| <= 31 * 63 (Q5_K), 15 * 128)
 //   A2   sum (u >> 4) * sc * x                              (Q6_K only: |.| <= 3 * 128)
-//   B    sum v * x, v the sub-block's scale (Q3_K, Q6_K: the offset term) or min (Q2_K, Q5_K)
-// and isum = A (Q2_K, Q5_K), A - 4 B (Q3_K), A + 16 A2 - 32 B (Q6_K); summ = B. A chain's products and partial sums
-// are integers, so it is exact whatever order the matrix core adds in while every partial sum stays below 2^24: A runs
-// over segments of SEG steps of 32 products (Q2_K, Q3_K: the whole block, at most 256 * 224 * 127 < 7.3e6; Q5_K,
-// Q6_K: two steps, at most 64 * 1953 * 127 < 1.6e7), A2 and B over the whole block; the segment totals are converted
-// to int32 (exactly) and the block sums formed in int32.
+//   B    sum v * x, v the sub-block's scale (Q6_K: the offset term) or min (Q5_K)
+// and isum = A (Q5_K) or A + 16 A2 - 32 B (Q6_K); summ = B. A chain's products and partial sums are integers, so it is
+// exact whatever order the matrix core adds in while every partial sum stays below 2^24: A runs over segments of two steps
+// of 32 products (at most 64 * 1953 * 127 < 1.6e7), A2 and B over the whole block; the segment totals are converted to int32
+// (exactly) and the block sums formed in int32.
 //
-// Work: as the IQ2_XXS grouped GEMM (moe_prefill.hip): a column is up to 64 dispatch slots of one expert (or of the
-// shared expert), an item is (column, 128 rows), one 8-wave workgroup per CU takes the items round-robin. Wave w owns
-// one 16-row tile (two spill: the slices' raw bytes are double-buffered in registers); lane (r, g) holds row r of the
-// tile and the lane slices 2 g, 2 g + 1 of each block (kquant_device.h's slices, 32 weights each). Step t of lane
-// group g covers 8 of them (slice 2 g + t / 4): Q2_K / Q3_K / Q6_K piece t % 4, block weights 128 n + 32 s + 8 jq ..
+// Work: a column is up to 64 dispatch slots of the expert, an item is (column, 128 rows), one 8-wave workgroup per CU takes
+// the items round-robin. Wave w owns one 16-row tile (two spill: the slices' raw bytes are double-buffered in registers);
+// lane (r, g) holds row r of the tile and the lane slices 2 g, 2 g + 1 of each block (kquant_device.h's slices, 32 weights
+// each). Step t of lane group g covers 8 of them (slice 2 g + t / 4): Q6_K piece t % 4, block weights 128 n + 32 s + 8 jq ..
 // + 7 (n = g / 2, s = t % 4, jq = 2 (g % 2) + t / 4); Q5_K half t % 2 of piece (t % 4) / 2, weights
 // 64 g + 32 h + 16 k + 8 e .. + 7 (h = (t % 4) / 2, k = t / 4, e = t % 2). The activation operand reads the same 8
 // positions, so both operands permute K alike. The column's activations go block by block from memory into LDS
@@ -89,9 +85,8 @@ template <bool BIG> __device__ __forceinline__ kh8 kg_weights(uint32_t u0, uint3
 
 template <int F> struct KgFmt {
     static constexpr bool Q5 = F == KF_Q5K, Q6 = F == KF_Q6K;
-    static constexpr bool MINS = F == KF_Q2K || F == KF_Q5K;   // summ terms
-    static constexpr int SEG = (Q5 || Q6) ? 2 : 8;              // steps per exact segment of chain A
-    static constexpr bool NT4 = !(Q5 || Q6);   // four token tiles per pass (Q5_K / Q6_K: two, a 64-slot column in two passes; four spill)
+    static constexpr bool MINS = Q5;           // summ terms
+    static constexpr int SEG = 2;              // steps per exact segment of chain A
 };
 
 template <int F, int NB>
@@ -109,13 +104,16 @@ __global__ void __launch_bounds__(KG_NT, 1) k_kq_gemm(const PrefillArgs a) {
     const int nrg = a.R / KG_ROWS;
     const uint32_t mbytes = (uint32_t) a.R * ROWB;   // one matrix
 
-    for (int it = blockIdx.x; it < ncols * nrg; it += gridDim.x) {
-        const int col = col0 + it / nrg, rg = it % nrg;
+    const int per = ncols * nrg, items = Fm::Q5 && a.udbg ? 2 * per : per;   // (a second matrix: its items after the first's)
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        const bool second = item >= per;
+        const int it = second ? item - per : item, col = col0 + it / nrg, rg = it % nrg;
+        float * out = second ? a.udbg : a.out;
         const u32x4 cv = *(const LK_GLOBAL u32x4 *) (a.cols + col);
         const bool routed = (int) cv.x >= 0;
         const int e = (int) cv.w;
         const __amdgpu_buffer_rsrc_t rb = kg_rsrc(a.bh, 0x7fffffff), rd = kg_rsrc(a.bd, 0x7fffffff);
-        const uint8_t * W = routed ? a.w[0] + (size_t) e * a.estride : a.sh[0];
+        const uint8_t * W = routed ? a.w[0] + (size_t) e * a.estride : a.sh[second ? 1 : 0];
         Src src;
         src.rs = kg_rsrc(kg_uniform(W), mbytes);
         src.vb = (uint32_t) r * ROWB;
@@ -212,8 +210,7 @@ __global__ void __launch_bounds__(KG_NT, 1) k_kq_gemm(const PrefillArgs a) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int b = (int) cb[tt][i];
-                        if constexpr (F == KF_Q3K) { is[tt][i] -= 4 * b; }
-                        else if constexpr (Fm::Q6) { is[tt][i] += 16 * (int) ca2[tt][i] - 32 * b; }
+                        if constexpr (Fm::Q6) { is[tt][i] += 16 * (int) ca2[tt][i] - 32 * b; }
                         else { sm[tt][i] = b; }
                     }
                 }
@@ -224,9 +221,7 @@ __global__ void __launch_bounds__(KG_NT, 1) k_kq_gemm(const PrefillArgs a) {
                     for (int i = 0; i < 4; ++i) {
                         const float d8 = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (16 * tt + 4 * g + i), __builtin_bit_cast(int, dxl)));
                         const float fi = (float) is[tt][i];
-                        if constexpr (F == KF_Q2K) {
-                            acc[tt][i] = acc[tt][i] + ((d8 * dd) * fi - (d8 * dm) * (float) sm[tt][i]);
-                        } else if constexpr (Fm::Q5) {
+                        if constexpr (Fm::Q5) {
                             acc[tt][i] = acc[tt][i] + (dd * d8) * fi;
                             accm[tt][i] = accm[tt][i] - (dm * d8) * (float) sm[tt][i];
                         } else {
@@ -260,14 +255,13 @@ __global__ void __launch_bounds__(KG_NT, 1) k_kq_gemm(const PrefillArgs a) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int n = 16 * tt + 4 * g + i;
-                    if (n < sc) { a.out[(size_t) (sb - a.orow0 + n) * a.R + row] = Fm::Q5 ? accm[tt][i] + acc[tt][i] : acc[tt][i]; }
+                    if (n < sc) { out[(size_t) (sb - a.orow0 + n) * a.R + row] = Fm::Q5 ? accm[tt][i] + acc[tt][i] : acc[tt][i]; }
                 }
             }
         };
         const int sb = (int) cv.y, sc = (int) cv.z;
-        if (sc > 32) {
-            if constexpr (Fm::NT4) { run_item(std::integral_constant<int, 4>{}, sb, sc); }
-            else { run_item(std::integral_constant<int, 2>{}, sb, 32); run_item(std::integral_constant<int, 2>{}, sb + 32, sc - 32); }
+        if (sc > 32) {   // two passes of two token tiles: four spill
+            run_item(std::integral_constant<int, 2>{}, sb, 32); run_item(std::integral_constant<int, 2>{}, sb + 32, sc - 32);
         } else if (sc > 16) { run_item(std::integral_constant<int, 2>{}, sb, sc); }
         else { run_item(std::integral_constant<int, 1>{}, sb, sc); }
         __syncthreads();   // the LDS buffers are refilled by the next item
@@ -282,24 +276,21 @@ template <int F, int NB> void kg_go(const PrefillArgs & a, int grid, hipStream_t
 }  // namespace
 
 hipError_t kq_gemm_init() {
-    hipError_t e = kg_setup<KF_Q2K, 8>();
-    if (e == hipSuccess) { e = kg_setup<KF_Q3K, 8>(); }
-    if (e == hipSuccess) { e = kg_setup<KF_Q6K, 8>(); }
+    hipError_t e = kg_setup<KF_Q6K, 8>();
     if (e == hipSuccess) { e = kg_setup<KF_Q5K, 28>(); }
-    return e;
+    return e == hipSuccess ? kq8_gemm_init() : e;
 }
 
 hipError_t launch_kq_gemm(const PrefillArgs & a, int fmt, int grid, hipStream_t st) {
+    if (kq8_gemm_takes(fmt, a.K, a.R)) { return launch_kq8_gemm(a, fmt, grid, st); }
     const int nb = a.K / QK;
-    const bool down = nb == 8 && (fmt == KF_Q2K || fmt == KF_Q3K || fmt == KF_Q6K), gu = nb == 28 && fmt == KF_Q5K;
+    const bool down = nb == 8 && fmt == KF_Q6K, gu = nb == 28 && fmt == KF_Q5K;
     if (grid < 1 || !a.cols || !a.ncols || !a.bh || !a.bd || !a.out || a.K % QK || a.R % KG_ROWS || !(down || gu) || a.col0 < 0 ||
         ((reinterpret_cast<uintptr_t>(a.w[0]) | reinterpret_cast<uintptr_t>(a.sh[0]) | a.estride) & 3u) ||
         (uint64_t) a.R * nb * kq_block_bytes(fmt) >= 0x7fffffffull) {
         return hipErrorInvalidValue;
     }
-    if (fmt == KF_Q2K) { kg_go<KF_Q2K, 8>(a, grid, st); }
-    else if (fmt == KF_Q3K) { kg_go<KF_Q3K, 8>(a, grid, st); }
-    else if (fmt == KF_Q6K) { kg_go<KF_Q6K, 8>(a, grid, st); }
+    if (fmt == KF_Q6K) { kg_go<KF_Q6K, 8>(a, grid, st); }
     else { kg_go<KF_Q5K, 28>(a, grid, st); }
     return hipGetLastError();
 }

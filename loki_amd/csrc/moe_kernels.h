@@ -132,13 +132,13 @@ size_t decode1_lds_bytes();
 hipError_t launch_moe_decode1(const DecodeArgs & a, bool cooperative, hipStream_t st);
 
 // Column tables. launch_prefill_cols cuts every expert's slots (the shared expert's first) into columns of at most tok
-// slots, the fewest possible and of equal size (rounded up to 16); the routed columns are ordered by class. Sized >= P /
-// tok + n / tok + NEXP_MAX + 2 entries. Classes by slots: broad 65..112, wide 33..64, narrow few + 1..32, few 1..few.
+// slots (the shared expert's stok), the fewest possible and of equal size (rounded up to 16); the routed columns are ordered
+// by class. Sized >= P / tok + n / stok + NEXP_MAX + 2 entries. Classes by slots: broad 65..112, wide 33..64, narrow few + 1..32, few 1..few.
 // ncols[0] all columns; [1 + k] end of the shared columns of class k; [PF_NCLS + 1 + k] end of the routed ones.
 constexpr int PF_TOK = 112, KQ_TOK = 64, FEW_TOK = 8;   // tok of the IQ2_XXS GEMMs, the K-quant GEMM, the few kernel
 enum { PF_BROAD = 0, PF_WIDE = 1, PF_NARROW = 2, PF_FEW = 3, PF_NCLS = 4 };
 constexpr int PF_NCOLS = 2 * PF_NCLS + 1;
-struct PfTable { int4 * cols; int * ncols; int tok, few; };
+struct PfTable { int4 * cols; int * ncols; int tok, few, stok; };
 // one or two tables (t1.cols may be null)
 hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, const PfTable & t0, const PfTable & t1, hipStream_t st);
 constexpr int prefill_shared_cols(int n, int tok) { return (n + tok - 1) / tok; }   // the shared expert's columns (the first ones)
@@ -146,6 +146,8 @@ constexpr int prefill_shared_cols(int n, int tok) { return (n + tok - 1) / tok; 
 // PF_FEW_N the columns of at most 8 run on the few kernel, above on the narrow one
 constexpr int PF_SPLIT_N = 128, PF_FEW_N = 256;
 constexpr int pf_tok(int n) { return n <= PF_SPLIT_N ? FEW_TOK : PF_TOK; }
+// the K-quant shared expert's columns: enough (column, 128 rows) items of its gate and up for the 256 CUs
+constexpr int kq_shared_tok(int n) { return n <= 128 ? 16 : n <= 256 ? 32 : KQ_TOK; }
 constexpr int pf_few(int n) { return n <= PF_FEW_N ? FEW_TOK : 0; }
 
 // ---------------------------------------------------------------- prefill grouped GEMM on MFMA (moe_prefill.hip)
@@ -158,7 +160,7 @@ struct PrefillArgs {
     int R, K, nmat;                      // rows, columns; nmat 2 = gate/up, 1 = down
     const int4 * cols; const int * ncols;   // launch_prefill_cols
     const int8_t * bq; const float * bd; // activations: Q8_K integers [rows][K] and scales [rows][K/256]
-    const _Float16 * bh;                 // the integers as fp16 (launch_kq_gemm only)
+    const _Float16 * bh;                 // the integers as fp16 (launch_kq_gemm's Q5_K and Q6_K)
     const uint4 * tab;                   // the decode table image (build_table_image), for that kernel
     float * out;                         // gate/up: h [P+n][R] (silu(g) * u); down: o [P+n][R]
     float * gdbg, * udbg;                // optional gate / up outputs
@@ -167,7 +169,8 @@ struct PrefillArgs {
     // the columns col0 .. col1 - 1 of launch_prefill_cols (col1 <= 0: to the last); the shared expert's come first,
     // ceil(n / 64) of them
     int col0, col1;
-    // launch_kq_gemm only: activation row = slot - arow0, output row = slot - orow0 (the shared expert's gate / up
+    // launch_kq_gemm with Q5_K: udbg != null: the output of a second matrix sh[1] of the shared expert, in the same launch
+    // launch_kq_gemm: activation row = slot - arow0, output row = slot - orow0 (the shared expert's gate / up
     // read the tokens' rows and write rows 0 .. n - 1 of their own outputs)
     int arow0, orow0;
 };
@@ -200,13 +203,15 @@ hipError_t launch_prefill_gemm(const PrefillArgs & a, int grid, hipStream_t st);
 hipError_t few_init();
 hipError_t launch_few_gemm(const PrefillArgs & a, int grid, hipStream_t st);
 
-// K-quant matrices on the matrix cores (kq_gemm.hip), bit-identical to launch_kq_matvec: columns col0 .. col1 - 1 of
-// launch_prefill_cols (routed: expert e at w[0] + e * estride; the shared expert's: sh[0]), ggml's blocks read in
-// place; activations bh / bd = Q8_K integers as fp16 [rows][K] and their scales (row = slot - arow0), outputs
-// out[(slot - orow0) * R + r]. fmt KF_Q2K / KF_Q3K / KF_Q6K with K = 2048 (downs), KF_Q5K with K = 7168 (the shared
-// gate / up); R % 128 == 0.
+// K-quant matrices on the matrix cores, bit-identical to launch_kq_matvec: columns col0 .. col1 - 1 of a KQ_TOK table
+// (routed: expert e at w[0] + e * estride; the shared expert's: sh[0]), ggml's blocks read in place; activation row = slot -
+// arow0, outputs out[(slot - orow0) * R + r]. KF_Q2K / KF_Q3K with K = 2048 (downs; kq8_gemm.hip: activations bq, bd; R % 256
+// == 0), KF_Q6K with K = 2048 and KF_Q5K with K = 7168 (kq_gemm.hip: bh, bd; R % 128 == 0).
 hipError_t kq_gemm_init();
 hipError_t launch_kq_gemm(const PrefillArgs & a, int fmt, int grid, hipStream_t st);
+bool kq8_gemm_takes(int fmt, int K, int R);
+hipError_t kq8_gemm_init();
+hipError_t launch_kq8_gemm(const PrefillArgs & a, int fmt, int grid, hipStream_t st);
 
 // y[t] = sum_k (o[inv[t*topk+k]] * w[t][k]) in k order + o[P+t] (+ resid[t] when given)
 // grid y extent of the row-looping kernels: min(rows, cap); the cap is 65535 unless a test lowers it

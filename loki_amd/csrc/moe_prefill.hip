@@ -80,13 +80,13 @@ __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, c
     const PfTable T = blockIdx.x ? t1 : t0;
     const int i = threadIdx.x, nact = *nact_p;
     auto cls = [&](int slots) -> int { return slots > 64 ? PF_BROAD : slots > 32 ? PF_WIDE : slots > T.few ? PF_NARROW : PF_FEW; };
-    auto cut = [&](int cnt, int & cols, int & size) {   // cols columns of size slots, the last one the rest
-        cols = (cnt + T.tok - 1) / T.tok;
-        size = cols > 0 ? min(T.tok, ((cnt + cols - 1) / cols + 15) / 16 * 16) : 0;
+    auto cut = [](int cnt, int tok, int & cols, int & size) {   // cols columns of size slots, the last one the rest
+        cols = (cnt + tok - 1) / tok;
+        size = cols > 0 ? min(tok, ((cnt + cols - 1) / cols + 15) / 16 * 16) : 0;
     };
     int e = 0, s0 = 0, cnt = 0, cols, size;
     if (i < nact) { e = act[i]; s0 = offsets[e]; cnt = offsets[e + 1] - s0; }
-    cut(cnt, cols, size);
+    cut(cnt, T.tok, cols, size);
     int nk[PF_NCLS] = { 0, 0, 0, 0 };                   // this expert's columns of each class
     if (cols > 0) { nk[cls(size)] += cols - 1; nk[cls(cnt - size * (cols - 1))] += 1; }
     for (int k = 0; k < PF_NCLS; ++k) { sc[k][i] = nk[k]; }
@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, c
         __syncthreads();
     }
     int nsh, ssize;
-    cut(n, nsh, ssize);
+    cut(n, T.stok, nsh, ssize);
     int at[PF_NCLS], end = nsh;
     for (int k = 0; k < PF_NCLS; ++k) {
         at[k] = end + sc[k][i] - nk[k];
