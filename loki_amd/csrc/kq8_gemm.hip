@@ -34,7 +34,9 @@ constexpr int K8_W = 16, K8_NT = K8_W * 64, K8_ROWS = K8_W * 16, K8_NB = 8;   //
 constexpr int K8_TT = 4;                       // 16-token tiles per column at most
 // LDS: (Q3_K) the scale lines, 64 x 32 copies of 8 bytes (lane l reads copy l % 32); two buffers of 64 block scales; two
 // activation buffers of 64 rows x 256 bytes
-constexpr int K8_DX = 64 * 256, K8_X = K8_DX + 1024, K8_BUF = K8_TT * 16 * QK, K8_LDS = K8_X + 2 * K8_BUF;
+constexpr int K8_DX = 64 * 256, K8_X = K8_DX + 1024, K8_BUF = K8_TT * 16 * QK, K8_W0 = K8_X + 2 * K8_BUF;
+constexpr int K8_LDS = K8_W0 + K8_W * 2 * 16 * 128;   // .. then every wave's two weight windows
+static_assert(K8_LDS <= 160 * 1024, "LDS budget");
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t k8_rsrc(const void * p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short) 0, (int) bytes, 0x00020000);
@@ -55,23 +57,23 @@ template <int SZ> __device__ __forceinline__ void k8_lds(__amdgpu_buffer_rsrc_t 
 #endif
 }
 
-// a lane's bytes of one block. Q2_K: q = its 16 quant bytes, s = the 8 scale bytes of its half, dd = d and dmin. Q3_K (blocks
-// start on 2-byte boundaries): aligned windows over the 16 quant bytes, the 16 high-bit bytes and the last 14 bytes
-// (scales and d), sh = 0 or 2 the offset inside them.
-template <int F> struct K8Raw;
-template <> struct K8Raw<KF_Q2K> { u32x4 q; u32v2 s; uint32_t dd; };
-template <> struct K8Raw<KF_Q3K> { u32x4 q, h, t; uint32_t q4, h4; };
-
-template <int F> __device__ __forceinline__ void k8_load(const Src & b, uint32_t blk, int g, K8Raw<F> & w) {
-    const uint32_t n = (uint32_t) g >> 1, h = (uint32_t) g & 1u;
-    if constexpr (F == KF_Q2K) {   // scales[16] qs[64] d dmin
-        Src s = b; s.vb += blk;
-        w.q = ld128(s, 16 + 32 * n + 16 * h); w.s = ld64(s, 8 * n); w.dd = ld32(s, 80);
-    } else {                       // hmask[32] qs[64] scales[12] d
-        Src s = b; s.vb += blk & ~3u;   // (sh is the same for every field: their offsets are multiples of 4)
-        w.q = ld128(s, 32 + 32 * n + 16 * h); w.q4 = ld32(s, 48 + 32 * n + 16 * h);
-        w.h = ld128(s, 16 * h); w.h4 = ld32(s, 16 + 16 * h);
-        w.t = ld128(s, 96);
+// A wave's 16 rows of one block come through LDS: rows are 110 (84) byte blocks side by side, so lanes that fetched their own
+// pieces would touch every cache line of the tile five times over, which bounded the first version (485 against 300 us at
+// 201 tokens). Two direct loads copy, per row, the 128-byte window of eight 16-byte units that holds the block (window start:
+// the block's offset rounded down to 16); unit u of row r sits at slot u ^ ((r / 2) % 8) of the row's 128 bytes, so the 16
+// rows of a read hit 16 bank quads. The block's offset in its window, DL, is the same for every row; a field of 16 bytes is
+// two units shifted by DL.
+constexpr int K8_WB = 16 * 128;
+template <int F, int J> constexpr int k8_delta() { return (J * kbytes<F>()) & 15; }
+__device__ __forceinline__ uint32_t k8_slot(int r, int u) { return (uint32_t) (r * 128 + ((u ^ ((r >> 1) & 7)) << 4)); }
+__device__ __forceinline__ u32x4 k8_read(uint32_t at) { return *(const LK_LOCAL u32x4 *) (size_t) at; }
+// N words at byte DL of two adjacent units
+template <int DL, int N> __device__ __forceinline__ void k8_shift(const u32x4 & a, const u32x4 & b, uint32_t (&o)[N]) {
+    const uint32_t w[9] = { a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, 0u };
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if constexpr ((DL & 3) == 0) { o[i] = w[DL / 4 + i]; }
+        else { o[i] = __builtin_amdgcn_alignbyte(w[DL / 4 + i + 1], w[DL / 4 + i], DL & 3); }
     }
 }
 
@@ -106,6 +108,11 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
         }
     }
     __syncthreads();
+    // the lane's units in its wave's windows: quants, high bits (Q2_K: scales), and the last field
+    const uint32_t wb = lds_addr(k8_dyn) + (uint32_t) (K8_W0 + wave * 2 * K8_WB);
+    constexpr int UQ = Q3 ? 2 : 1, UT = Q3 ? 6 : 5;
+    const uint32_t aq0 = wb + k8_slot(r, UQ + g), aq1 = wb + k8_slot(r, UQ + 1 + g), ah0 = wb + k8_slot(r, Q3 ? (g & 1) : 0);
+    const uint32_t ah1 = wb + k8_slot(r, Q3 ? (g & 1) + 1 : 1), at0 = wb + k8_slot(r, UT), at1 = wb + k8_slot(r, UT + 1);
     const uint32_t sela = (g & 1) ? 0x01010101u : 0u;   // Q2_K: the byte of a scale word the lane's sub-blocks start at
 
     for (int it = blockIdx.x; it < ncols * nrg; it += gridDim.x) {
@@ -115,10 +122,17 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
         const int sb = (int) cv.y, sc = (int) cv.z;
         const uint8_t * Wm = routed ? a.w[0] + (size_t) (int) cv.w * a.estride : a.sh[0];
         const __amdgpu_buffer_rsrc_t rb = k8_rsrc(a.bq, 0x7fffffff), rd = k8_rsrc(a.bd, 0x7fffffff);
-        Src src;
-        src.rs = k8_rsrc(k8_uniform(Wm), (uint32_t) a.R * ROWB);
-        src.vb = (uint32_t) r * ROWB;
-        src.so = (uint32_t) (rg * K8_ROWS + wave * 16) * ROWB;
+        const __amdgpu_buffer_rsrc_t rw = k8_rsrc(k8_uniform(Wm), (uint32_t) a.R * ROWB);
+        const uint32_t tile = (uint32_t) (rg * K8_ROWS + wave * 16) * ROWB;
+        // copy instruction i: lane L takes unit (L % 8) ^ .. of row 8 i + L / 8
+        uint32_t ow[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) { const int row = 8 * i + (lane >> 3); ow[i] = (uint32_t) row * ROWB + (uint32_t) (((lane & 7) ^ ((row >> 1) & 7)) << 4); }
+        auto load_w = [&](int j, int buf) {   // past the matrix's end a load returns 0
+            LK_LOCAL uint8_t * dst = lds + K8_W0 + (wave * 2 + buf) * K8_WB;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) { k8_lds<16>(rw, dst + i * 1024, ow[i], tile + (uint32_t) ((j * BS) & ~15)); }
+        };
         const int ar0 = sb - a.arow0;
         auto run_item = [&](auto ntc) {
             constexpr int NT = decltype(ntc)::value;
@@ -134,21 +148,20 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
             kf4 acc[NT];
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt) { acc[tt] = (kf4) { 0.f, 0.f, 0.f, 0.f }; }
-            auto block = [&](const K8Raw<F> & w, auto par) {
-                constexpr int buf = decltype(par)::value;   // the block's parity: buffer and (Q3_K) byte alignment
+            auto block = [&](auto jc) {
+                constexpr int J = decltype(jc)::value, buf = J & 1, DL = k8_delta<F, J>();
                 // the lane's four operands: plane s of its bytes (sub-block 8 n + 2 s + h)
                 ki4 wv[4];
                 uint32_t mn[4];
                 float dd, dm = 0.f;
-                if constexpr (Q3) {
-                    constexpr uint32_t sh = (uint32_t) (buf * BS) & 3u;
-                    const uint32_t q[4] = { __builtin_amdgcn_alignbyte(w.q.y, w.q.x, sh), __builtin_amdgcn_alignbyte(w.q.z, w.q.y, sh),
-                                            __builtin_amdgcn_alignbyte(w.q.w, w.q.z, sh), __builtin_amdgcn_alignbyte(w.q4, w.q.w, sh) };
-                    const uint32_t hb[4] = { __builtin_amdgcn_alignbyte(w.h.y, w.h.x, sh), __builtin_amdgcn_alignbyte(w.h.z, w.h.y, sh),
-                                             __builtin_amdgcn_alignbyte(w.h.w, w.h.z, sh), __builtin_amdgcn_alignbyte(w.h4, w.h.w, sh) };
-                    const uint32_t a0 = __builtin_amdgcn_alignbyte(w.t.y, w.t.x, sh), a1 = __builtin_amdgcn_alignbyte(w.t.z, w.t.y, sh);
-                    const uint32_t a2 = __builtin_amdgcn_alignbyte(w.t.w, w.t.z, sh);
-                    dd = h2f((uint16_t) (sh ? w.t.w >> 16 : w.t.w));
+                constexpr uint32_t wo = (uint32_t) (buf * K8_WB);
+                if constexpr (Q3) {   // hmask[32] qs[64] scales[12] d
+                    uint32_t q[4], hb[4], ts[4];
+                    k8_shift<DL, 4>(k8_read(aq0 + wo), k8_read(aq1 + wo), q);
+                    k8_shift<DL, 4>(k8_read(ah0 + wo), k8_read(ah1 + wo), hb);
+                    k8_shift<DL, 4>(k8_read(at0 + wo), k8_read(at1 + wo), ts);
+                    const uint32_t a0 = ts[0], a1 = ts[1], a2 = ts[2];
+                    dd = h2f((uint16_t) ts[3]);
                     const uint32_t n4 = (uint32_t) (g >> 1) * 4, s4 = 8u * (uint32_t) (g & 1) + n4;
                     // 6-bit scales j = 8 n + 2 s + h (kquant_device.h): s = 0, 1 at bits 0 and 16 of p01, s = 2, 3 of p23
                     const uint32_t p01 = ((a0 >> s4) & 0x000F000Fu) | (rotr(a2, s4 - 4u) & 0x00300030u);
@@ -162,16 +175,22 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
                             wv[s][i] = (int) __builtin_amdgcn_perm(t[s].y, t[s].x, u);
                         }
                     }
-                } else {
-                    dd = h2f((uint16_t) (w.dd & 0xFFFFu)); dm = h2f((uint16_t) (w.dd >> 16));
+                } else {              // scales[16] qs[64] d dmin
+                    uint32_t q[4], sc8[4], td[1];
+                    k8_shift<DL, 4>(k8_read(aq0 + wo), k8_read(aq1 + wo), q);
+                    k8_shift<DL, 4>(k8_read(ah0 + wo), k8_read(ah1 + wo), sc8);
+                    const u32x4 tu = k8_read(at0 + wo);
+                    k8_shift<DL, 1>(tu, tu, td);
+                    dd = h2f((uint16_t) (td[0] & 0xFFFFu)); dm = h2f((uint16_t) (td[0] >> 16));
+                    const uint32_t sw2[2] = { g >> 1 ? sc8[2] : sc8[0], g >> 1 ? sc8[3] : sc8[1] };
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
-                        const uint32_t sw = s < 2 ? w.s.x : w.s.y, sel = sela + (s & 1 ? 0x02020202u : 0u);
+                        const uint32_t sw = sw2[s >> 1], sel = sela + (s & 1 ? 0x02020202u : 0u);
                         const uint32_t b = __builtin_amdgcn_perm(sw, sw, sel);              // the sub-block's byte, four times
                         const uint32_t t = (uint32_t) __umul24(b & 15u, 0x030201u) << 8;    // bytes sc * {0, 1, 2, 3}
                         mn[s] = (b >> 4) & 0x0F0F0F0Fu;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) { wv[s][i] = (int) __builtin_amdgcn_perm(t, t, (w.q[i] >> (2 * s)) & 0x03030303u); }
+                        for (int i = 0; i < 4; ++i) { wv[s][i] = (int) __builtin_amdgcn_perm(t, t, (q[i] >> (2 * s)) & 0x03030303u); }
                     }
                 }
                 // chunk 8 n + 2 s + h of the lane's token row at slot chunk ^ r: one address word per product, the tile and the
@@ -208,28 +227,29 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
                         if constexpr (Q3) { acc[tt][i] = acc[tt][i] - (dd * dx[i]) * (float) D[i]; }
                         else { acc[tt][i] = acc[tt][i] + ((dx[i] * dd) * (float) D[i] - (dx[i] * dm) * (float) M[i]); }
                     }
+                    // the fold belongs to this block (unrolled, the compiler would carry the sums of all eight to the end)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) { float v = acc[tt][i]; __asm__ volatile("" : "+v"(v)); acc[tt][i] = v; }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
-            K8Raw<F> w0, w1;
             load_b(0, 0);
-            k8_load<F>(src, 0, g, w0);
-            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block 0's activations are in LDS
+            load_w(0, 0);
+            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block 0 is in LDS
             __syncthreads();
-            auto step = [&](int j, auto par, const K8Raw<F> & cur, K8Raw<F> & ahead) {
-                const int jn = j + 1 < NB ? j + 1 : NB - 1;   // the last step reloads its own block (unread)
-                load_b(jn, (j + 1) & 1);                       // that buffer was last read in step j - 1, before its barrier
-                k8_load<F>(src, (uint32_t) (jn * BS), g, ahead);
+            auto step = [&](auto jc) {
+                constexpr int J = decltype(jc)::value;
+                // the other buffers were last read in step J - 1, before its barrier
+                if constexpr (J + 1 < NB) { load_b(J + 1, (J + 1) & 1); load_w(J + 1, (J + 1) & 1); }
                 __builtin_amdgcn_sched_barrier(0);
-                block(cur, par);
-                __builtin_amdgcn_s_waitcnt(0x0f70);            // vmcnt(0): block j + 1's activations have landed in LDS
+                block(jc);
+                __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block J + 1 has landed in LDS
                 __builtin_amdgcn_s_barrier();
             };
-#pragma unroll 1
-            for (int j = 0; j < NB; j += 2) {
-                step(j, std::integral_constant<int, 0>{}, w0, w1);
-                step(j + 1, std::integral_constant<int, 1>{}, w1, w0);
-            }
+            step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{});
+            step(std::integral_constant<int, 2>{}); step(std::integral_constant<int, 3>{});
+            step(std::integral_constant<int, 4>{}); step(std::integral_constant<int, 5>{});
+            step(std::integral_constant<int, 6>{}); step(std::integral_constant<int, 7>{});
             const int orow = rg * K8_ROWS + wave * 16 + r;
             int t0 = 4 * g;
             __asm__ volatile("" : "+v"(t0));   // the output rows are formed here, not kept (and spilled) across the items
