@@ -35,7 +35,7 @@ constexpr int K8_TT = 4;                       // 16-token tiles per column at m
 // LDS: (Q3_K) the scale lines, 64 x 32 copies of 8 bytes (lane l reads copy l % 32); two buffers of 64 block scales; two
 // activation buffers of 64 rows x 256 bytes
 constexpr int K8_DX = 64 * 256, K8_X = K8_DX + 1024, K8_BUF = K8_TT * 16 * QK, K8_W0 = K8_X + 2 * K8_BUF;
-constexpr int K8_LDS = K8_W0 + K8_W * 2 * 16 * 128;   // .. then every wave's two weight windows
+constexpr int K8_RING = 3, K8_LDS = K8_W0 + K8_W * K8_RING * 16 * 128;   // .. then every wave's weight windows
 static_assert(K8_LDS <= 160 * 1024, "LDS budget");
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t k8_rsrc(const void * p, uint32_t bytes) {
@@ -109,42 +109,57 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
     }
     __syncthreads();
     // the lane's units in its wave's windows: quants, high bits (Q2_K: scales), and the last field
-    const uint32_t wb = lds_addr(k8_dyn) + (uint32_t) (K8_W0 + wave * 2 * K8_WB);
+    const uint32_t wb = lds_addr(k8_dyn) + (uint32_t) (K8_W0 + wave * K8_RING * K8_WB);
     constexpr int UQ = Q3 ? 2 : 1, UT = Q3 ? 6 : 5;
     const uint32_t aq0 = wb + k8_slot(r, UQ + g), aq1 = wb + k8_slot(r, UQ + 1 + g), ah0 = wb + k8_slot(r, Q3 ? (g & 1) : 0);
     const uint32_t ah1 = wb + k8_slot(r, Q3 ? (g & 1) + 1 : 1), at0 = wb + k8_slot(r, UT), at1 = wb + k8_slot(r, UT + 1);
     const uint32_t sela = (g & 1) ? 0x01010101u : 0u;   // Q2_K: the byte of a scale word the lane's sub-blocks start at
 
-    for (int it = blockIdx.x; it < ncols * nrg; it += gridDim.x) {
-        const int col = col0 + it / nrg, rg = it % nrg;
-        const u32x4 cv = *(const LK_GLOBAL u32x4 *) (a.cols + col);
-        const bool routed = (int) cv.x >= 0;
-        const int sb = (int) cv.y, sc = (int) cv.z;
-        const uint8_t * Wm = routed ? a.w[0] + (size_t) (int) cv.w * a.estride : a.sh[0];
-        const __amdgpu_buffer_rsrc_t rb = k8_rsrc(a.bq, 0x7fffffff), rd = k8_rsrc(a.bd, 0x7fffffff);
-        const __amdgpu_buffer_rsrc_t rw = k8_rsrc(k8_uniform(Wm), (uint32_t) a.R * ROWB);
-        const uint32_t tile = (uint32_t) (rg * K8_ROWS + wave * 16) * ROWB;
-        // copy instruction i: lane L takes unit (L % 8) ^ .. of row 8 i + L / 8
-        uint32_t ow[2];
+    // An item's place (uniform); the loads are aimed at one item at a time, and the last step of an item already loads block 0
+    // of the next one. Activations: wave w copies token rows 4 w .. 4 w + 3, lane L of row (L / 16) the row's chunk (L % 16) ^
+    // (row % 16); the block scales by the last wave. Weights: copy instruction i takes unit (L % 8) ^ .. of row 8 i + L / 8.
+    struct Item { int e, sb, sc, rg; };   // e: the routed expert, or -1 for the shared one
+    auto item_of = [&](int it) -> Item {
+        const u32x4 cv = *(const LK_CONST u32x4 *) (a.cols + (col0 + it / nrg));
+        return Item { (int) cv.x < 0 ? -1 : (int) cv.w, (int) cv.y, (int) cv.z, it % nrg };
+    };
+    const __amdgpu_buffer_rsrc_t rb = k8_rsrc(a.bq, 0x7fffffff), rd = k8_rsrc(a.bd, 0x7fffffff);
+    __amdgpu_buffer_rsrc_t rw;
+    uint32_t tile = 0, ob = 0, od = 0, ow[2];
+    int ncopy = 0;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) { const int row = 8 * i + (lane >> 3); ow[i] = (uint32_t) row * ROWB + (uint32_t) (((lane & 7) ^ ((row >> 1) & 7)) << 4); }
-        auto load_w = [&](int j, int buf) {   // past the matrix's end a load returns 0
-            LK_LOCAL uint8_t * dst = lds + K8_W0 + (wave * 2 + buf) * K8_WB;
+    for (int i = 0; i < 2; ++i) { const int row = 8 * i + (lane >> 3); ow[i] = (uint32_t) row * ROWB + (uint32_t) (((lane & 7) ^ ((row >> 1) & 7)) << 4); }
+    auto aim = [&](const Item & t) {
+        const uint8_t * Wm = t.e >= 0 ? a.w[0] + (size_t) t.e * a.estride : a.sh[0];
+        rw = k8_rsrc(k8_uniform(Wm), (uint32_t) a.R * ROWB);   // past the matrix's end a load returns 0
+        tile = (uint32_t) (t.rg * K8_ROWS + wave * 16) * ROWB;
+        const int ar0 = t.sb - a.arow0, row = 4 * wave + (lane >> 4);
+        ob = (uint32_t) (ar0 + (row < t.sc ? row : 0)) * (NB * QK) + (uint32_t) (((lane & 15) ^ (row & 15)) << 4);
+        od = (uint32_t) (ar0 + (lane < t.sc ? lane : 0)) * (NB * 4);
+        ncopy = 4 * ((t.sc + 15) >> 4);
+    };
+    auto load_w = [&](int j, int buf) {
+        LK_LOCAL uint8_t * dst = lds + K8_W0 + (wave * K8_RING + buf) * K8_WB;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) { k8_lds<16>(rw, dst + i * 1024, ow[i], tile + (uint32_t) ((j * BS) & ~15)); }
-        };
-        const int ar0 = sb - a.arow0;
+        for (int i = 0; i < 2; ++i) { k8_lds<16>(rw, dst + i * 1024, ow[i], tile + (uint32_t) ((j * BS) & ~15)); }
+    };
+    auto load_b = [&](int j, int buf) {
+        if (wave < ncopy) { k8_lds<16>(rb, lds + K8_X + buf * K8_BUF + wave * 1024, ob, j * QK); }
+        if (wave == K8_W - 1) { k8_lds<4>(rd, lds + K8_DX + buf * 256, od, j * 4); }
+    };
+    const int items = ncols * nrg;
+    if ((int) blockIdx.x >= items) { return; }
+    Item cur = item_of(blockIdx.x);
+    aim(cur);
+    load_b(0, 0);
+    load_w(0, 0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block 0 is in LDS
+    __syncthreads();
+    for (int it = blockIdx.x; it < items; it += gridDim.x) {
+        const Item nxt = item_of(it + (int) gridDim.x < items ? it + (int) gridDim.x : it);   // (none: its loads are not read)
+        const int sb = cur.sb, sc = cur.sc, rg = cur.rg;
         auto run_item = [&](auto ntc) {
             constexpr int NT = decltype(ntc)::value;
-            // activations: wave w copies token rows 4 w .. 4 w + 3 (w < 4 NT), lane L of row (L / 16) the row's chunk
-            // (L % 16) ^ (row % 16); the block scales by the last wave
-            const int row = 4 * wave + (lane >> 4);
-            const uint32_t ob = (uint32_t) (ar0 + (row < sc ? row : 0)) * (NB * QK) + (uint32_t) (((lane & 15) ^ (row & 15)) << 4);
-            const uint32_t od = (uint32_t) (ar0 + (lane < sc ? lane : 0)) * (NB * 4);
-            auto load_b = [&](int j, int buf) {
-                if (wave < 4 * NT) { k8_lds<16>(rb, lds + K8_X + buf * K8_BUF + wave * 1024, ob, j * QK); }
-                if (wave == K8_W - 1) { k8_lds<4>(rd, lds + K8_DX + buf * 256, od, j * 4); }
-            };
             kf4 acc[NT];
 #pragma unroll
             for (int tt = 0; tt < NT; ++tt) { acc[tt] = (kf4) { 0.f, 0.f, 0.f, 0.f }; }
@@ -154,7 +169,7 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
                 ki4 wv[4];
                 uint32_t mn[4];
                 float dd, dm = 0.f;
-                constexpr uint32_t wo = (uint32_t) (buf * K8_WB);
+                constexpr uint32_t wo = (uint32_t) (J % K8_RING * K8_WB);
                 if constexpr (Q3) {   // hmask[32] qs[64] scales[12] d
                     uint32_t q[4], hb[4], ts[4];
                     k8_shift<DL, 4>(k8_read(aq0 + wo), k8_read(aq1 + wo), q);
@@ -233,17 +248,19 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
                     __builtin_amdgcn_sched_barrier(0);
                 }
             };
-            load_b(0, 0);
-            load_w(0, 0);
-            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block 0 is in LDS
-            __syncthreads();
+            // Activations one block ahead, weights two (a ring of three windows; block 0 of an item comes with the last step
+            // of the item before, block 1 in step 0): the wait of a step leaves the two newest weight copies outstanding.
             auto step = [&](auto jc) {
                 constexpr int J = decltype(jc)::value;
-                // the other buffers were last read in step J - 1, before its barrier
-                if constexpr (J + 1 < NB) { load_b(J + 1, (J + 1) & 1); load_w(J + 1, (J + 1) & 1); }
+                // the windows and buffers written here were last read in step J - 1, before its barrier
+                if constexpr (J + 1 < NB) { load_b(J + 1, (J + 1) & 1); }
+                else { aim(nxt); load_b(0, 0); load_w(0, 0); }
+                if constexpr (J == 0) { load_w(1, 1); }
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (J + 2 < NB) { load_w(J + 2, (J + 2) % K8_RING); }
                 __builtin_amdgcn_sched_barrier(0);
                 block(jc);
-                __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block J + 1 has landed in LDS
+                __builtin_amdgcn_s_waitcnt(0x0f70 | (J + 2 < NB ? 2 : 0));   // block J + 1 has landed in LDS
                 __builtin_amdgcn_s_barrier();
             };
             step(std::integral_constant<int, 0>{}); step(std::integral_constant<int, 1>{});
@@ -266,6 +283,7 @@ __global__ void __launch_bounds__(K8_NT, 1) k_kq8_gemm(const PrefillArgs a) {
         else if (sc > 32) { run_item(std::integral_constant<int, 3>{}); }
         else if (sc > 16) { run_item(std::integral_constant<int, 2>{}); }
         else { run_item(std::integral_constant<int, 1>{}); }
+        cur = nxt;
     }
 }
 

@@ -215,64 +215,91 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
     const size_t dreg = (size_t) (a.R / 64) * NB * 4096;   // d region offset of a tiled matrix
     __syncthreads();
 
-    for (int it = blockIdx.x; it < runs.count() * nrg; it += gridDim.x) {
-        const int col = runs.col(it / nrg), rg = it % nrg;
-        const u32x4 cv = *(const LK_GLOBAL u32x4 *) (a.cols + col);
-        const int4 cd = make_int4((int) cv.x, (int) cv.y, (int) cv.z, (int) cv.w);
-        const bool routed = cd.x >= 0;
-        const int sb = cd.y, sc = cd.z;
-        auto brow = [&](int t) -> int {   // activation row of token t of the column
-            const int s = sb + (t < sc ? t : 0);
-            return NMAT == 2 ? (routed ? gptr(a.perm)[s] / a.topk : s - a.P) : s;
-        };
-        // Buffer loads: a scalar resource (base, no bounds that matter) + a 32-bit lane offset + a scalar block offset,
-        // so no 64-bit per-lane address lives in vector registers.
-        const __amdgpu_buffer_rsrc_t rb = pf_rsrc(a.bq), rd = pf_rsrc(a.bd);
-        // the wave's tiles: combo c = (matrix Geo::mat, 16-row tile Geo::tile): scalar resources at the tile's qs / d
-        // bases, the lane's offset (chunk g of row r) in one vector register
-        __amdgpu_buffer_rsrc_t uq[C], ud[C];
+    // An item's place: its column (uniform) and row group. The loads are aimed at one item at a time: buffer loads with a
+    // scalar resource (base, no bounds that matter), a 32-bit lane offset and a scalar block offset, so no 64-bit per-lane
+    // address lives in vector registers. AHEAD (the down's short rows: eight steps an item): the last step of an item already
+    // loads block 0 of the next one (its wait was a tenth of the pass); the gate/up's 28 steps have no registers left for it.
+    constexpr bool AHEAD = NMAT == 1;
+    struct Item { int e, sb, sc, rg; };   // e: the routed expert, or -1 for the shared one
+    auto item_of = [&](int it) -> Item {
+        const u32x4 cv = *(const LK_CONST u32x4 *) (a.cols + runs.col(it / nrg));
+        return Item { (int) cv.x < 0 ? -1 : (int) cv.w, (int) cv.y, (int) cv.z, it % nrg };
+    };
+    // The column's activations of block j go straight from memory into LDS buffer j % 2 (buffer loads to LDS: lane L's 16
+    // bytes land at L * 16 of the instruction's 1 KB, no registers): copy instruction i covers token rows 4 i .. 4 i + 3,
+    // i < 4 token tiles, taken by waves i % W; lane L of row (L / 16) takes the row's chunk (L % 16) ^ (row % 16) -- the
+    // swizzle applied on the memory side. gfx950 serves a ds_read_b128 in four passes of 16 lanes (equal bit 5, equal bit
+    // 4 ^ bit 3); lane (r, g) reads slot (4 g + m) ^ r of row r, so a pass holds 16 different slots. The tokens' block
+    // scales follow, 64 tokens per instruction (waves W - 1, W - 2).
+    constexpr int NI = (4 * NTM + W - 1) / W, ND = (NTM + 3) / 4;
+    const __amdgpu_buffer_rsrc_t rb = pf_rsrc(a.bq), rd = pf_rsrc(a.bd);
+    const uint32_t lq = (uint32_t) g * 1024 + (uint32_t) r * 16, ldo = (uint32_t) r * 2;
+    const int dw0 = W - 1 - wave;                 // which 64 tokens' scales this wave copies (0 .. ND - 1)
+    __amdgpu_buffer_rsrc_t uq[C], ud[C];          // the wave's tiles: qs / d bases of combo c (Geo::mat, Geo::tile)
+    uint32_t ob[NI], od = 0;
+    int ncopy = 0;                                // copy instructions of the column
+    int rows[NI + 1];                             // the activation rows behind ob and od, read ahead of their use
+    auto rows_of = [&](const Item & t) {
+        const int n16 = (t.sc + 15) & ~15;
+        auto slot = [&](int i) { return t.sb + (i < t.sc ? i : 0); };
+        auto row = [&](int i) { const int s = slot(i); return NMAT == 2 ? (t.e >= 0 ? gptr(a.perm)[s] : s - a.P) : s; };
+#pragma unroll
+        for (int i = 0; i < NI; ++i) { const int q = 4 * (wave + W * i) + (lane >> 4); rows[i] = row(q < n16 ? q : 0); }
+        rows[NI] = dw0 < ND ? row(64 * dw0 + lane) : 0;
+    };
+    auto aim = [&](const Item & t) {              // after rows_of(t)
+        auto arow = [&](int v) { return (uint32_t) (NMAT == 2 && t.e >= 0 ? v / a.topk : v); };
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int q = 4 * (wave + W * i) + (lane >> 4);
+            ob[i] = arow(rows[i]) * Geo::K + (uint32_t) (((lane & 15) ^ (q & 15)) << 4);
+        }
+        od = arow(rows[NI]) * (NB * 4);
+        ncopy = 4 * ((t.sc + 15) >> 4);
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const int mat = Geo::mat(wave, c), ti = Geo::tile(wave, c);
-            const uint8_t * Wm = routed ? a.w[mat] + (size_t) cd.w * a.estride : a.sh[mat];
-            const int row0 = rg * Geo::ROWS + ti * 16;   // a 16-row tile lies inside one 64-row group
+            const uint8_t * Wm = t.e >= 0 ? a.w[mat] + (size_t) t.e * a.estride : a.sh[mat];
+            const int row0 = t.rg * Geo::ROWS + ti * 16;   // a 16-row tile lies inside one 64-row group
             const int g64 = row0 >> 6, r0 = row0 & 63;
             uq[c] = pf_rsrc(pf_uniform(Wm + (size_t) g64 * NB * 4096 + r0 * 16));
             ud[c] = pf_rsrc(pf_uniform(Wm + dreg + (size_t) g64 * NB * 128 + r0 * 2));
         }
-        const uint32_t lq = (uint32_t) g * 1024 + (uint32_t) r * 16, ldo = (uint32_t) r * 2;
-        auto load_w = [&](int j, PfW (&w)[C]) {
+    };
+    auto load_w = [&](int j, PfW (&w)[C]) {
 #pragma unroll
-            for (int c = 0; c < C; ++c) {
-                w[c].q = __builtin_amdgcn_raw_buffer_load_b128(uq[c], lq, j * 4096, 2);   // nt: streamed once
-                w[c].d = __builtin_amdgcn_raw_buffer_load_b16(ud[c], ldo, j * 128, 0);
-            }
-        };
+        for (int c = 0; c < C; ++c) {
+            w[c].q = __builtin_amdgcn_raw_buffer_load_b128(uq[c], lq, j * 4096, 2);   // nt: streamed once
+            w[c].d = __builtin_amdgcn_raw_buffer_load_b16(ud[c], ldo, j * 128, 0);
+        }
+    };
+    auto load_b = [&](int j, int buf) {
+        LK_LOCAL uint8_t * dst = lds + Geo::L_X + buf * Geo::BUF;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if (wave + W * i < ncopy) { buf_lds<16>(rb, dst + (wave + W * i) * 1024, ob[i], j * QK); }
+        }
+        if (dw0 < ND) { buf_lds<4>(rd, lds + L_DX + buf * Geo::DXB + dw0 * 256, od, j * 4); }
+    };
+
+    const int items = runs.count() * nrg;
+    PfW w0[C], w1[C];
+    Item cur = item_of(blockIdx.x);
+    auto begin = [&]() {
+        rows_of(cur);
+        aim(cur);
+        load_w(0, w0);
+        load_b(0, 0);
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block 0's activations are in LDS
+        __syncthreads();
+    };
+    if (AHEAD) { begin(); }
+    for (int it = blockIdx.x; it < items; it += gridDim.x) {
+        const Item nxt = item_of(it + (int) gridDim.x < items ? it + (int) gridDim.x : it);   // (none: its loads are not used)
+        if (!AHEAD) { begin(); }
+        const int sb = cur.sb, sc = cur.sc, rg = cur.rg;
         auto run_item = [&](auto ntc) {
             constexpr int NT = decltype(ntc)::value;   // token tiles of the column
-            // the column's activations of block j go straight from memory into LDS buffer j % 2 (buffer loads to LDS:
-            // lane L's 16 bytes land at L * 16 of the instruction's 1 KB, no registers): copy instruction i covers token
-            // rows 4 i .. 4 i + 3, i < 4 NT, taken by waves i % W; lane L of row (L / 16) takes the row's chunk
-            // (L % 16) ^ (row % 16) -- the swizzle applied on the memory side. gfx950 serves a ds_read_b128 in four passes
-            // of 16 lanes (equal bit 5, equal bit 4 ^ bit 3); lane (r, g) reads slot (4 g + m) ^ r of row r, so a pass holds
-            // 16 different slots. The tokens' block scales follow, 64 tokens per instruction (waves W - 1, W - 2).
-            constexpr int NI = (4 * NT + W - 1) / W, ND = (NT + 3) / 4;
-            uint32_t ob[NI], od = 0;
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const int row = 4 * (wave + W * i) + (lane >> 4);
-                ob[i] = (uint32_t) brow(row < 16 * NT ? row : 0) * Geo::K + (uint32_t) (((lane & 15) ^ (row & 15)) << 4);
-            }
-            const int dw0 = W - 1 - wave;   // which 64 tokens' scales this wave copies (0 .. ND - 1)
-            if (dw0 < ND) { od = (uint32_t) brow(64 * dw0 + lane) * (NB * 4); }
-            auto load_b = [&](int j, int buf) {
-                LK_LOCAL uint8_t * dst = lds + Geo::L_X + buf * Geo::BUF;
-#pragma unroll
-                for (int i = 0; i < NI; ++i) {
-                    if (wave + W * i < 4 * NT) { buf_lds<16>(rb, dst + (wave + W * i) * 1024, ob[i], j * QK); }
-                }
-                if (dw0 < ND) { buf_lds<4>(rd, lds + L_DX + buf * Geo::DXB + dw0 * 256, od, j * 4); }
-            };
             f4 acc[C][NT];
 #pragma unroll
             for (int c = 0; c < C; ++c) { for (int tt = 0; tt < NT; ++tt) { acc[c][tt] = (f4) { 0.f, 0.f, 0.f, 0.f }; } }
@@ -364,31 +391,31 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
                 for (int i = 0; i < 4; ++i) { fold(NT - 1, i, dp[i]); }
             };
 
-            // pipeline: weights and activations one block ahead (registers; the other of two LDS buffers). Every step
-            // issues the same loads (the last one reloads its own block, which nobody reads any more).
-            PfW w0[C], w1[C];
-            load_w(0, w0);
-            load_b(0, 0);
-            __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): block 0's activations are in LDS
-            __syncthreads();
-            auto step = [&](int j, const PfW (&cur)[C], PfW (&ahead)[C]) {
-                const int jn = j + 1 < NB ? j + 1 : NB - 1;
+            // pipeline: weights and activations one block ahead (registers; the other of two LDS buffers)
+            auto step = [&](int j, int jn, const PfW (&now)[C], PfW (&ahead)[C]) {
                 load_b(jn, (j + 1) & 1);             // buffer (j + 1) % 2 was last read in step j - 1, before its barrier
                 load_w(jn, ahead);
                 __builtin_amdgcn_sched_barrier(0);   // nothing of the block moves above the loads
-                dequant(cur);
+                dequant(now);
                 products(j & 1);
-                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): block j + 1's activations have landed in LDS (and the
-                __builtin_amdgcn_s_barrier();        // weights of the next block are in): the barrier publishes them
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the next block's activations have landed in LDS (and its
+                __builtin_amdgcn_s_barrier();        // weights are in): the barrier publishes them
             };
             static_assert(NB % 2 == 0, "two steps per trip");
 #pragma unroll 1
-            for (int j = 0; j < NB; j += 2) { step(j, w0, w1); step(j + 1, w1, w0); }
+            for (int j = 0; j < NB; j += 2) {
+                const bool end = j == NB - 2;
+                if (AHEAD && end) { rows_of(nxt); }
+                step(j, j + 1, w0, w1);
+                if (AHEAD && end) { aim(nxt); }
+                step(j + 1, end ? (AHEAD ? 0 : NB - 1) : j + 2, w1, w0);   // (not ahead: a reload, which nobody reads)
+            }
 
             // outputs: lane (r, g) holds tokens 4 g + i of each token tile for row r of each of its tiles
             if constexpr (Geo::XG) {
-                // the gate waves leave 0.125 g in the second activation buffer (last read before the last step's barrier,
-                // next filled after the next item's first one), the up waves form h for the same tile
+                // the gate waves leave 0.125 g in LDS (maybe in the second activation buffer, last read before the last step's
+                // barrier and next filled in the next item's first step, after the second barrier here), the up waves form h
+                // for the same tile
                 LK_LOCAL f4 * xg = reinterpret_cast<LK_LOCAL f4 *>(lds + Geo::L_G);
                 const int ti = Geo::tile(wave, 0);
                 if (Geo::mat(wave, 0) == 0) {
@@ -396,19 +423,22 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
                     for (int tt = 0; tt < NT; ++tt) { xg[(ti * NTM + tt) * 64 + lane] = 0.125f * acc[0][tt]; }
                 }
                 __syncthreads();
+                f4 gt[NT];
+#pragma unroll
+                for (int tt = 0; tt < NT; ++tt) { gt[tt] = xg[(ti * NTM + tt) * 64 + lane]; }
+                __syncthreads();
                 if (Geo::mat(wave, 0) == 1) {
                     const int row = rg * Geo::ROWS + ti * 16 + r;
 #pragma unroll
                     for (int tt = 0; tt < NT; ++tt) {
-                        const f4 gt = xg[(ti * NTM + tt) * 64 + lane];
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const int t = 16 * tt + 4 * g + i;
                             if (t < sc) {
                                 const size_t o = (size_t) (sb + t) * a.R + row;
                                 const float uv = 0.125f * acc[0][tt][i];
-                                a.out[o] = det_silu(gt[i]) * uv;
-                                if (a.gdbg) { a.gdbg[o] = gt[i]; a.udbg[o] = uv; }
+                                a.out[o] = det_silu(gt[tt][i]) * uv;
+                                if (a.gdbg) { a.gdbg[o] = gt[tt][i]; a.udbg[o] = uv; }
                             }
                         }
                     }
@@ -449,6 +479,7 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
             else if (sc > 80) { run_item(std::integral_constant<int, 6>{}); }
             else { run_item(std::integral_constant<int, 5>{}); }
         }
+        cur = nxt;
     }
 }
 
