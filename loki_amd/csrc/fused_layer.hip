@@ -552,13 +552,16 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     const size_t rows = (size_t) P + n;
     // K-quant matrices: at decode sizes the per-pass path (the n <= 8 decode block reads IQ2_XXS tiles), except for
     // one token on the real shards' formats (routed down Q2_K / Q3_K, shared expert Q5_K / Q5_K / Q6_K), which the
-    // one-token kernel reads in place; at prefill sizes the routed gate/up (always IQ2_XXS) on the MFMA GEMM and the
-    // K-quant matrices on the K-quant mat-vecs
+    // one-token kernel reads in place; at prefill sizes every matrix on a grouped GEMM that takes its format
     static_assert(FL_Q6K == 1 && FL_Q5K == 3 && FL_Q2K == 5 && FL_Q3K == 6, "the FL_ codes are the K-quant kernels' format codes");
     const int kd1 = (lf[0] == FL_Q2K || lf[0] == FL_Q3K) && lf[1] == FL_Q5K && lf[2] == FL_Q5K && lf[3] == FL_Q6K ? lf[0] : 0;
     const bool kq1 = kq && kd1 != 0 && n == 1 && tsel == MAXK && tk == MAXK && decode1_ready(c);
     const bool fused = (!kq || kq1) && c->fused && n <= 8 && E == 7168 && H == 2048 && decode_rule_ok(ne, c->n_group) && decode_ready(c);
     const bool mfma = !fused && c->pf_mfma && n > 8 && E == 7168 && H == 2048;
+    // a decode batch of a K-quant layer: its IQ2_XXS matrices on the matrix-core kernel of columns of at most 8 slots. Two
+    // more launches (the columns, Q8_K of h), so from 16 slots: 2 rows of 8 picks 98.8 -> 95.8 us, 6 rows 195 -> 164, 8 rows
+    // 238 -> 202, 8 rows of 2 picks 109 -> 99; at 6 slots (3 rows of 2) 75.4 -> 77.6
+    const bool few = !fused && !mfma && kq && c->pf_mfma && P >= 16 && E == 7168 && H == 2048;
     const bool q5 = lf[1] == FL_Q5K && lf[2] == FL_Q5K, q6 = lf[3] == FL_Q6K;   // shared matrices on fp16 activations
     ALLOC(c, c->xq, (size_t) n * E); ALLOC(c, c->xd, (size_t) n * (E / 256));
     ALLOC(c, c->logits, (size_t) n * ne); ALLOC(c, c->probs, (size_t) n * ne);
@@ -598,6 +601,16 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         if (q5) { ALLOC(c, c->xh, (size_t) n * E); }
         if (q6) { ALLOC(c, c->hh, (size_t) n * H); }
     }
+    if (!mfma && lf[1] != FL_IQ2) { ALLOC(c, c->ksg, (size_t) n * H); ALLOC(c, c->ksu, (size_t) n * H); }
+    if (few) {
+        if (int rc = prefill_ready(c)) { return rc; }
+        ALLOC(c, c->pcols, rows / pf_tok(n) + NEXP_MAX + 4); ALLOC(c, c->pncols, 2 * PF_NCOLS);
+    }
+    double * rp = nullptr;   // the matrix-core router's parts
+    if (const size_t nd = router_part_doubles(n, ne, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
+    if (share) { ALLOC(c, c->sel8, (size_t) n * tsel); ALLOC(c, c->w8, (size_t) n * tsel); }
+    int * dsc = nullptr;
+    if (const size_t nd = dispatch_scratch_ints(P)) { ALLOC(c, c->dscr, nd); dsc = c->dscr.p; }
     prof_mark(c, ev, 0);
     if (prenorm) {   // the per-pass path normalises into a context buffer first (k_rmsnorm: the same arithmetic)
         ALLOC(c, c->xn, (size_t) n * E);
@@ -607,20 +620,28 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     TRY(c, launch_quant_q8k(x, n, E, c->xq.p, c->xd.p, st));
     if (mfma && q5) { TRY(c, launch_q8_to_h(c->xq.p, c->xh.p, (int64_t) n * E, st)); }
     prof_mark(c, ev, 1);
-    double * rp = nullptr;   // the matrix-core kernel's parts
-    if (const size_t nd = router_part_doubles(n, ne, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
+    // Off the GEMMs, a K-quant shared expert (latency-bound mat-vecs of 10-12 MB per matrix) runs on the side stream from
+    // here on: beside the router, the selection and the dispatch, which leave the chip idle, and then the routed launches (6
+    // rows of the real formats 209 -> 195 us against a start beside the routed gate / up). It reads x's Q8_K and writes
+    // only its own rows (h / Q8_K(h) rows P .. P + n - 1, o rows P .., ksg / ksu), which no routed kernel touches; the
+    // combine waits for it. Everything that can fail to allocate is allocated before the fork.
+    const bool ksh = lf[1] != FL_IQ2;
+    const bool side = !mfma && ksh && kq && lf[3] != FL_IQ2 && !c->no_side;
+    if (side) {
+        TRY(c, hipEventRecord(c->efork, st)); TRY(c, hipStreamWaitEvent(c->side, c->efork, 0));
+        if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
+        if (int rc = shared_down_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
+        TRY(c, hipEventRecord(c->ejoin, c->side));
+    }
     TRY(c, launch_router_logits(L->gate_inp, x, n, ne, E, c->logits.p, rp, st));
     prof_mark(c, ev, 2);
     if (share) {   // every row's topk picks, then the keep across the rows
-        ALLOC(c, c->sel8, (size_t) n * tsel); ALLOC(c, c->w8, (size_t) n * tsel);
         TRY(c, launch_router_select(c->logits.p, rp, E, L->probs_b, n, ne, c->n_group, c->topk_group, tsel, c->scale, c->probs.p, c->sel8.p, c->w8.p, st, tsel, 0.f));
         TRY(c, launch_keep_share(c->sel8.p, c->w8.p, n, tsel, tk, renorm, c->sel.p, c->wts.p, st));
     } else {
         TRY(c, launch_router_select(c->logits.p, rp, E, L->probs_b, n, ne, c->n_group, c->topk_group, tsel, c->scale, c->probs.p, c->sel.p, c->wts.p, st, tk, renorm));
     }
     prof_mark(c, ev, 3);
-    int * dsc = nullptr;
-    if (const size_t nd = dispatch_scratch_ints(P)) { ALLOC(c, c->dscr, nd); dsc = c->dscr.p; }
     TRY(c, launch_dispatch(c->sel.p, P, ne, c->counts.p, c->offsets.p, c->perm.p, c->inv.p, c->act.p, c->nact.p, st, dsc));
     if (mfma) {
         const PfTable iq = { c->pcols.p, c->pncols.p, pf_tok(n), pf_few(n), pf_tok(n) };
@@ -680,8 +701,36 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         prof_mark(c, ev, 6);
         return FL_OK;
     }
+    if (few) {
+        const PfTable iq = { c->pcols.p, c->pncols.p, pf_tok(n), pf_few(n), pf_tok(n) };
+        TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, n, P, iq, PfTable{}, st));
+        prof_mark(c, ev, 4);
+        const int nshi = prefill_shared_cols(n, iq.tok);
+        PrefillArgs g{};
+        g.tab = c->tab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
+        g.estride = (size_t) H * (E / 256) * IQ2B; g.sh[0] = (const uint8_t *) L->sh_gate; g.sh[1] = (const uint8_t *) L->sh_up;
+        g.perm = c->perm.p; g.topk = tk; g.P = P; g.R = H; g.K = E; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = n;
+        g.bq = c->xq.p; g.bd = c->xd.p; g.out = c->h.p; g.gdbg = c->dbg_gu ? c->g.p : nullptr; g.udbg = c->dbg_gu ? c->u.p : nullptr;
+        g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr; g.col0 = ksh ? nshi : 0;
+        TRY(c, launch_few_gemm(g, c->ncu, st));
+        if (ksh && !side) { if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, st)) { return rc; } }
+        TRY(c, launch_quant_q8k(c->h.p, (int64_t) (ksh ? P : P + n), H, c->hq.p, c->hd.p, st));   // (a K-quant shared expert's rows: shared_swiglu)
+        prof_mark(c, ev, 5);
+        if (lf[0] == FL_IQ2) {
+            PrefillArgs d = g;
+            d.w[0] = (const uint8_t *) L->down_exps; d.w[1] = nullptr; d.sh[0] = (const uint8_t *) L->sh_down; d.sh[1] = nullptr;
+            d.R = E; d.K = H; d.nmat = 1; d.bq = c->hq.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr; d.col0 = nshi;
+            TRY(c, launch_few_gemm(d, c->ncu, st));
+        } else {
+            TRY(c, routed_down_kq(c, L, P, E, H, ne));
+        }
+        if (side) { TRY(c, hipStreamWaitEvent(st, c->ejoin, 0)); }
+        else if (int rc = shared_down_sep(c, L, n, P, E, H, tk, st)) { return rc; }
+        TRY(c, launch_combine(c->o.p, c->inv.p, c->wts.p, n, tk, E, P, resid, y, nullptr, st));
+        prof_mark(c, ev, 6);
+        return FL_OK;
+    }
     prof_mark(c, ev, 4);
-    const bool ksh = lf[1] != FL_IQ2;   // the shared gate / up in K-quants: run beside the routed IQ2_XXS tasks
     ExpertArgs a = expert_args(c, n, P, ksh ? 0 : 1);
     a.w[0] = (const uint8_t *) L->gate_exps; a.w[1] = (const uint8_t *) L->up_exps; a.estride = (size_t) H * (E / 256) * IQ2B;
     a.sh[0] = (const uint8_t *) L->sh_gate; a.sh[1] = (const uint8_t *) L->sh_up;
@@ -690,17 +739,6 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     a.h = c->h.p; a.hq = c->hq.p; a.hd = c->hd.p;
     a.gdbg = c->dbg_gu ? c->g.p : nullptr; a.udbg = c->dbg_gu ? c->u.p : nullptr;
     expert_counters(c, a, 0);
-    // A K-quant shared expert (one latency-bound mat-vec of 10-12 MB per matrix) runs on the side stream beside the
-    // routed launches: it reads x's Q8_K and writes only its own rows (h / Q8_K(h) rows P .. P + n - 1, o rows P ..,
-    // ksg / ksu), which no routed kernel touches; the combine waits for it.
-    const bool side = ksh && kq && lf[3] != FL_IQ2 && !c->no_side;
-    if (side) {
-        ALLOC(c, c->ksg, (size_t) n * H); ALLOC(c, c->ksu, (size_t) n * H);
-        TRY(c, hipEventRecord(c->efork, st)); TRY(c, hipStreamWaitEvent(c->side, c->efork, 0));
-        if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
-        if (int rc = shared_down_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
-        TRY(c, hipEventRecord(c->ejoin, c->side));
-    }
     TRY(c, launch_experts_gateup(a, c->ncu, st));
     if (ksh && !side) { if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, st)) { return rc; } }   // h rows P .. P + n - 1
     prof_mark(c, ev, 5);

@@ -470,3 +470,46 @@ def test_prefill_mixed_formats_mfma(ctx, fm, n):
         assert ok, err
     del layer, base, down, shg, shu, shd
     torch.cuda.empty_cache()
+
+
+# rows at the edges of the kernels' column sizes: the decode batches (from 16 slots on the columns of at most 8), the
+# 16-token tiles and 64-token columns of the K-quant downs, the 8- and 112-token columns of the IQ2_XXS matrices
+EDGE_N = {orc.Q3K: (2, 8, 9, 16, 17, 48, 49, 65, 129), orc.Q2K: (2, 7, 9, 17, 33, 64, 129), 4: (3, 8, 129, 161, 224, 257, 300)}
+
+
+@pytest.mark.parametrize("fm", [PF_FMTS[0], PF_FMTS[1], PF_FMTS[2], (4, 4, 4, 4)], ids=["q3k_q5q5q6", "q2k_iq2", "iq2_q5q5q6", "iq2"])
+def test_column_edges_match_per_pass(ctx, fm):
+    """The grouped kernels against the per-pass ones, bit for bit (h, its Q8_K, o, y), where the column sizes change: a
+    router bias so wide that nearly every row takes the same experts, so the columns hold about n slots (or their equal
+    parts), beside experts with a few. 8 and 2 kept picks; a 64-expert layer."""
+    import torch
+    from loki_amd import MoeLayerWeights
+    from tests._helpers import make_x
+    ne, seed = 64, 8600 + 10 * (fm[0] + fm[1])
+    base = MoeLayerWeights.synthetic(ctx, seed, n_exp=ne, bias_sigma=0.4)
+    mats = [_kq_device(torch, f, r * k, c, seed + 1 + i) if f != 4 else m
+            for i, (f, r, k, c, m) in enumerate(((fm[0], ne, E, H, base.down), (fm[1], 1, H, E, base.sh_gate),
+                                                 (fm[2], 1, H, E, base.sh_up), (fm[3], 1, E, H, base.sh_down)))]
+    layer = MoeLayerWeights(base.gate_inp, base.probs_b, base.gate, base.up, *mats, n_exp=ne)
+    ctx.set_layer_formats(*fm)
+    try:
+        for n in EDGE_N[fm[0]]:
+            x = make_x(ctx, n, seed=seed + n)
+            for keep in (0, 2):
+                print("column edges %s n %d keep %d" % (fm, n, keep), flush=True)
+                ctx.set_keep(keep, 2.5)
+                got = {}
+                for on in (True, False):
+                    ctx.set_prefill_mfma(on)
+                    with ctx.using_fused(0):
+                        y = ctx.moe_layer(layer, x)
+                        ctx.sync()
+                    d = ctx.debug()
+                    got[on] = {"y": y.cpu().numpy(), "h": ctx.d2h(d.h, (d.P + n, H), np.float32), "hq": ctx.d2h(d.hq, (d.P + n, H), np.int8),
+                               "o": ctx.d2h(d.o, (d.P + n, E), np.float32)}
+                for k in got[False]:
+                    assert np.array_equal(got[True][k].view(np.uint8), got[False][k].view(np.uint8)), (n, keep, k)
+    finally:
+        ctx.set_prefill_mfma(True); ctx.set_layer_formats(); ctx.set_keep(0)
+    del layer, base, mats
+    torch.cuda.empty_cache()
