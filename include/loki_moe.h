@@ -261,9 +261,9 @@ int fl_set_debug(FLCtx *, int flags);
  * the caller must check before trusting any output of a mode-2 decode, and, without waiting, by the next
  * fl_moe_layer / fl_moe_layer_normed call on the context, which returns FL_EHIP until fl_sync has reported it. */
 int fl_set_fused(FLCtx *, int mode);
-/* single-token decode with all 8 picks kept, on a 256-CU device: 1 (default) = the single launch organised by XCD
- * (pick k's expert runs on the 32 CUs of XCD k, its down split by K-block among the four workgroups that produce each
- * h block), 0 = the general single-launch decode block. Both give bit-identical outputs. */
+/* single-token decode with 8 picks drawn, on a 256-CU device: 1 (default) = the single launch organised by XCD
+ * (with all 8 kept pick k's expert runs on the 32 CUs of XCD k, with 3 or 4 kept on two XCDs, with 1 or 2 on four; its
+ * down split by K-block among the workgroups that produce each h block), 0 = the general single-launch decode block. Both give bit-identical outputs. */
 int fl_set_decode1(FLCtx *, int on);
 /* batches above the decode sizes (n > 8, E 7168, H 2048): 1 (default) = the expert products as grouped GEMMs on the
  * matrix cores (no counterpart in the reference, whose wide path is tc_matvec per arena batch, src/fused_layer.cu:540-561);

@@ -410,7 +410,7 @@ int decode_picks(FLCtx * c, DecodeArgs & d) {
     if (int rc = decode_tagged(c, c->st)) { return rc; }
     d.tab = c->tab.p; d.tlogits = c->dlogit.p; d.th = c->dth.p; d.to = c->dto.p; d.xqx = decode_xq(c);
     d.epoch = c->epoch; d.err = c->derr.p; d.herr = c->herr ? c->herr_dev : nullptr;
-    if (d.n == 1 && d.topk == MAXK && d.keep == MAXK && decode1_ready(c)) {
+    if (decode1_takes(d) && decode1_ready(c)) {
         TRY(c, launch_moe_decode1(d, c->fused == 1, c->st));
         c->last_kernel = 2;
     } else {
@@ -421,7 +421,7 @@ int decode_picks(FLCtx * c, DecodeArgs & d) {
     return FL_OK;
 }
 static hipError_t launch_decode(FLCtx * c, const DecodeArgs & d, hipStream_t st) {
-    if (d.n == 1 && d.topk == MAXK && d.keep == MAXK && decode1_ready(c)) { c->last_kernel = 2; return launch_moe_decode1(d, c->fused == 1, st); }
+    if (decode1_takes(d) && decode1_ready(c)) { c->last_kernel = 2; return launch_moe_decode1(d, c->fused == 1, st); }
     c->last_kernel = 1;
     return launch_moe_decode(d, c->dec_grid, c->fused == 1, st);
 }
@@ -555,7 +555,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     // one-token kernel reads in place; at prefill sizes every matrix on a grouped GEMM that takes its format
     static_assert(FL_Q6K == 1 && FL_Q5K == 3 && FL_Q2K == 5 && FL_Q3K == 6, "the FL_ codes are the K-quant kernels' format codes");
     const int kd1 = (lf[0] == FL_Q2K || lf[0] == FL_Q3K) && lf[1] == FL_Q5K && lf[2] == FL_Q5K && lf[3] == FL_Q6K ? lf[0] : 0;
-    const bool kq1 = kq && kd1 != 0 && n == 1 && tsel == MAXK && tk == MAXK && decode1_ready(c);
+    const bool kq1 = kq && kd1 != 0 && n == 1 && tsel == MAXK && decode1_ready(c);
     const bool fused = (!kq || kq1) && c->fused && n <= 8 && E == 7168 && H == 2048 && decode_rule_ok(ne, c->n_group) && decode_ready(c);
     const bool mfma = !fused && c->pf_mfma && n > 8 && E == 7168 && H == 2048;
     // a decode batch of a K-quant layer: its IQ2_XXS matrices on the matrix-core kernel of columns of at most 8 slots. Two

@@ -1,4 +1,4 @@
-// moe_decode1.hip -- the MoE block for one decode token (top-8 kept) in one launch, organised by XCD.
+// moe_decode1.hip -- the MoE block for one decode token (top-8, all or fewer kept) in one launch, organised by XCD.
 //
 // Reference path (src/fused_layer.cu): router_probs + router_topk (:313-332), the host round-trip (fl_fetch :587-598,
 // eng:793-818), fl_moe (:599-612): quant_x, tc_matvec gate/up, swiglu_q8, tc_matvec down, moe_combine. Here the
@@ -14,7 +14,8 @@
 //      expert sel[x] in two phases of 32 rows, 256 kb_p + 32 (i % 8) .. + 31 with kb_0 = i / 8 and kb_1 = 4 + i / 8,
 //      each 28 items (one matrix, two 256-weight blocks, 32 rows) that the waves claim from an LDS counter, so the
 //      eight workgroups of (slot, i / 8) complete h block kb_0 half-way through the gate/up and h block kb_1 at its end
-//      (the K-quant variants: h rows kb * 256 + q * 64 .. + 63 with kb = i / 4, q = i % 4, as 56 items of 64 rows);
+//      (the K-quant variants: h rows kb * 256 + q * 64 .. + 63 with kb = i / 4, q = i % 4, as 56 items of 64 rows; with
+//      fewer than eight picks kept a slot takes 1, 2 or 4 XCDs: gate_upk);
 //   3. each workgroup quantises the h blocks it needs to Q8_K and runs the slot's down on them (split-K: one
 //      256-weight block per row, one row per lane): K-block kb_0 for an eighth of its 7168 rows, 3 or 4 row groups of
 //      the shared expert's down for K-block x, then K-block kb_1 for the same eighth -- the first two while block kb_1's
@@ -47,8 +48,6 @@ using GX1 = Geo<7, 0>;                 // the token's staged Q8_K row: 28 blocks
 constexpr int NBX1 = E1 / QK, NBH1 = H1 / QK;    // 28, 8 blocks
 constexpr int SLOTS1 = 9;              // 8 picks + the shared expert (slot 8)
 constexpr int BCAST1 = 1024;           // tagged words 1024 + 16 x .. + 15: XCD x's picks and weights (one-token calls use 0..255)
-constexpr int QROWS1 = E1 / 4;         // routed down rows per workgroup (a quarter): 1792 = 28 row groups
-constexpr int RGQ1 = QROWS1 / 64;      // 28
 constexpr int RGE1 = E1 / 64;          // 112 row groups of the shared expert's down block
 constexpr int CROWS1 = E1 / G1;        // combine rows per workgroup: 28
 constexpr int GU_STEPS1 = NBX1 / 4;    // 7
@@ -241,8 +240,8 @@ __device__ __noinline__ void router1(const D1Args & a, lds1_t lds, int wave, LK_
 constexpr int S_P = M_TERMS;   // select_ds8's scratch (the gate/up terms' space, unused until the picks are known)
 static_assert(S_P + 112 * 4 <= M_TERMS + NITEM1 * 64 * 4, "select_ds8's scratch inside the gate/up terms");
 
-// returns whether the picks and weights in M_SEL are valid
-__device__ __forceinline__ bool select1(const D1Args & a, lds1_t lds) {
+// returns whether the picks and weights in M_SEL are valid; KEEP: a.keep of the picks are kept
+template <bool KEEP> __device__ __forceinline__ bool select1(const D1Args & a, lds1_t lds) {
 #pragma clang fp contract(off)
     const int lane = lane_id();
     float bv[4];
@@ -278,6 +277,13 @@ __device__ __forceinline__ bool select1(const D1Args & a, lds1_t lds) {
         TRACE1V(24, fast ? 1 : 2);
     } else {
         select_token_p<false>(pv, bv, a.n_exp, a.n_group, a.topk_group, MAXK, a.scale, nullptr, so, wo, MAXK, 0.f);
+    }
+    if constexpr (KEEP) {
+        lds_visible();
+        const int sm = lane < MAXK ? so[lane] : -1;
+        const float wm = lane < MAXK ? wo[lane] : 0.f;
+        lds_visible();
+        keep_heaviest(sm, wm, MAXK, a.keep, a.renorm, so, wo);
     }
     return true;
 }
@@ -609,6 +615,60 @@ __device__ __forceinline__ void gate_up2(const D1Args & a, lds1_t lds, LK_LOCAL 
     __builtin_amdgcn_s_setprio(0);
 }
 
+// The routed gate/up when fewer than 8 picks are kept: slot s runs on the M XCDs M s .. M s + M - 1 (M = 1 for 5 .. 7 kept, 2
+// for 3 .. 4, 4 for 1 .. 2), each computing 8 / M of the slot's h blocks, so that few experts' weights stream through twice
+// or four times the CUs. Role (x, i)
+// takes the 64 / M h rows hrowk(x, i) .. in one phase of 56 / M items (one matrix, M consecutive blocks, 64 / M rows: lane
+// l the block l / (64 / M) and row l % (64 / M)); the 4 M workgroups of an h block share the XCD, as the down's hand-off
+// wants. One token on the n <= 8 block -> here: 1 kept expert 33.8 -> 20.5 us, 2 34.2 -> 19.6, 3 34.9 -> 24.2, 4 35.6 ->
+// 25.1, 5 36.2 -> 29.6, 7 38.4 -> 30.7 (of the real formats, against the per-pass kernels, 2 67.8 -> 27.5, 4 69.7 -> 33.1); what is left is the router, the picks' hand-off and two memory latencies behind them.
+template <int M> __device__ __forceinline__ int hblkk(int xcd, int li) { return xcd % M * (NBH1 / M) + li / (4 * M); }
+template <int M> __device__ __forceinline__ void gate_upk(const D1Args & a, lds1_t lds, LK_LOCAL unsigned * ctl, const uint8_t * gm,
+                                                          const uint8_t * um, int slot, int h0, uint32_t tr, int r) {
+#pragma clang fp contract(off)
+    constexpr int RW = 64 / M, NIT = 2 * NBX1 / M;
+    static_assert(NBX1 % M == 0 && 2 * NBX1 * RW * 4 <= NITEM1 * 64 * 4, "whole items; the terms' space");
+    const int lane = lane_id(), bl = lane / RW, rr = lane % RW;
+    LK_LOCAL float * terms = reinterpret_cast<LK_LOCAL float *>(lds + M_TERMS);   // [matrix][block][RW rows]
+    const uint8_t * xr = (const uint8_t *) (lds + M_X);
+    constexpr size_t DREG = (size_t) (H1 / 64) * NBX1 * 4096;
+    const int g64 = h0 >> 6, row = (h0 & 63) + rr;
+    auto claim = [&](GuItem & it) {
+        unsigned c = 0;
+        if (lane == 0) { c = __hip_atomic_fetch_add(ctl + C_GUCLAIM, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+        it.c = (int) __builtin_amdgcn_readfirstlane(c);
+        if (it.c >= NIT) { return; }
+        const int j = M * (it.c >> 1) + bl;
+        const uint8_t * mat = uniform1((it.c & 1) ? um : gm);
+        it.d = *gptr(reinterpret_cast<const uint16_t *>(mat + DREG + ((size_t) g64 * NBX1 + j) * 128 + row * 2));
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t * qb = mat + ((size_t) g64 * NBX1 + j) * 4096 + row * 16;
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4) { it.w[c4] = load_nt(qb + c4 * 1024); }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    GuItem it;
+    claim(it);
+    while (it.c < NIT) {
+        const int m = it.c & 1, j = M * (it.c >> 1) + bl;
+        const int bsum = block_bsum_dpp(it.w, tr, xr + j * GX1::XBLK, r);   // each 16-lane row reads its own block
+        const float dx = reinterpret_cast<const float *>(xr + NBX1 * GX1::XBLK)[j];
+        terms[(m * NBX1 + j) * RW + rr] = (h2f(it.d) * dx) * (float) bsum;
+        if (arrive1(ctl + C_GUDONE, NIT)) {
+            // lanes 0 .. RW - 1 fold the gate rows in block order, the next RW (M = 1: the same ones) the up rows
+            const LK_LOCAL float * tp = terms + (bl & 1) * NBX1 * RW + rr;
+            float v = 0.f, u = 0.f;
+#pragma unroll 4
+            for (int k = 0; k < NBX1; ++k) { v = v + tp[k * RW]; if constexpr (M == 1) { u = u + tp[(NBX1 + k) * RW]; } }
+            if constexpr (M > 1) { u = __shfl_xor(v, RW); }
+            if (bl == 0) {
+                st_xcd1(a.th + (size_t) slot * H1 + h0 + rr, a.epoch, __builtin_bit_cast(uint32_t, det_silu(0.125f * v) * (0.125f * u)));
+            }
+        }
+        claim(it);
+    }
+}
+
 // ---------------------------------------------------------------- down: one 256-weight block per row
 // A unit is one 64-row group of one down matrix at one K-block: lane l owns row l (4 chunks + d); every lane's block
 // product uses the same staged h block, so the activations come by DPP from the 16 lanes that hold them.
@@ -734,13 +794,14 @@ __device__ __forceinline__ int dn_run1(const D1Args & a, DnRing1<F> & g, int uen
 // thread (row i, slot s) of the first 252: the 8 tagged block terms of its row and slot, folded in block order,
 // * 0.125 for an IQ2_XXS matrix (its grid scale; the K-quant terms carry their scales); then thread i < 28 forms
 // y = sum_k w_k o_k (k order) + o_shared (+ the residual)
-template <bool KQ> __device__ __forceinline__ bool combine1(const D1Args & a, lds1_t lds) {
+template <bool KQ, bool KEEP> __device__ __forceinline__ bool combine1(const D1Args & a, lds1_t lds) {
 #pragma clang fp contract(off)
     LK_LOCAL float * cmb = reinterpret_cast<LK_LOCAL float *>(lds + M_CMB);
     const LK_LOCAL float * wts = reinterpret_cast<const LK_LOCAL float *>(lds + M_SEL + MAXK * 4);
     const int t = threadIdx.x, row0 = blockIdx.x * CROWS1;
     bool ok = true;
-    if (t < CROWS1 * SLOTS1) {
+    const int keep = KEEP ? a.keep : MAXK;   // (slots keep .. 7 do not exist)
+    if (t < CROWS1 * SLOTS1 && (!KEEP || t % SLOTS1 < keep || t % SLOTS1 == MAXK)) {
         const int i = t / SLOTS1, s = t % SLOTS1, row = row0 + i;
         uint64_t w[NBH1];
         auto issue = [&]() {
@@ -781,7 +842,7 @@ template <bool KQ> __device__ __forceinline__ bool combine1(const D1Args & a, ld
         } else {
             float mv = cmb[t * SLOTS1] * wts[0];
 #pragma unroll
-            for (int k = 1; k < MAXK; ++k) { mv = mv + cmb[t * SLOTS1 + k] * wts[k]; }
+            for (int k = 1; k < MAXK; ++k) { if (!KEEP || k < keep) { mv = mv + cmb[t * SLOTS1 + k] * wts[k]; } }
             float yv = mv + cmb[t * SLOTS1 + MAXK];
             if (a.resid) { yv = yv + gptr(a.resid)[row]; }
             gptr(a.y)[row] = yv;
@@ -791,25 +852,26 @@ template <bool KQ> __device__ __forceinline__ bool combine1(const D1Args & a, ld
     return true;
 }
 
-// the layer's routing outputs from the picks (workgroup 0): for one token the eight picks are distinct experts, so the
+// the layer's routing outputs from the K kept picks (workgroup 0): for one token they are distinct experts, so the
 // dispatch is their sort by expert id (ties impossible): perm / inv / act from the ranks, counts / offsets by expert
-__device__ __noinline__ void routing1(const D1Args & a, lds1_t lds) {
+template <bool KEEP> __device__ __noinline__ void routing1(const D1Args & a, lds1_t lds) {
+    const int K = KEEP ? a.keep : MAXK;
     const LK_LOCAL int * sel = reinterpret_cast<const LK_LOCAL int *>(lds + M_SEL);
     const LK_LOCAL float * wts = reinterpret_cast<const LK_LOCAL float *>(lds + M_SEL + MAXK * 4);
     const int lane = lane_id();
-    if (lane < MAXK) {
+    if (lane < K) {
         const int e = sel[lane];
         int rank = 0;
 #pragma unroll
-        for (int j = 0; j < MAXK; ++j) { rank += sel[j] < e ? 1 : 0; }
+        for (int j = 0; j < MAXK; ++j) { rank += j < K && sel[j] < e ? 1 : 0; }
         gptr(a.sel)[lane] = e; gptr(a.wts)[lane] = wts[lane];
         gptr(a.perm)[rank] = lane; gptr(a.inv)[lane] = rank; gptr(a.act)[rank] = e;
     }
-    if (lane == 0) { *gptr(a.nact) = MAXK; }
+    if (lane == 0) { *gptr(a.nact) = K; }
     for (int x = lane; x <= a.n_exp; x += 64) {
         int lt = 0, eq = 0;
 #pragma unroll
-        for (int j = 0; j < MAXK; ++j) { const int ej = sel[j]; lt += ej < x ? 1 : 0; eq += ej == x ? 1 : 0; }
+        for (int j = 0; j < MAXK; ++j) { const int ej = j < K ? sel[j] : NEXP_MAX; lt += ej < x ? 1 : 0; eq += ej == x ? 1 : 0; }
         gptr(a.offsets)[x] = lt;
         if (x < a.n_exp) { gptr(a.counts)[x] = eq; }
     }
@@ -839,7 +901,8 @@ __device__ __forceinline__ void ext_list1(lds1_t lds) {
 
 // ---------------------------------------------------------------- the kernel
 // FD: 0 (every matrix IQ2_XXS), or the routed down's K-quant (the shared expert then Q5_K / Q5_K / Q6_K)
-template <int FD>
+// KEEP: fewer than eight picks are kept, a slot on M XCDs: 5 .. 7 (M = 1), 3 .. 4 (M = 2), 1 .. 2 (M = 4)
+template <int FD, int M, bool KEEP>
 __global__ void __launch_bounds__(NT1, 1) k_moe_decode1(const DecodeArgs args) {
 #pragma clang fp contract(off)
     (void) sizeof(args);   // read in place in the kernarg segment (scalar loads), as the general decode kernel does
@@ -913,7 +976,7 @@ __global__ void __launch_bounds__(NT1, 1) k_moe_decode1(const DecodeArgs args) {
         }
     } else if (li == 0 && wave == 0) {
         __builtin_amdgcn_s_setprio(3);
-        const bool ok = select1(a, lds);
+        const bool ok = select1<KEEP>(a, lds);
         __builtin_amdgcn_s_setprio(0);
         {
             lds_visible();
@@ -952,12 +1015,15 @@ __global__ void __launch_bounds__(NT1, 1) k_moe_decode1(const DecodeArgs args) {
     // 3. routed gate/up: expert sel[xcd], h rows kb * 256 + qq * 64 .. + 63 (one row group of gate and up), as items
     //    the waves claim from an LDS counter
     const int kb = li / 4, qq = li % 4;
-    {
-        const int e = reinterpret_cast<const LK_LOCAL int *>(lds + M_SEL)[xcd];
+    const int slot = xcd / M, hk = KEEP ? hblkk<M>(xcd, li) : kb;   // the slot, the workgroup's h block (FD 0, eight kept: two)
+    const bool mine = !KEEP || slot < a.keep;                       // (without a slot: the shared expert's units alone)
+    if (mine) {
+        const int e = reinterpret_cast<const LK_LOCAL int *>(lds + M_SEL)[slot];
         if ((unsigned) e >= (unsigned) a.n_exp) { report1(a, 32); return; }
         const uint8_t * gm = uniform1(a.gate + (size_t) e * a.estride), * um = uniform1(a.up + (size_t) e * a.estride);
         TRACE1(5);
-        if constexpr (FD == 0) { gate_up2(a, lds, ctl, gm, um, xcd, li, tr, r); }
+        if constexpr (KEEP) { gate_upk<M>(a, lds, ctl, gm, um, slot, hk * QK + li % (4 * M) * (64 / M), tr, r); }
+        else if constexpr (FD == 0) { gate_up2(a, lds, ctl, gm, um, xcd, li, tr, r); }
         else { gate_up1(a, lds, ctl, gm, um, xcd, kb * QK + qq * 64, tr, r); }
         TRACE1(6);
     }
@@ -965,10 +1031,47 @@ __global__ void __launch_bounds__(NT1, 1) k_moe_decode1(const DecodeArgs args) {
     // 4. down: the workgroup's units (28 routed row groups at K-block kb, 3 or 4 shared row groups at K-block xcd),
     //    claimed by the waves in order; each wave's first unit streams in while the h blocks are polled and staged
     const int nsh = li < RGE1 - 3 * 32 ? 4 : 3;   // shared row groups li, li + 32, .. (< 112)
-    const int nunits = RGQ1 + nsh;
-    const int e_dn = reinterpret_cast<const LK_LOCAL int *>(lds + M_SEL)[xcd];
+    constexpr int RGK = RGE1 / (4 * M);           // routed row groups of a workgroup when it has one h block
+    const int rg0 = li % (4 * M) * RGK, nunits = nsh + (mine ? RGK : 0);
+    const int e_dn = mine ? reinterpret_cast<const LK_LOCAL int *>(lds + M_SEL)[slot] : 0;
     LK_LOCAL unsigned * dclaim = ctl + C_DNCLAIM;
-    if constexpr (FD == 0) {
+    if constexpr (KEEP && FD == 0) {
+        // units in claim order: the shared expert's row groups at K-block x (h block x, long complete), then the slot's row
+        // groups at the workgroup's own K-block; the first wave out of gate/up items stages the two h blocks in that order
+        const uint8_t * dmat = uniform1(a.down + (size_t) e_dn * a.estride), * smat = uniform1(a.sh_down);
+        auto claim_unit = [&](Dn1 & d) -> int {
+            unsigned c = 0;
+            if (lane == 0) { c = __hip_atomic_fetch_add(dclaim, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+            const int u = (int) __builtin_amdgcn_readfirstlane(c);
+            if (u < nsh) { dn1_issue(smat, li + 32 * u, xcd, d); }
+            else if (u < nunits) { dn1_issue(dmat, rg0 + (u - nsh), hk, d); }
+            return u;
+        };
+        unsigned got = 0;
+        if (lane == 0) { got = __hip_atomic_fetch_add(ctl + C_LR, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+        if (__builtin_amdgcn_readfirstlane(got) == 0) {
+            bool ok = stage_h1(a, a.th + (size_t) 8 * H1 + (size_t) xcd * QK, lds + M_HS);
+            if (!ok) { report1(a, 1); }
+            flag1(ctl + C_HS, ok ? 1u : 2u);
+            if (mine) {
+                ok = stage_h1(a, a.th + (size_t) slot * H1 + (size_t) hk * QK, lds + M_HR);
+                if (!ok) { report1(a, 1); }
+                flag1(ctl + C_HR, ok ? 1u : 2u);
+            }
+        }
+        Dn1 dn;
+        for (int u = claim_unit(dn); u < nunits; u = claim_unit(dn)) {
+            const bool sh = u < nsh;
+            const unsigned v = wait1(ctl + (sh ? C_HS : C_HR), 1);
+            lds_visible();
+            if (v != 1) { if (v == 0) { report1(a, 8); } return; }
+            const uint8_t * hbp = (const uint8_t *) (lds + (sh ? M_HS : M_HR));
+            const int bsum = block_bsum_dpp(dn.w, tr, hbp, r);
+            const float dx = *reinterpret_cast<const float *>(hbp + QK);
+            const int g = sh ? li + 32 * u : rg0 + (u - nsh);
+            st_tag1(a.to + ((size_t) (sh ? 8 : slot) * NBH1 + (sh ? xcd : hk)) * E1 + (size_t) g * 64 + lane, a.epoch, (h2f(dn.d) * dx) * (float) bsum);
+        }
+    } else if constexpr (FD == 0) {
         // units in claim order: the 14 row groups (i % 8) * 14 .. + 13 at K-block kb_0 (h block kb_0, complete since
         // phase 1), the shared expert's row groups at K-block x, then the same 14 row groups at K-block kb_1. The first
         // wave to need an h block polls and stages it (the others wait on its LDS flag), so the hand-off of block kb_1
@@ -1040,13 +1143,13 @@ __global__ void __launch_bounds__(NT1, 1) k_moe_decode1(const DecodeArgs args) {
         };
         const uint32_t r8 = (uint32_t) lane >> 3;
         const Src ssrc = src1(a.sh_down, (uint64_t) E1 * RB6, r8 * RB6 + (uint32_t) xcd * kbytes<KF_Q6K>());
-        const Src rsrc = src1(a.down + (size_t) e_dn * a.dstride, (uint64_t) E1 * RBD, r8 * RBD + (uint32_t) kb * kbytes<FD>());
+        const Src rsrc = src1(a.down + (size_t) e_dn * a.dstride, (uint64_t) E1 * RBD, r8 * RBD + (uint32_t) hk * kbytes<FD>());
         auto g_s = [&](int u) { return li + 32 * u; };              // units 0 .. nsh - 1
-        auto g_r = [&](int u) { return qq * RGQ1 + (u - nsh); };    // units nsh .. nunits - 1
+        auto g_r = [&](int u) { return rg0 + (u - nsh); };           // units nsh .. nunits - 1
         // wave 0 stages the routed h block first (it polls until the block is complete), the others claim and
         // prime their rings while the h blocks form
-        if (wave == 0) {
-            const bool ok = stage_h1(a, a.th + (size_t) xcd * H1 + (size_t) kb * QK, lds + M_HR);
+        if (wave == 0 && mine) {
+            const bool ok = stage_h1(a, a.th + (size_t) slot * H1 + (size_t) hk * QK, lds + M_HR);
             if (!ok) { report1(a, 1); }
             flag1(ctl + C_HR, ok ? 1u : 2u);
         }
@@ -1062,22 +1165,25 @@ __global__ void __launch_bounds__(NT1, 1) k_moe_decode1(const DecodeArgs args) {
         lds_visible();
         const int un = dn_run1<KF_Q6K>(a, rs, nsh, ssrc, reinterpret_cast<const LK_LOCAL int8_t *>(lds + M_HS),
                                        *reinterpret_cast<const LK_LOCAL float *>(lds + M_HS + QK), 8, xcd, g_s, claim);
-        DnRing1<FD> rr;
-        dn_prime1<FD>(rr, un, nunits, rsrc, g_r, claim);
-        if (wait1(ctl + C_HR, 1) != 1) { return; }
-        lds_visible();
-        TRACE1(8);
-        (void) dn_run1<FD>(a, rr, nunits, rsrc, reinterpret_cast<const LK_LOCAL int8_t *>(lds + M_HR),
-                           *reinterpret_cast<const LK_LOCAL float *>(lds + M_HR + QK), xcd, kb, g_r, claim);
+        if (mine) {
+            DnRing1<FD> rr;
+            dn_prime1<FD>(rr, un, nunits, rsrc, g_r, claim);
+            if (wait1(ctl + C_HR, 1) != 1) { return; }
+            lds_visible();
+            TRACE1(8);
+            (void) dn_run1<FD>(a, rr, nunits, rsrc, reinterpret_cast<const LK_LOCAL int8_t *>(lds + M_HR),
+                               *reinterpret_cast<const LK_LOCAL float *>(lds + M_HR + QK), slot, hk, g_r, claim);
+        }
     }
     TRACE1(9);
 
     // 5. combine rows 28 b .. 28 b + 27 (a timed-out poll is flagged in LDS; no __syncthreads_and: it would take static
     //    LDS and move the table base off its 64 KB alignment)
-    combine1<FD != 0>(a, lds);
+    //    The last wave of workgroup 0 writes the routing outputs while the first four poll.
+    if (blockIdx.x == 0 && wave == W1 - 1 && !a.ext_sel) { routing1<KEEP>(a, lds); }
+    combine1<FD != 0, KEEP>(a, lds);
     if (wave == 0 && __hip_atomic_load(ctl + C_CMBFAIL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) { report1(a, 16); }
     TRACE1(10);
-    if (blockIdx.x == 0 && wave == W1 - 1 && !a.ext_sel) { routing1(a, lds); }
     if (a.fdone && wave == 0) {
         // this workgroup's combine rows are written (wave 0 wrote them): count it; the last one tells the host. No fence
         // per workgroup (an L2 write-back each): the rows go to the caller's memory before the count, and the last
@@ -1104,14 +1210,18 @@ __device__ int g_xcc1[G1];
 __global__ void k_xcc_probe1() { if (threadIdx.x == 0) { g_xcc1[blockIdx.x] = xcc_id1(); } }
 
 // the kernel's variants: every matrix IQ2_XXS; routed down Q2_K or Q3_K with the shared expert in Q5_K / Q5_K / Q6_K
-static const void * const kernels1[3] = { (const void *) k_moe_decode1<0>, (const void *) k_moe_decode1<KF_Q2K>,
-                                          (const void *) k_moe_decode1<KF_Q3K> };
+// by format and, with fewer than eight picks kept, by the XCDs of a slot
+#define LK_D1(F) { (const void *) k_moe_decode1<F, 1, false>, (const void *) k_moe_decode1<F, 1, true>, \
+                   (const void *) k_moe_decode1<F, 2, true>, (const void *) k_moe_decode1<F, 4, true> }
+static const void * const kernels1[3][4] = { LK_D1(0), LK_D1(KF_Q2K), LK_D1(KF_Q3K) };
+#undef LK_D1
 
 hipError_t decode1_init(int ncu, int * ok) {
     *ok = 0;
     if (ncu != G1) { return hipSuccess; }   // the XCD mapping needs one workgroup on each of 256 CUs
     hipError_t e = hipSuccess;
-    for (const void * k : kernels1) {   // every format variant fits one workgroup per CU
+    for (int v = 0; v < 12; ++v) {   // every variant fits one workgroup per CU
+        const void * k = kernels1[v / 4][v % 4];
         if ((e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, DEC1_LDS)) != hipSuccess) { return e; }
         int per = 0;
         if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, NT1, DEC1_LDS)) != hipSuccess) { return e; }
@@ -1131,13 +1241,13 @@ hipError_t decode1_init(int ncu, int * ok) {
 hipError_t launch_moe_decode1(const DecodeArgs & a, bool cooperative, hipStream_t st) {
     if ((a.ext_sel || a.spec_combine) && ((a.ext_sel && !a.ext_w) || !a.moe_out || !a.resid || a.prenorm)) { return hipErrorInvalidValue; }   // fl_moe's combine
     if ((a.spec_combine && (a.ext_sel || !a.hsel || !a.hdone)) || (a.fdone && !a.fcnt)) { return hipErrorInvalidValue; }
-    if (a.n != 1 || a.topk != MAXK || a.keep != MAXK || (!a.ext_sel && !decode_rule_ok(a.n_exp, a.n_group)) || a.E != E1 || a.H != H1 ||
+    if (!decode1_takes(a) || (!a.ext_sel && !decode_rule_ok(a.n_exp, a.n_group)) || a.E != E1 || a.H != H1 ||
         !a.th || !a.to || !a.tlogits || a.n_exp > NEXP_MAX || (a.kdown != 0 && a.kdown != KF_Q2K && a.kdown != KF_Q3K) ||
         (a.kdown != 0 && ((reinterpret_cast<uintptr_t>(a.down) | reinterpret_cast<uintptr_t>(a.sh_gate) |
                            reinterpret_cast<uintptr_t>(a.sh_up) | reinterpret_cast<uintptr_t>(a.sh_down) | a.dstride) & 3u))) {
         return hipErrorInvalidValue;   // K-quant matrices: 4-byte aligned (the slices' word loads)
     }
-    const void * k = kernels1[a.kdown == 0 ? 0 : a.kdown == KF_Q2K ? 1 : 2];
+    const void * k = kernels1[a.kdown == 0 ? 0 : a.kdown == KF_Q2K ? 1 : 2][a.keep == MAXK ? 0 : a.keep > 4 ? 1 : a.keep > 2 ? 2 : 3];
     DecodeArgs arg = a;
     void * params[] = { &arg };
     if (!cooperative) { return hipLaunchKernel(k, dim3(G1), dim3(NT1), params, DEC1_LDS, st); }

@@ -579,6 +579,29 @@ __device__ __forceinline__ void load_bias(const float * bias, int n_exp, float (
 #pragma unroll
     for (int j = 0; j < 4; ++j) { b[j] = 4 * lane + j < n_exp ? gptr(bias)[4 * lane + j] : 0.f; }
 }
+// the keep of select_token_p from its picks: lane r < topk holds pick r (sel_mine) and its weight (w_mine)
+template <class SO, class WO>
+__device__ __forceinline__ void keep_heaviest(int sel_mine, float w_mine, int topk, int keep, float renorm, SO sel_out, WO w_out) {
+#pragma clang fp contract(off)
+    const int lane = lane_id();
+    // rank of lane r's weight among the topk picks: heavier picks, then equal ones picked earlier
+    int rank = 0;
+    for (int j = 0; j < topk; ++j) {
+        const float o = __builtin_bit_cast(float, rdlane(__builtin_bit_cast(uint32_t, w_mine), j));
+        rank += (o > w_mine || (o == w_mine && j < lane)) ? 1 : 0;
+    }
+    const bool kept = lane < topk && rank < keep;
+    float f = 1.f; bool rescale = false;
+    if (renorm > 0.f) {
+        float sw = 0.0f;
+        for (int q = 0; q < keep; ++q) {   // the kept weights in kept order
+            const int l = first_lane(lane < topk && rank == q);
+            sw = sw + __builtin_bit_cast(float, rdlane(__builtin_bit_cast(uint32_t, w_mine), l));
+        }
+        if (sw > 1e-6f) { f = renorm / sw; rescale = true; }
+    }
+    if (kept) { sel_out[rank] = sel_mine; w_out[rank] = rescale ? w_mine * f : w_mine; }
+}
 // the rule from the lane's 4 probabilities p[j] = sigmoid(logit) of experts 4 lane + j
 // SCRATCH = false: the caller guarantees the DPP group path (decode_rule_ok) and passes no scratch
 template <bool SCRATCH = true>
@@ -675,23 +698,7 @@ __device__ __forceinline__ void select_token_p(const float (&p)[4], const float 
         if (lane < topk) { sel_out[lane] = sel_mine; w_out[lane] = w_mine; }
         return;
     }
-    // rank of lane r's weight among the topk picks: heavier picks, then equal ones picked earlier
-    int rank = 0;
-    for (int j = 0; j < topk; ++j) {
-        const float o = __builtin_bit_cast(float, rdlane(__builtin_bit_cast(uint32_t, w_mine), j));
-        rank += (o > w_mine || (o == w_mine && j < lane)) ? 1 : 0;
-    }
-    const bool kept = lane < topk && rank < keep;
-    float f = 1.f; bool rescale = false;
-    if (renorm > 0.f) {
-        float sw = 0.0f;
-        for (int q = 0; q < keep; ++q) {   // the kept weights in kept order
-            const int l = first_lane(lane < topk && rank == q);
-            sw = sw + __builtin_bit_cast(float, rdlane(__builtin_bit_cast(uint32_t, w_mine), l));
-        }
-        if (sw > 1e-6f) { f = renorm / sw; rescale = true; }
-    }
-    if (kept) { sel_out[rank] = sel_mine; w_out[rank] = rescale ? w_mine * f : w_mine; }
+    keep_heaviest(sel_mine, w_mine, topk, keep, renorm, sel_out, w_out);
 }
 // DeepSeek's rule (256 experts, 8 groups of 32, 4 groups kept, top 8 kept whole) on one wave, with the same picks in
 // the same order and the same weights as select_token_p, in far fewer dependent steps. The group stage is

@@ -125,8 +125,12 @@ size_t decode_xq_bytes();
 // grid workgroups (at most one per CU can be resident): a cooperative launch guarantees they are all resident; a
 // regular launch assumes it (nothing else running on the CUs) -- a violation ends in a reported wait timeout
 hipError_t launch_moe_decode(const DecodeArgs & a, int grid, bool cooperative, hipStream_t st);
-// one decode token with all topk = 8 picks kept, organised by XCD (moe_decode1.hip): 256 workgroups, one per CU of a
-// 256-CU device (*ok = 0 on other devices); same arguments, tagged buffers and results as launch_moe_decode
+// one decode token organised by XCD (moe_decode1.hip): 256 workgroups, one per CU of a 256-CU device (*ok = 0 on other
+// devices); same arguments, tagged buffers and results as launch_moe_decode. It takes all topk = 8 picks kept, or fewer
+// where the kernel routes (a slot on 1, 2 or 4 XCDs)
+inline bool decode1_takes(const DecodeArgs & a) {
+    return a.n == 1 && a.topk == MAXK && (a.keep == MAXK || (a.keep >= 1 && a.keep < MAXK && !a.ext_sel && !a.spec_combine && !a.share));
+}
 hipError_t decode1_init(int ncu, int * ok);
 size_t decode1_lds_bytes();
 hipError_t launch_moe_decode1(const DecodeArgs & a, bool cooperative, hipStream_t st);

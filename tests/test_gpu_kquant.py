@@ -354,6 +354,41 @@ def test_decode1_real_formats(ctx, down_fmt):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("down_fmt", [orc.Q2K, orc.Q3K], ids=["q2_K", "q3_K"])
+def test_decode1_real_formats_kept(ctx, down_fmt):
+    """One token of the real shards' formats with 1, 2, 3 and 6 kept picks (a slot on four, four, two XCDs and one) through
+    the one-token kernel: picks, weights and y bit-identical to the per-pass kernels, y also with the residual."""
+    import torch
+    from loki_amd import MoeLayerWeights
+    from tests._helpers import make_x
+    ne = 64
+    base = MoeLayerWeights.synthetic(ctx, 8180 + down_fmt, n_exp=ne)
+    down = _kq_device(torch, down_fmt, ne * E, H, 8190 + down_fmt)
+    sh = (_kq_device(torch, orc.Q5K, H, E, 8191), _kq_device(torch, orc.Q5K, H, E, 8192), _kq_device(torch, orc.Q6K, E, H, 8193))
+    layer = MoeLayerWeights(base.gate_inp, base.probs_b, base.gate, base.up, down, *sh, n_exp=ne)
+    ctx.set_layer_formats(down_fmt, orc.Q5K, orc.Q5K, orc.Q6K)
+    try:
+        for keep in (1, 2, 3, 6):
+            ctx.set_keep(keep, 2.5)
+            x, got = make_x(ctx, 1, seed=8200 + keep), {}
+            print("decode-1 real formats: down %s keep %d" % (NAMES[down_fmt], keep), flush=True)
+            for mode in (2, 0):
+                with ctx.using_fused(mode):
+                    y = ctx.moe_layer(layer, x).clone()
+                    ctx.sync()
+                    d = ctx.debug()
+                    assert d.kernel == (2 if mode else 0)
+                    got[mode] = (ctx.d2h(d.sel, (keep,), np.int32), ctx.d2h(d.wts, (keep,), np.float32), y.cpu().numpy(),
+                                 ctx.moe_layer_normed(layer, x, None, 1e-6, residual=True).cpu().numpy())
+                    ctx.sync()
+            for k in range(4):
+                assert np.array_equal(got[2][k].view(np.uint8), got[0][k].view(np.uint8)), (keep, k)
+    finally:
+        ctx.set_keep(0); ctx.set_layer_formats()
+    del layer, base, down, sh
+    torch.cuda.empty_cache()
+
+
 DEC_FMTS = [(orc.Q3K, orc.Q5K, orc.Q5K, orc.Q6K), (4, orc.Q5K, orc.Q5K, orc.Q6K)]
 
 

@@ -790,6 +790,49 @@ def test_decode1_fewer_experts(ctx):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("nexp,keep", [(256, 1), (256, 2), (256, 3), (256, 4), (256, 5), (256, 7), (64, 2), (128, 4)])
+def test_decode1_kept_matches_general(ctx, nexp, keep):
+    """One token with fewer than eight kept picks on the kernel organised by XCD (a slot on one, two or four XCDs) against the n <= 8
+    block and the per-pass kernels, and the checker's keep: every routing output and y bit for bit, also with the norm in
+    front and the residual behind (the two launches, which share that arithmetic)."""
+    import torch
+    from loki_amd import MoeLayerWeights
+    layer = MoeLayerWeights.synthetic(ctx, 7600 + nexp, n_exp=nexp, bias_sigma=0.01)
+    ctx.set_keep(keep, 2.5)
+    try:
+        for i in range(3):
+            x, got = make_x(ctx, 1, seed=7610 + i), {}
+            for name, m, d1 in (("decode1", 2, True), ("coop", 1, True), ("general", 2, False), ("per_pass", 0, True)):
+                ctx.set_decode1(d1)
+                with ctx.using_fused(m):
+                    y = ctx.moe_layer(layer, x).clone()
+                    ctx.sync()
+                    dbg = ctx.debug()
+                    assert dbg.kernel == {"general": 1, "per_pass": 0}.get(name, 2), name
+                    assert dbg.P == keep
+                    got[name] = [ctx.d2h(p, (k,), t) for p, k, t in (
+                        (dbg.sel, keep, np.int32), (dbg.wts, keep, np.float32), (dbg.perm, keep, np.int32), (dbg.inv, keep, np.int32),
+                        (dbg.act, keep, np.int32), (dbg.nact, 1, np.int32), (dbg.counts, nexp, np.int32),
+                        (dbg.offsets, nexp + 1, np.int32), (dbg.logits, nexp, np.float32), (dbg.probs, nexp, np.float32))] + [y.cpu().numpy()]
+                    if m == 2:
+                        for res in (False, True):
+                            got[name].append(ctx.moe_layer_normed(layer, x, None, 1e-6, residual=res).cpu().numpy())
+                        ctx.sync()
+            for name in ("decode1", "coop", "general"):
+                for k, v in enumerate(got["per_pass"][:11]):
+                    assert np.array_equal(got[name][k].view(np.uint8), v.view(np.uint8)), (name, k, i)
+            for k in (11, 12):
+                assert np.array_equal(got["decode1"][k].view(np.uint8), got["general"][k].view(np.uint8)), (k, i)
+            xs, W, b = x.cpu().numpy(), layer.gate_inp.cpu().numpy(), layer.probs_b.cpu().numpy()
+            _, _, so, wo = orc.router(W, b, xs)
+            sk, wk = orc.keep_experts(so, wo, keep, 2.5)
+            assert np.array_equal(got["decode1"][0], sk.ravel()) and np.array_equal(got["decode1"][1].view(np.uint32), wk.ravel().view(np.uint32))
+    finally:
+        ctx.set_decode1(True); ctx.set_keep(0)
+    del layer
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("pattern", ["pairs", "groups", "quads"])
 def test_decode1_selection_ties(ctx, pattern):
     """Exact ties in the selection, made by copying router rows and biases: "pairs" (expert e ^ 1 = e: tied keys
