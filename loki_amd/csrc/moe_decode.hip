@@ -13,7 +13,8 @@
 //      counting sort of the n * topk pairs) in its own LDS -- redundant, but cheaper than another device-wide hand-off.
 //      Waves without a token meanwhile run the shared expert's gate/up tasks (no routing needed);
 //   3. gate/up tasks: a task computes 8 gate rows and the same 8 up rows of one expert for one token and publishes
-//      h = silu(g) * u as epoch-tagged words; a workgroup's 8 waves take 8 consecutive tasks (one 64-row group);
+//      h = silu(g) * u as epoch-tagged words; a workgroup's 8 waves take 8 consecutive tasks (one 64-row group); the
+//      few tasks of a last round are shared by a workgroup's waves (gate_up_tail);
 //   4. down units round-robin over the workgroups: a unit is 256 output rows of one expert for one token (32 per wave).
 //      The waves issue their first weight loads, then wave w polls the tagged h of Q8_K block w and quantises it into
 //      LDS; after a barrier each wave computes its rows and publishes o as epoch-tagged words;
@@ -51,11 +52,17 @@ constexpr int PRE_BYTES = 2 * 7 * 64 * 4;
 constexpr int L_SCR = L_PRE;                                      // router sums [token][quarter] (phase 1) overlay them
 constexpr int L_RT = L_PRE + PRE_BYTES;                           // routing tables
 constexpr int RT_INTS = 4 * DMAX_P + 3 * (DMAX_P + 1) + 1 + 2 * DMAX_PS + 1;
-constexpr int L_CTL = L_RT + RT_INTS * 4;                         // hand-off words [8], staging flags [DW]
-constexpr int L_NRM = L_CTL + (8 + DW) * 4;                       // pre-norm scale per token [DMAX_N]
+constexpr int L_CTL = L_RT + RT_INTS * 4;                         // hand-off words [8], staging flags [DW], last round [8]
+constexpr int L_NRM = L_CTL + (16 + DW) * 4;                      // pre-norm scale per token [DMAX_N]
 // the caller's picks (ext_sel): per token its distinct ids ascending as [first k][summed weight], then their count
 constexpr int L_EXT = L_NRM + DMAX_N * 4, EXT_TOK = 2 * MAXK + 1;
 constexpr int DEC_LDS = L_EXT + DMAX_N * EXT_TOK * 4;
+// the last round's block terms [task][2][7][64] floats: in the rows of the tokens that the call does not have, two tasks
+// a row; with all eight, one task in the early shared task's area (which eight tokens do not use)
+constexpr int TAIL_MAX = 2;
+static_assert(2 * PRE_BYTES <= GG::XROW, "two tasks' terms in a token row");
+__device__ __forceinline__ int tail_tasks(int n) { return n == DMAX_N ? 1 : TAIL_MAX; }
+__device__ __forceinline__ int tail_terms(int n) { return n == DMAX_N ? L_PRE : L_XS + n * GG::XROW; }
 static_assert(DEC_LDS <= 160 * 1024, "LDS budget");
 static_assert(DMAX_N * 4 * 8 <= PRE_BYTES && DW * 112 * 4 <= PRE_BYTES, "router sums and selection scratch overlay the early task terms");
 
@@ -596,6 +603,59 @@ __device__ __forceinline__ void pre_shared_split(const DArgs & a, lds_t lds, con
     }
 }
 
+// The last round's tasks t0 + blockIdx.x + G i < t_end when they leave many waves idle (at most tail_tasks(n) of the eight a
+// workgroup runs in a round): a workgroup's waves share its tasks' steps. Items (task, step) are claimed from an LDS counter, each
+// wave with the next item's loads in flight; block terms go to LDS, and the wave completing a task folds them in block
+// order and publishes h -- the arithmetic of a pass. 3 rows of 3 picks (9 experts:
+// a ninth of the tasks left for a second round) 64.8 -> 56.1 us, with the shared keep 65.1 -> 58.6, 2 rows of 1 pick 35.8 ->
+// 32.5. At three or four tasks a workgroup it gained nothing (4 rows of 3 shared picks 67.1 -> 68.3), at six it lost (2 rows
+// of 3 picks 38.4 -> 41.8), hence TAIL_MAX; a call of its own instead of inline costs more than it gains (saved registers).
+__device__ __forceinline__ void gate_up_tail(const DArgs & a, lds_t lds, const Lane ln, int t0, int t_end, int ps0, int P, int nact) {
+#pragma clang fp contract(off)
+    const int G = gridDim.x, lane = lane_id();
+    const int nt = t0 + (int) blockIdx.x < t_end ? (t_end - 1 - t0 - (int) blockIdx.x) / G + 1 : 0;
+    LK_LOCAL unsigned * ctl = reinterpret_cast<LK_LOCAL unsigned *>(lds + L_CTL) + 8 + DW;   // [0] claims, [1 + i] steps of task i done
+    LK_LOCAL float * terms = reinterpret_cast<LK_LOCAL float *>(lds + tail_terms(a.n));
+    struct Item { GuTask t; uint4 w[4]; uint16_t d; int i, s; };
+    auto take = [&](Item & x) -> bool {
+        unsigned c = 0;
+        if (lane == 0) { c = __hip_atomic_fetch_add(ctl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+        c = __builtin_amdgcn_readfirstlane(c);
+        x.i = (int) c / GU_STEPS; x.s = (int) c % GU_STEPS;
+        if (x.i >= nt || !gu_task(a, lds, ln, t0 + (int) blockIdx.x + G * x.i, t_end, false, ps0, P, nact, x.t)) { return false; }
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4) { x.w[c4] = load_nt(x.t.ql + x.s * GU_QSTEP + c4 * 1024); }
+        x.d = *gptr(reinterpret_cast<const uint16_t *>(x.t.dl + x.s * GU_DSTEP));
+        return true;
+    };
+    auto run = [&](const Item & x) {
+        const int j = x.s * 4 + ln.q;
+        GuTask t = x.t;
+        for (t.u = 0; t.u < t.c; ++t.u) {   // both tokens from one load
+            const uint8_t * xr = gu_xrow(a, lds, t, P);
+            const int bsum = block_bsum_dpp(x.w, ln.tr, xr + j * GG::XBLK, ln.r);
+            const float dx = reinterpret_cast<const float *>(xr + GG::NB * GG::XBLK)[j];
+            terms[((2 * x.i + t.u) * GU_STEPS + x.s) * 64 + lane] = (h2f(x.d) * dx) * (float) bsum;
+        }
+        if (!lds_arrive(ctl + 1 + x.i, GU_STEPS)) { return; }
+        for (t.u = 0; t.u < t.c; ++t.u) {
+            float acc = 0.f;
+#pragma unroll
+            for (int s = 0; s < GU_STEPS; ++s) { acc = fold_rows(acc, terms[((2 * x.i + t.u) * GU_STEPS + s) * 64 + lane]); }
+            gu_publish(a, ln, t, acc);
+        }
+    };
+    Item x0, x1;
+    bool more = take(x0);
+    while (more) {
+        const bool m1 = take(x1);
+        run(x0);
+        if (!m1) { break; }
+        more = take(x0);
+        run(x1);
+    }
+}
+
 // ---------------------------------------------------------------- phase 4: down units
 // A unit is row group rg (256 output rows) of one pair-slot: wave w owns rows rg * 256 + 32 w .. + 31 (two 16-row sets of
 // one 64-row group). Once its waves have finished their gate/up passes, a workgroup stages the h of all its units at
@@ -804,7 +864,7 @@ __global__ void __launch_bounds__(DNT, 1) k_moe_decode(const DecodeArgs args) {
     // 1. table copy in flight; router (the whole workgroup)
     TRACE(wave, 0);
     if (lds_addr(dyn_lds) & 0xFFFFu) { report(a, 4); return; }   // table addressing needs a 64 KB aligned base
-    if (threadIdx.x < 8) { ctl[threadIdx.x] = 0; }
+    if (threadIdx.x < 16 + DW) { ctl[threadIdx.x] = 0; }
     tables_dma(lds, a.tab, wave);
     __syncthreads();   // the hand-off words are clear
     if (a.prenorm) { norm_phase(a, lds, wave); }
@@ -913,7 +973,10 @@ __global__ void __launch_bounds__(DNT, 1) k_moe_decode(const DecodeArgs args) {
     const int nact = *rt.nact, nps = *rt.nps, ps0 = pre ? n : 0;
     const int t_gu = (nps - ps0) * NGU;
     TRACE(wave, 8);
-    const int ntask = gate_up_stream<GU_PD>(a, lds, ln, blockIdx.x * DW + wave, G * DW, t_gu, false, ps0, P, nact);
+    const int rest = t_gu % (G * DW);
+    const bool tail = rest > 0 && rest <= tail_tasks(n) * G;
+    const int ntask = gate_up_stream<GU_PD>(a, lds, ln, blockIdx.x * DW + wave, G * DW, tail ? t_gu - rest : t_gu, false, ps0, P, nact);
+    if (tail) { gate_up_tail(a, lds, ln, t_gu - rest, t_gu, ps0, P, nact); }
     TRACE(wave, 7);
 
     // 4. down units (pair-slot, 256 rows), round-robin over the workgroups: unit u = row group u / nps of pair-slot u % nps

@@ -833,6 +833,25 @@ def test_decode1_kept_matches_general(ctx, nexp, keep):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("n,keep", [(2, 1), (2, 2), (3, 3), (3, 0), (5, 2), (7, 0), (8, 1), (8, 0)])
+def test_decode_last_round_matches_per_pass(ctx, layer, hot_layer, n, keep):
+    """The n <= 8 block where its gate/up tasks leave a last round of one or two tasks a workgroup, whose waves then share
+    the tasks' steps (and where they do not): several batches, whose distinct experts and pairs differ, and a layer whose
+    rows share experts (two tokens a task), bit for bit against the per-pass kernels."""
+    ctx.set_keep(keep, 2.5)
+    try:
+        for lay in (layer, hot_layer):
+            for i in range(4):
+                x = make_x(ctx, n, seed=7700 + 10 * n + i)
+                y = ctx.moe_layer(lay, x).clone()
+                with ctx.using_fused(0):
+                    y0 = ctx.moe_layer(lay, x).clone()
+                ctx.sync()
+                assert np.array_equal(y.cpu().numpy().view(np.uint32), y0.cpu().numpy().view(np.uint32)), i
+    finally:
+        ctx.set_keep(0)
+
+
 @pytest.mark.parametrize("pattern", ["pairs", "groups", "quads"])
 def test_decode1_selection_ties(ctx, pattern):
     """Exact ties in the selection, made by copying router rows and biases: "pairs" (expert e ^ 1 = e: tied keys
