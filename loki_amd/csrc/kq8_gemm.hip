@@ -12,13 +12,16 @@
 // the stored quants (2 or 3 bits, one per byte) are the selectors into the sub-block's 4 or 8 products, which Q2_K forms by
 // one multiply (sc * {0, 1, 2, 3}) and Q3_K reads from an LDS line per scale ((4 - u) * sc, u = 0..7). That is about 1.6
 // (Q3_K) VALU instructions per weight and 4 MFMAs per 16 x 16 x 256 block, where the fp16 form this replaces took over 2
-// and 16 (its offsets were a second product); it ran the 201-token routed Q3_K down in 678 us.
+// and 16 (its offsets were a second product). The routed Q3_K down at 201 tokens: 678 us in fp16, 485 here with lanes that
+// fetch their own pieces, 331 through coalesced windows, 270 with the ring of three and the next item's first block. What
+// bounds it now is the VALU work of building operands: about 150 instructions a wave and block, four waves a SIMD, against
+// 0.73 GB of weights and mins that pass at 2.7 TB/s.
 //
 // Work: an item is (column of up to 64 slots, 256 rows), one workgroup of 16 waves per CU takes them round-robin; wave w
 // owns one 16-row tile. Lane (r, g), g = 2 n + h, holds of row r the quant bytes 32 n + 16 h .. + 15: the 16-weight
 // sub-blocks 8 n + 2 s + h in its four bit planes s. Product s takes plane s: weights 128 n + 32 s + 16 h .. + 15 of the
 // block, and the activation operand the same positions. The column's Q8_K rows go block by block from memory into
-// XOR-swizzled LDS (direct loads, double-buffered), the next block's weight bytes are in flight while a block computes.
+// XOR-swizzled LDS (direct loads, double-buffered, one block ahead), the weight bytes two blocks ahead.
 #include "kquant_device.h"
 #include "moe_kernels.h"
 #include <type_traits>

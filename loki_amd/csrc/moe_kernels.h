@@ -146,11 +146,14 @@ struct PfTable { int4 * cols; int * ncols; int tok, few, stok; };
 // one or two tables (t1.cols may be null)
 hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, const PfTable & t0, const PfTable & t1, hipStream_t st);
 constexpr int prefill_shared_cols(int n, int tok) { return (n + tok - 1) / tok; }   // the shared expert's columns (the first ones)
-// IQ2_XXS tables by batch size: up to PF_SPLIT_N tokens every column has at most 8 slots (launch_few_gemm alone), up to
-// PF_FEW_N the columns of at most 8 run on the few kernel, above on the narrow one
+// IQ2_XXS tables by batch size: up to PF_SPLIT_N tokens every column has at most 8 slots (launch_few_gemm alone: 100 tokens
+// 610 -> 567 us; at 201 the cut columns read the weights too often), up to PF_FEW_N the columns of at most 8 run on the few
+// kernel, above on the narrow one (at 512 tokens the few kernel beside the others costs more in clocks than it saves in
+// work: 1295 -> 1350 us, an unchanged router 5% slower too)
 constexpr int PF_SPLIT_N = 128, PF_FEW_N = 256;
 constexpr int pf_tok(int n) { return n <= PF_SPLIT_N ? FEW_TOK : PF_TOK; }
-// the K-quant shared expert's columns: enough (column, 128 rows) items of its gate and up for the 256 CUs
+// the K-quant shared expert's columns: enough (column, 128 rows) items of its gate and up for the 256 CUs (at 201 tokens
+// 64-slot columns are 128 items in two launches, 32-slot ones 224 in one)
 constexpr int kq_shared_tok(int n) { return n <= 128 ? 16 : n <= 256 ? 32 : KQ_TOK; }
 constexpr int pf_few(int n) { return n <= PF_FEW_N ? FEW_TOK : 0; }
 

@@ -143,9 +143,15 @@ hipError_t launch_q8_to_h(const int8_t * q, _Float16 * h, int64_t n, hipStream_t
 // ---------------------------------------------------------------- the grouped GEMM
 // NMAT = 2: gate/up (K = 7168, rows 2048, B rows = tokens, writes h); NMAT = 1: down (K = 2048, rows 7168, B rows =
 // slots, writes o). W waves per workgroup, C 16-row tiles per wave, columns of at most 16 NTM slots:
-//   * narrow (W 16, C 2, NTM 2): columns of at most 32 slots, four waves per SIMD;
+//   * narrow (W 16, C 1, NTM 2): columns of at most 32 slots, four waves per SIMD (two tiles a wave spill);
 //   * wide (W 8, C 2, NTM 4): 33..64 slots;
-//   * broad (W 8, C 1, NTM 7): 65..112 slots, the dequantised weights of a tile serve up to seven token tiles.
+//   * broad (W 8, C 1, NTM 7): 65..112 slots, the dequantised weights of a tile serve up to seven token tiles (two row
+//     tiles a wave spill).
+// Bound: a wave's VALU work (72 instructions a tile and block for the digits, 20 a token tile for the fold) and its MFMAs
+// (8 a token tile) share the SIMD's issue, together about 0.73 of their sum. The digits against the fp16 operands they
+// replaced (92 + 16 instructions, twice the LDS bytes), then the registers held over the token tiles: the step at 512 tokens
+// 1295 -> 1208 -> 1150 us, with 16 hot experts of 2048 tokens 3270 -> 3000 -> 2860; with the router's matrix cores and the
+// down's next item ahead 1108 and 2660.
 // With C = 2 a wave's tiles are the gate and up rows of one 16-row tile (gate/up: h forms in registers) or two row tiles
 // (down); with C = 1 the gate waves hand g to the up waves through LDS. Every output is computed once, in the same
 // arithmetic.
