@@ -345,7 +345,7 @@ static void shared_expert(FLCtx * c, Compat * s, const int8_t * xq, const float 
         iq = { s->pcols.p, s->pncols.p, pf_tok(N), pf_few(N), pf_tok(N) };
         kt = { s->pcols.p + prefill_shared_cols(N, FEW_TOK), s->pncols.p + PF_NCOLS, KQ_TOK, 0, kq_shared_tok(N) };
         FCK(launch_prefill_cols(zero_int(c), zero_int(c), zero_int(c), N, 0, iq, kt, c->st));
-        g.ptab = c->ptab.p; g.tab = c->tab.p; g.perm = zero_int(c); g.topk = 1; g.P = 0; g.most = N;
+        g.ptab = c->ptab.p; g.tab = c->tab.p; g.perm = zero_int(c); g.topk = 1; g.P = 0; g.most = N; g.few = iq.few;
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
     }
     ExpertArgs a = expert_args(c, N, 0, 1);
@@ -448,7 +448,7 @@ static void routed_experts(FLCtx * c, Compat * s, const Arena & ar, const int8_t
         FCK(launch_prefill_cols(act, nact, offsets, 0, P, iq, kt, st));
         PrefillArgs g{};
         g.ptab = c->ptab.p; g.tab = c->tab.p; g.w[0] = ar.g; g.w[1] = ar.u; g.estride = mat_bytes(H_, E_); g.sh[0] = ar.g; g.sh[1] = ar.u;   // no shared columns
-        g.perm = perm; g.topk = KE; g.P = P; g.R = H_; g.K = E_; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = P;
+        g.perm = perm; g.topk = KE; g.P = P; g.R = H_; g.K = E_; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = P; g.few = iq.few;
         g.bq = xq; g.bd = xd; g.out = s->h.p; g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
         FCK(iq2_gemm(g, c->ncu, st));
         FCK(launch_quant_q8k(s->h.p, P, H_, s->hq.p, s->hd.p, st));

@@ -657,7 +657,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         g.ptab = c->ptab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
         g.estride = (size_t) H * (E / 256) * IQ2B; g.sh[0] = (const uint8_t *) L->sh_gate; g.sh[1] = (const uint8_t *) L->sh_up;
         g.perm = c->perm.p; g.topk = tk; g.P = P; g.R = H; g.K = E; g.nmat = 2;
-        g.cols = iq.cols; g.ncols = iq.ncols; g.most = n;
+        g.cols = iq.cols; g.ncols = iq.ncols; g.most = n; g.few = iq.few;
         g.bq = c->xq.p; g.tab = c->tab.p; g.bd = c->xd.p; g.out = c->h.p; g.gdbg = c->dbg_gu ? c->g.p : nullptr; g.udbg = c->dbg_gu ? c->u.p : nullptr;
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
         g.col0 = lf[1] == FL_IQ2 ? 0 : nshi;
@@ -709,7 +709,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         PrefillArgs g{};
         g.tab = c->tab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
         g.estride = (size_t) H * (E / 256) * IQ2B; g.sh[0] = (const uint8_t *) L->sh_gate; g.sh[1] = (const uint8_t *) L->sh_up;
-        g.perm = c->perm.p; g.topk = tk; g.P = P; g.R = H; g.K = E; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = n;
+        g.perm = c->perm.p; g.topk = tk; g.P = P; g.R = H; g.K = E; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = n; g.few = iq.few;
         g.bq = c->xq.p; g.bd = c->xd.p; g.out = c->h.p; g.gdbg = c->dbg_gu ? c->g.p : nullptr; g.udbg = c->dbg_gu ? c->u.p : nullptr;
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr; g.col0 = ksh ? nshi : 0;
         TRY(c, launch_few_gemm(g, c->ncu, st));

@@ -161,6 +161,7 @@ constexpr int pf_few(int n) { return n <= PF_FEW_N ? FEW_TOK : 0; }
 struct PrefillArgs {
     const uint4 * ptab;                  // digit table image (build_prefill_tables)
     int most;                            // no expert has more slots than this (classes above it are not launched)
+    int few;                             // the table's few: columns of at most so many slots are the few kernel's (0: none)
     const uint8_t * w[2]; size_t estride;   // routed matrices (tiled), expert e at + e * estride
     const uint8_t * sh[2];               // shared expert matrices (tiled)
     const int * perm; int topk, P;       // gate/up: slot -> token = perm[slot] / topk (shared slots P + t -> t)
