@@ -121,7 +121,7 @@ extern "C" FLCtx * fl_init(int kvp, int sc_cap) {
 
 extern "C" void fl_free(FLCtx * c) {
     if (!c) { return; }
-    (void) hipStreamSynchronize(c->st);
+    (void) hipStreamSynchronize(c->st); (void) hipStreamSynchronize(c->side);
     c->xq.release(); c->hq.release(); c->xd.release(); c->logits.release(); c->probs.release(); c->wts.release();
     c->h.release(); c->hd.release(); c->o.release(); c->g.release(); c->u.release(); c->xn.release();
     c->sel8.release(); c->w8.release();
@@ -203,6 +203,7 @@ extern "C" int fl_set_debug(FLCtx * c, int flags) {
     if (!c) { return FL_EINVAL; }
     c->dbg_gu = (flags & 1) ? 1 : 0;
     c->no_side = (flags & 4) ? 1 : 0;
+    c->dbg_fail = (flags & 8) ? 1 : 0;
     set_grid_ycap((flags & 2) ? 7 : 65535);   // process-wide: the row loops of the combine / scatter kernels at small sizes
     return FL_OK;
 }
@@ -511,6 +512,31 @@ int prefill_ready(FLCtx * c) {
     return FL_OK;
 }
 
+// The second stream's work of one call: forked from the context's stream (what is queued there so far), joined into it by
+// join(), or by the destructor on every return in between: what that stream still reads and writes (x's Q8_K, the shared
+// rows) belongs to the next call on the context's stream, so an error return must not leave it behind.
+struct SideFork {
+    FLCtx * c; bool live = false;
+    explicit SideFork(FLCtx * ctx) : c(ctx) {}
+    SideFork(const SideFork &) = delete;
+    SideFork & operator=(const SideFork &) = delete;
+    hipError_t fork() {
+        hipError_t e = hipEventRecord(c->efork, c->st);
+        if (e == hipSuccess) { e = hipStreamWaitEvent(c->side, c->efork, 0); }
+        live = e == hipSuccess;
+        return e;
+    }
+    hipError_t join() {
+        if (!live) { return hipSuccess; }
+        live = false;
+        hipError_t e = hipEventRecord(c->ejoin, c->side);
+        if (e == hipSuccess) { e = hipStreamWaitEvent(c->st, c->ejoin, 0); }
+        if (e != hipSuccess) { (void) hipStreamSynchronize(c->side); }   // (no event: wait here instead)
+        return e;
+    }
+    ~SideFork() { (void) join(); }
+};
+
 static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, float * y, bool prenorm, const float * nw, float eps,
                      const float * resid) {
     if (!c) { return FL_EINVAL; }
@@ -624,14 +650,16 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     // here on: beside the router, the selection and the dispatch, which leave the chip idle, and then the routed launches (6
     // rows of the real formats 209 -> 195 us against a start beside the routed gate / up). It reads x's Q8_K and writes
     // only its own rows (h / Q8_K(h) rows P .. P + n - 1, o rows P .., ksg / ksu), which no routed kernel touches; the
-    // combine waits for it. Everything that can fail to allocate is allocated before the fork.
+    // combine waits for it, and so does the context's stream when the call fails in between (SideFork). Everything that
+    // can fail to allocate is allocated before the fork.
     const bool ksh = lf[1] != FL_IQ2;
     const bool side = !mfma && ksh && kq && lf[3] != FL_IQ2 && !c->no_side;
+    SideFork beside(c);
     if (side) {
-        TRY(c, hipEventRecord(c->efork, st)); TRY(c, hipStreamWaitEvent(c->side, c->efork, 0));
+        TRY(c, beside.fork());
         if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
         if (int rc = shared_down_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
-        TRY(c, hipEventRecord(c->ejoin, c->side));
+        if (c->dbg_fail) { return fail(c, FL_EHIP, "failure after the second stream's start, asked for by fl_set_debug"); }
     }
     TRY(c, launch_router_logits(L->gate_inp, x, n, ne, E, c->logits.p, rp, st));
     prof_mark(c, ev, 2);
@@ -724,7 +752,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         } else {
             TRY(c, routed_down_kq(c, L, P, E, H, ne));
         }
-        if (side) { TRY(c, hipStreamWaitEvent(st, c->ejoin, 0)); }
+        if (side) { TRY(c, beside.join()); }
         else if (int rc = shared_down_sep(c, L, n, P, E, H, tk, st)) { return rc; }
         TRY(c, launch_combine(c->o.p, c->inv.p, c->wts.p, n, tk, E, P, resid, y, nullptr, st));
         prof_mark(c, ev, 6);
@@ -753,7 +781,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         } else {
             TRY(c, routed_down_kq(c, L, P, E, H, ne));
         }
-        if (side) { TRY(c, hipStreamWaitEvent(st, c->ejoin, 0)); }
+        if (side) { TRY(c, beside.join()); }
         else if (int rc = shared_down_sep(c, L, n, P, E, H, tk, st)) { return rc; }
         TRY(c, launch_combine(c->o.p, c->inv.p, c->wts.p, n, tk, E, P, resid, y, nullptr, st));
         prof_mark(c, ev, 6);

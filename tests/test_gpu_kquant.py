@@ -446,6 +446,55 @@ def test_decode_batch_real_formats(ctx, fm):
     torch.cuda.empty_cache()
 
 
+def test_failed_call_joins_the_second_stream(ctx):
+    """A fl_moe_layer call of 6 rows that fails after the K-quant shared expert's launches are queued on the second stream
+    (fl_set_debug bit 3) leaves them ordered before whatever the context's stream runs next: when fl_sync returns, the shared
+    expert's rows of h and o are those of the same call when it succeeds, and the calls that follow, on other rows, give
+    their own results bit for bit. A 64-expert layer in the real shards' formats."""
+    import torch
+    from loki_amd import LokiError, MoeLayerWeights, lib
+    from tests._helpers import make_x
+    ne, n, fm, seed = 64, 6, DEC_FMTS[0], 8390
+    base = MoeLayerWeights.synthetic(ctx, seed, n_exp=ne, bias_sigma=0.01)
+    down = _kq_device(torch, fm[0], ne * E, H, seed + 1)
+    sh = (_kq_device(torch, fm[1], H, E, seed + 2), _kq_device(torch, fm[2], H, E, seed + 3), _kq_device(torch, fm[3], E, H, seed + 4))
+    layer = MoeLayerWeights(base.gate_inp, base.probs_b, base.gate, base.up, down, *sh, n_exp=ne)
+    xa, xb = make_x(ctx, n, seed=seed + 5), make_x(ctx, n, seed=seed + 6)
+
+    def shared_rows():
+        d = ctx.debug()
+        return (ctx.d2h(d.h + d.P * H * 4, (n, H), np.float32), ctx.d2h(d.o + d.P * E * 4, (n, E), np.float32))
+
+    ctx.set_layer_formats(*fm)
+    try:
+        print("failed call joins the second stream: reference calls", flush=True)
+        ya = ctx.moe_layer(layer, xa).clone()
+        ctx.sync()
+        want = shared_rows()
+        yb = ctx.moe_layer(layer, xb).clone()
+        ctx.sync()
+        for k in range(8):
+            print("failed call joins the second stream: failing call %d" % k, flush=True)
+            ctx.check(lib().fl_set_debug(ctx.ctx, 8))
+            with pytest.raises(LokiError):
+                ctx.moe_layer(layer, xa)
+            ctx.check(lib().fl_set_debug(ctx.ctx, 0))
+            if k % 2:      # the next call at once: its Q8_K(x) goes where the failed call's launches still read
+                got = ctx.moe_layer(layer, xb).clone()
+                assert torch.equal(got.view(torch.int32), yb.view(torch.int32)), k
+            else:
+                ctx.sync()
+                for a, b in zip(shared_rows(), want):
+                    assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), k
+        got = ctx.moe_layer(layer, xa).clone()
+        ctx.sync()
+        assert torch.equal(got.view(torch.int32), ya.view(torch.int32))
+    finally:
+        ctx.check(lib().fl_set_debug(ctx.ctx, 0)); ctx.set_layer_formats()
+    del layer, base, down, sh
+    torch.cuda.empty_cache()
+
+
 # (routed down, shared gate, up, down): the real shards'; a K-quant routed down with the shared expert in IQ2_XXS (GEMM
 # columns); a K-quant shared expert beside an IQ2_XXS routed down (the down GEMM); an IQ2_XXS shared gate/up with a
 # Q6_K shared down (the shared gate/up on the per-pass kernel)
