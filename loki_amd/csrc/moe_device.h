@@ -143,27 +143,7 @@ __device__ __forceinline__ double logit_tree(const double (&s)[4]) {
     t = t + dppd<DPP_MIRROR>(t);
     return (rdlaned(t, 0) + rdlaned(t, 16)) + (rdlaned(t, 32) + rdlaned(t, 48));
 }
-// chunk sums of the lane's 4 chunks of w . x (w, x: the row starts); L4 = K / 1024 float4 per chunk
-template <int L4>
-__device__ __forceinline__ void logit_chunks(const float * w, const float * x, double (&s)[4]) {
-#pragma clang fp contract(off)
-    const int lane = lane_id();
-    const float * wl = w + (size_t) lane * 16 * L4, * xl = x + (size_t) lane * 16 * L4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) { s[j] = 0.0; }
-#pragma unroll
-    for (int i = 0; i < L4; ++i) {
-        float4 wv[4], xv[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { wv[j] = gloadf4(wl + j * 4 * L4 + 4 * i); xv[j] = gloadf4(xl + j * 4 * L4 + 4 * i); }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            s[j] += (double) xv[j].x * (double) wv[j].x; s[j] += (double) xv[j].y * (double) wv[j].y;
-            s[j] += (double) xv[j].z * (double) wv[j].z; s[j] += (double) xv[j].w * (double) wv[j].w;
-        }
-    }
-}
-// the same for any K % 1024 == 0 (runtime chunk length)
+// chunk sums of the lane's 4 chunks of w . x (w, x: the row starts), any K % 1024 == 0
 __device__ __forceinline__ void logit_chunks_any(const float * w, const float * x, int K, double (&s)[4]) {
 #pragma clang fp contract(off)
     const int lane = lane_id(), L = K / 256;

@@ -5,6 +5,7 @@
 #include <stdint.h>
 #include <stddef.h>
 #include "moe_common.h"
+#include "launch_rules.h"
 
 namespace lk {
 
@@ -13,9 +14,7 @@ hipError_t launch_quant_q8k(const float * x, int64_t nrows, int K, int8_t * q, f
 
 // router logits [n][n_exp] under the fp64 chunk contract (K % 256 == 0)
 // part2: fp64 scratch of router_part_doubles(n, n_exp, K) for the matrix-core kernel (k_router_mfma), which then leaves the
-// logits as parts [router_parts][n][n_exp] for launch_router_select to add up, round and write (null or no parts: written
-// here)
-int router_parts(int n, int n_exp, int K);
+// logits as parts [router_parts][n][n_exp] for launch_router_select to add up, round and write (no parts: null, written here)
 size_t router_part_doubles(int n, int n_exp, int K);
 hipError_t launch_router_logits(const float * W, const float * x, int n, int n_exp, int K, float * logits, double * part2, hipStream_t st);
 // sigmoid, bias, grouped top-k, normalised weights; probs [n][n_exp], sel/wts [n][keep]: with 0 < keep < topk each

@@ -17,15 +17,14 @@ namespace lk {
 
 constexpr int RT = 8;   // tokens per router wave
 
-// one wave per (expert, 8-token tile); every token's logit is a full wave reduction (logit_tree)
+// K other than 7168: one wave per (expert, 8-token tile); every token's logit is a full wave reduction (logit_tree)
 __global__ void __launch_bounds__(64) k_router_logits(const float * __restrict__ W, const float * __restrict__ x, int n, int n_exp, int K,
                                                       float * __restrict__ logits) {
     const int e = blockIdx.x, t0 = blockIdx.y * RT;
     const int nt = min(RT, n - t0);
     for (int t = 0; t < nt; ++t) {
         double s[4];
-        if (K == 7168) { logit_chunks<7>(W + (size_t) e * K, x + (size_t) (t0 + t) * K, s); }
-        else { logit_chunks_any(W + (size_t) e * K, x + (size_t) (t0 + t) * K, K, s); }
+        logit_chunks_any(W + (size_t) e * K, x + (size_t) (t0 + t) * K, K, s);
         const double tot = logit_tree(s);
         if (threadIdx.x == 0) { logits[(size_t) (t0 + t) * n_exp + e] = (float) tot; }
     }
@@ -35,7 +34,7 @@ __global__ void __launch_bounds__(64) k_router_logits(const float * __restrict__
 // token and keeps its 28 weights in registers. Per token the chunk sum runs in element order with v_fma_f64 (exact
 // products, one rounding each), tree levels 1-6 are lane butterflies inside the wave (chunks 64 q .. 64 q + 63 of wave
 // q), and levels 7-8 add the four waves' totals as (q0 + q1) + (q2 + q3) through LDS. Four tokens per pass.
-constexpr int RW_MAXN = 16;
+constexpr int RW_MAXN = RM_MIN - 1;
 __device__ __forceinline__ void router_wg_logits(const float * __restrict__ W, const float * __restrict__ x, int n, int n_exp,
                                                  float * __restrict__ logits, double (*part)[4]) {
 #pragma clang fp contract(off)
@@ -278,13 +277,6 @@ __global__ void __launch_bounds__(RM_W * 64, 1) k_router_mfma(const float * __re
     }
 }
 
-// parts of the chunks for n tokens: enough workgroups of a 32 x 32 tile for the CUs (0: the logits are written whole, by
-// k_router_mfma<1> above RM_MAX, which keeps the parts' scratch at 8 MiB)
-constexpr int RM_MIN = 17, RM_MAX = 2048;
-int router_parts(int n, int n_exp, int K) {
-    (void) n_exp;
-    return K != 7168 || n < RM_MIN || n > RM_MAX ? 0 : n <= 128 ? 8 : n <= 256 ? 4 : 2;
-}
 size_t router_part_doubles(int n, int n_exp, int K) { return (size_t) router_parts(n, n_exp, K) * n * n_exp; }
 
 hipError_t launch_router_logits(const float * W, const float * x, int n, int n_exp, int K, float * logits, double * part2, hipStream_t st) {
@@ -300,11 +292,11 @@ hipError_t launch_router_logits(const float * W, const float * x, int n, int n_e
         }
         return hipGetLastError();
     }
-    if (K == 7168 && n > RM_MAX) {
+    if (K == 7168 && n >= RM_MIN) {
         k_router_mfma<1><<<dim3((n_exp + 31) / 32, (n + 31) / 32), RM_W * 64, RM_LDS, st>>>(W, x, n, n_exp, nullptr, logits);
         return hipGetLastError();
     }
-    if (K == 7168 && n <= RW_MAXN) {
+    if (K == 7168) {
         k_router_wg<<<dim3(n_exp), 256, 0, st>>>(W, x, n, n_exp, logits);
         return hipGetLastError();
     }

@@ -67,8 +67,8 @@ def test_pack_layout(ctx):
 
 
 # n covers every logit kernel: the logits and the selection in one launch (n <= 8; 5 gives one wave two tokens), one
-# workgroup per expert (k_router_wg, n < 40), LDS-staged 32 x 32 tiles with the chunks split over 16 workgroups and
-# joined (40..2048) and whole (above 2048: the ragged-expert test), with ragged last tiles
+# workgroup per expert (k_router_wg, up to 20: test_router_parts_bitwise), 32 x 32 tiles on the matrix cores with the
+# chunks split over 8, 4 or 2 workgroups (whole above 512 tiles: the ragged-expert test), with ragged last tiles
 @pytest.mark.parametrize("n,rule", [(1, (8, 4)), (5, (8, 4)), (8, (8, 4)), (21, (8, 4)), (39, (8, 4)), (40, (8, 4)), (77, (8, 4)),
                                     (200, (8, 4)), (300, (8, 4)), (1037, (8, 4)), (8, (1, 1))])
 def test_router_bitwise(ctx, layer, n, rule):
@@ -88,8 +88,8 @@ def test_router_bitwise(ctx, layer, n, rule):
 
 
 # a layer whose expert count is not a multiple of the 32-expert tiles (48 = 8 groups of 6): the last expert tile is
-# ragged in every logit kernel, the K-split tiles (96, 1030) and the whole tiles (2050) included
-@pytest.mark.parametrize("n", [9, 96, 1030, 2050])
+# ragged in every logit kernel, the split tiles (96: 8 parts, 1030: 2) and the whole tiles (8200) included
+@pytest.mark.parametrize("n", [9, 96, 1030, 2050, 8200])
 def test_router_bitwise_ragged_experts(ctx, n):
     import torch
     g = torch.Generator(device="cpu").manual_seed(500 + n)
@@ -959,18 +959,21 @@ def test_few_slot_columns_match_per_pass(ctx, n, hot):
         assert np.array_equal(got[k].view(np.uint8), ref[k].view(np.uint8)), k
 
 
-@pytest.mark.parametrize("n", [9, 16, 31, 32, 33, 128, 129, 256, 257, 2049])
-def test_router_parts_bitwise(ctx, n):
-    """The router on the fp64 matrix cores (from 9 tokens): the edges of its 32-token tiles and of the chunk split (8, 4,
-    2 parts and whole logits), with rows of very different sizes and rows that cancel almost completely. Logits bit for
-    bit the checker's."""
+@pytest.mark.parametrize("n,ne", [(9, 256), (16, 256), (17, 256), (20, 256), (21, 256), (31, 256), (32, 256), (33, 256), (128, 256),
+                                  (129, 256), (256, 256), (257, 256), (2048, 256), (2049, 256), (20, 64), (21, 64), (400, 64), (513, 64),
+                                  (1024, 64), (1025, 64)])
+def test_router_parts_bitwise(ctx, n, ne):
+    """The router's kernels at their edges: one workgroup per expert up to 20 tokens, the fp64 matrix cores from 21 on, at the
+    edges of their 32-token tiles and of the chunk split (8 parts up to 32 tiles, 4 up to 64, 2 up to 512, then whole logits;
+    64 experts reach them at other token counts), with rows of very different sizes and rows that cancel almost completely.
+    Logits bit for bit the checker's."""
     import torch
     rng = np.random.default_rng(n)
-    W = (rng.standard_normal((NEXP, E)) * 0.02).astype(np.float32)
+    W = (rng.standard_normal((ne, E)) * 0.02).astype(np.float32)
     x = (rng.standard_normal((n, E)) * np.exp2(rng.integers(-12, 12, (n, 1)))).astype(np.float32)
     x[0, 1::2] = -x[0, ::2]
     W[::7, 1::2] = W[::7, ::2]
-    b = (rng.standard_normal(NEXP) * 0.05).astype(np.float32)
+    b = (rng.standard_normal(ne) * 0.05).astype(np.float32)
     lg, pr, sel, w = ctx.route(torch.from_numpy(W).cuda(), torch.from_numpy(b).cuda(), torch.from_numpy(x).cuda())
     ctx.sync()
     rows = np.arange(n) if n <= 257 else np.r_[0:64, n - 64:n]
