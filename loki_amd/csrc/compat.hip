@@ -341,22 +341,22 @@ static void shared_expert(FLCtx * c, Compat * s, const int8_t * xq, const float 
         CK(prefill_ready(c) == FL_OK ? hipSuccess : hipErrorOutOfMemory);
         // shared columns only (wide_base runs every row of a wide pass here, so N is not bounded by 64): one table for the
         // IQ2_XXS GEMMs, one for the K-quant GEMM
-        FALLOC(s->pcols, (size_t) prefill_shared_cols(N, FEW_TOK) + prefill_shared_cols(N, 16)); FALLOC(s->pncols, 2 * PF_NCOLS);
-        iq = { s->pcols.p, s->pncols.p, pf_tok(N), pf_few(N), pf_tok(N) };
-        kt = { s->pcols.p + prefill_shared_cols(N, FEW_TOK), s->pncols.p + PF_NCOLS, KQ_TOK, 0, kq_shared_tok(N) };
-        FCK(launch_prefill_cols(zero_int(c), zero_int(c), zero_int(c), N, 0, iq, kt, c->st));
+        iq = iq2_table(nullptr, nullptr, N, 0, 0, N); kt = kq_table(nullptr, nullptr, N);
+        const size_t ni = pf_table_cols(iq, 0);
+        FALLOC(s->pcols, ni + pf_table_cols(kt, 0)); FALLOC(s->pncols, 2 * PF_NCOLS);
+        iq.cols = s->pcols.p; iq.ncols = s->pncols.p; kt.cols = s->pcols.p + ni; kt.ncols = s->pncols.p + PF_NCOLS;
+        FCK(launch_prefill_cols(zero_int(c), zero_int(c), zero_int(c), 0, iq, kt, c->st));
         g.ptab = c->ptab.p; g.tab = c->tab.p; g.perm = zero_int(c); g.topk = 1; g.P = 0; g.most = N; g.few = iq.few;
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
     }
     ExpertArgs a = expert_args(c, N, 0, 1);
-    const auto iq2_gemm = iq.tok == FEW_TOK ? launch_few_gemm : launch_prefill_gemm;
     if (gu_gemm) {
         PrefillArgs k = g;
         k.R = H_; k.K = E_; k.bq = xq; k.bd = xd;
         if (s->shf[0] == FL_IQ2) {
             k.cols = iq.cols; k.ncols = iq.ncols;
             k.w[0] = tm[0]; k.w[1] = tm[1]; k.sh[0] = tm[0]; k.sh[1] = tm[1]; k.nmat = 2; k.out = s->h.p;
-            FCK(iq2_gemm(k, c->ncu, c->st));
+            FCK(launch_prefill_gemm(k, c->ncu, c->st));
         } else {
             FALLOC(s->xh, (size_t) N * E_);
             FCK(launch_q8_to_h(xq, s->xh.p, (int64_t) N * E_, c->st));
@@ -392,7 +392,7 @@ static void shared_expert(FLCtx * c, Compat * s, const int8_t * xq, const float 
         k.R = E_; k.K = H_; k.nmat = 1; k.bq = s->hq.p; k.bd = s->hd.p; k.out = out;
         if (s->shf[2] == FL_IQ2) {
             k.w[0] = k.sh[0] = tm[2]; k.cols = iq.cols; k.ncols = iq.ncols;
-            FCK(iq2_gemm(k, c->ncu, c->st));
+            FCK(launch_prefill_gemm(k, c->ncu, c->st));
         } else {
             if (s->shf[2] == FL_Q6K) { FALLOC(s->hh, (size_t) N * H_); FCK(launch_q8_to_h(s->hq.p, s->hh.p, (int64_t) N * H_, c->st)); }
             k.cols = kt.cols; k.ncols = kt.ncols; k.bh = s->hh.p;
@@ -440,23 +440,22 @@ static void routed_experts(FLCtx * c, Compat * s, const Arena & ar, const int8_t
     if (c->pf_mfma && P >= 32 && P >= 2 * nexp) {
         CK(prefill_ready(c) == FL_OK ? hipSuccess : hipErrorOutOfMemory);
         hipStream_t st = c->st;
-        const size_t nc = (size_t) P / pf_tok(n) + NEXP_MAX + 4;   // entries of the first table
-        FALLOC(s->pcols, nc + (size_t) P / KQ_TOK + NEXP_MAX + 4); FALLOC(s->pncols, 2 * PF_NCOLS);
-        const PfTable iq = { s->pcols.p, s->pncols.p, pf_tok(n), pf_few(n), pf_tok(n) };
-        const PfTable kt = { down_fmt == FL_IQ2 ? nullptr : s->pcols.p + nc, s->pncols.p + PF_NCOLS, KQ_TOK, 0, KQ_TOK };
-        const auto iq2_gemm = iq.tok == FEW_TOK ? launch_few_gemm : launch_prefill_gemm;
-        FCK(launch_prefill_cols(act, nact, offsets, 0, P, iq, kt, st));
+        PfTable iq = iq2_table(nullptr, nullptr, 0, P, nexp, max_slots), kt = kq_table(nullptr, nullptr, 0);
+        const size_t ni = pf_table_cols(iq, P);
+        FALLOC(s->pcols, ni + pf_table_cols(kt, P)); FALLOC(s->pncols, 2 * PF_NCOLS);
+        iq.cols = s->pcols.p; iq.ncols = s->pncols.p; kt.cols = down_fmt == FL_IQ2 ? nullptr : s->pcols.p + ni; kt.ncols = s->pncols.p + PF_NCOLS;
+        FCK(launch_prefill_cols(act, nact, offsets, P, iq, kt, st));
         PrefillArgs g{};
         g.ptab = c->ptab.p; g.tab = c->tab.p; g.w[0] = ar.g; g.w[1] = ar.u; g.estride = mat_bytes(H_, E_); g.sh[0] = ar.g; g.sh[1] = ar.u;   // no shared columns
-        g.perm = perm; g.topk = KE; g.P = P; g.R = H_; g.K = E_; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = P; g.few = iq.few;
+        g.perm = perm; g.topk = KE; g.P = P; g.R = H_; g.K = E_; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = max_slots; g.few = iq.few;
         g.bq = xq; g.bd = xd; g.out = s->h.p; g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
-        FCK(iq2_gemm(g, c->ncu, st));
+        FCK(launch_prefill_gemm(g, c->ncu, st));
         FCK(launch_quant_q8k(s->h.p, P, H_, s->hq.p, s->hd.p, st));
         PrefillArgs d = g;
         d.R = E_; d.K = H_; d.nmat = 1; d.bq = s->hq.p; d.bd = s->hd.p; d.out = o; d.w[1] = nullptr; d.sh[1] = nullptr;
         if (down_fmt == FL_IQ2) {
             d.w[0] = ar.d; d.sh[0] = ar.d; d.estride = mat_bytes(E_, H_);
-            FCK(iq2_gemm(d, c->ncu, st));
+            FCK(launch_prefill_gemm(d, c->ncu, st));
         } else {   // src/fused_layer.cu:607-608 (tc_matvec<F_Q2K / F_Q3K>)
             d.w[0] = (const uint8_t *) down; d.sh[0] = (const uint8_t *) down; d.estride = fmt_bytes(down_fmt, E_, H_);
             d.cols = kt.cols; d.ncols = kt.ncols;

@@ -588,6 +588,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     // more launches (the columns, Q8_K of h), so from 16 slots: 2 rows of 8 picks 98.8 -> 95.8 us, 6 rows 195 -> 164, 8 rows
     // 238 -> 202, 8 rows of 2 picks 109 -> 99; at 6 slots (3 rows of 2) 75.4 -> 77.6
     const bool few = !fused && !mfma && kq && c->pf_mfma && P >= 16 && E == 7168 && H == 2048;
+    const int nsi = lf[1] == FL_IQ2 || lf[3] == FL_IQ2 ? n : 0;   // the shared expert's slots in the IQ2_XXS column table
     const bool q5 = lf[1] == FL_Q5K && lf[2] == FL_Q5K, q6 = lf[3] == FL_Q6K;   // shared matrices on fp16 activations
     ALLOC(c, c->xq, (size_t) n * E); ALLOC(c, c->xd, (size_t) n * (E / 256));
     ALLOC(c, c->logits, (size_t) n * ne); ALLOC(c, c->probs, (size_t) n * ne);
@@ -622,15 +623,15 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     }
     if (mfma) {
         if (int rc = prefill_ready(c)) { return rc; }
-        ALLOC(c, c->pcols, rows / pf_tok(n) + NEXP_MAX + 4); ALLOC(c, c->pncols, 2 * PF_NCOLS);
-        if (kq) { ALLOC(c, c->pcolsk, P / KQ_TOK + n / 16 + NEXP_MAX + 4); }
+        ALLOC(c, c->pcols, pf_table_cols(iq2_table(nullptr, nullptr, nsi, P, ne, n), P)); ALLOC(c, c->pncols, 2 * PF_NCOLS);
+        if (kq) { ALLOC(c, c->pcolsk, pf_table_cols(kq_table(nullptr, nullptr, n), P)); }
         if (q5) { ALLOC(c, c->xh, (size_t) n * E); }
         if (q6) { ALLOC(c, c->hh, (size_t) n * H); }
     }
     if (!mfma && lf[1] != FL_IQ2) { ALLOC(c, c->ksg, (size_t) n * H); ALLOC(c, c->ksu, (size_t) n * H); }
     if (few) {
         if (int rc = prefill_ready(c)) { return rc; }
-        ALLOC(c, c->pcols, rows / pf_tok(n) + NEXP_MAX + 4); ALLOC(c, c->pncols, 2 * PF_NCOLS);
+        ALLOC(c, c->pcols, pf_table_cols(iq2_table(nullptr, nullptr, nsi, P, ne, n), P)); ALLOC(c, c->pncols, PF_NCOLS);
     }
     double * rp = nullptr;   // the matrix-core router's parts
     if (const size_t nd = router_part_doubles(n, ne, E)) { ALLOC(c, c->rpart, nd); rp = c->rpart.p; }
@@ -672,15 +673,13 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     prof_mark(c, ev, 3);
     TRY(c, launch_dispatch(c->sel.p, P, ne, c->counts.p, c->offsets.p, c->perm.p, c->inv.p, c->act.p, c->nact.p, st, dsc));
     if (mfma) {
-        const PfTable iq = { c->pcols.p, c->pncols.p, pf_tok(n), pf_few(n), pf_tok(n) };
-        const PfTable kt = { kq ? c->pcolsk.p : nullptr, c->pncols.p + PF_NCOLS, KQ_TOK, 0, kq_shared_tok(n) };
-        TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, n, P, iq, kt, st));
+        const PfTable iq = iq2_table(c->pcols.p, c->pncols.p, nsi, P, ne, n), kt = kq_table(kq ? c->pcolsk.p : nullptr, c->pncols.p + PF_NCOLS, n);
+        TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, P, iq, kt, st));
         prof_mark(c, ev, 4);
-        // Columns: the shared expert's first (nsh of them), then the routed experts'. Each matrix runs where its format
+        // Columns: the shared expert's first, then the routed experts'. Each matrix runs where its format
         // does: IQ2_XXS on the IQ2_XXS GEMM, Q2_K / Q3_K / Q6_K downs and a Q5_K shared gate / up on the K-quant GEMM,
         // any other K-quant on the mat-vecs.
-        const int nsh = prefill_shared_cols(n, kt.stok), nshi = prefill_shared_cols(n, iq.tok);   // K-quant, IQ2_XXS tables
-        const auto iq2_gemm = iq.tok == FEW_TOK ? launch_few_gemm : launch_prefill_gemm;
+        const int nsh = prefill_shared_cols(n, kt.stok);   // of the K-quant table
         PrefillArgs g{};
         g.ptab = c->ptab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
         g.estride = (size_t) H * (E / 256) * IQ2B; g.sh[0] = (const uint8_t *) L->sh_gate; g.sh[1] = (const uint8_t *) L->sh_up;
@@ -688,8 +687,8 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         g.cols = iq.cols; g.ncols = iq.ncols; g.most = n; g.few = iq.few;
         g.bq = c->xq.p; g.tab = c->tab.p; g.bd = c->xd.p; g.out = c->h.p; g.gdbg = c->dbg_gu ? c->g.p : nullptr; g.udbg = c->dbg_gu ? c->u.p : nullptr;
         g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr;
-        g.col0 = lf[1] == FL_IQ2 ? 0 : nshi;
-        TRY(c, iq2_gemm(g, c->ncu, st));
+        g.part = lf[1] == FL_IQ2 ? PF_ALL : PF_ROUTED;
+        TRY(c, launch_prefill_gemm(g, c->ncu, st));
         if (q5) {   // the real shards' shared gate / up: ksg / ksu rows 0 .. n - 1
             ALLOC(c, c->ksg, (size_t) n * H); ALLOC(c, c->ksu, (size_t) n * H);
             PrefillArgs k{};
@@ -709,13 +708,13 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         d.R = E; d.K = H; d.nmat = 1; d.bq = c->hq.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr;
         const bool sh_iq = lf[3] == FL_IQ2, sh_kg = lf[3] == FL_Q2K || lf[3] == FL_Q3K || lf[3] == FL_Q6K;
         if (lf[0] == FL_IQ2) {   // routed (+ the shared expert when it is IQ2_XXS)
-            d.col0 = sh_iq ? 0 : nshi;
-            TRY(c, iq2_gemm(d, c->ncu, st));
+            d.part = sh_iq ? PF_ALL : PF_ROUTED;
+            TRY(c, launch_prefill_gemm(d, c->ncu, st));
         } else {
             PrefillArgs k = d;
             k.estride = fmt_mat_bytes(lf[0], E, H); k.cols = kt.cols; k.ncols = kt.ncols; k.col0 = nsh;
             TRY(c, launch_kq_gemm(k, lf[0], c->ncu, st));
-            if (sh_iq) { d.col0 = 0; d.col1 = nshi; TRY(c, iq2_gemm(d, c->ncu, st)); }
+            if (sh_iq) { d.part = PF_SHARED; TRY(c, launch_prefill_gemm(d, c->ncu, st)); }
         }
         if (sh_kg) {
             PrefillArgs k = d;
@@ -730,25 +729,24 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         return FL_OK;
     }
     if (few) {
-        const PfTable iq = { c->pcols.p, c->pncols.p, pf_tok(n), pf_few(n), pf_tok(n) };
-        TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, n, P, iq, PfTable{}, st));
+        const PfTable iq = iq2_table(c->pcols.p, c->pncols.p, nsi, P, ne, n);   // (at most 8 slots an expert: few columns only)
+        TRY(c, launch_prefill_cols(c->act.p, c->nact.p, c->offsets.p, P, iq, PfTable{}, st));
         prof_mark(c, ev, 4);
-        const int nshi = prefill_shared_cols(n, iq.tok);
         PrefillArgs g{};
-        g.tab = c->tab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
+        g.ptab = c->ptab.p; g.tab = c->tab.p; g.w[0] = (const uint8_t *) L->gate_exps; g.w[1] = (const uint8_t *) L->up_exps;
         g.estride = (size_t) H * (E / 256) * IQ2B; g.sh[0] = (const uint8_t *) L->sh_gate; g.sh[1] = (const uint8_t *) L->sh_up;
         g.perm = c->perm.p; g.topk = tk; g.P = P; g.R = H; g.K = E; g.nmat = 2; g.cols = iq.cols; g.ncols = iq.ncols; g.most = n; g.few = iq.few;
         g.bq = c->xq.p; g.bd = c->xd.p; g.out = c->h.p; g.gdbg = c->dbg_gu ? c->g.p : nullptr; g.udbg = c->dbg_gu ? c->u.p : nullptr;
-        g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr; g.col0 = ksh ? nshi : 0;
-        TRY(c, launch_few_gemm(g, c->ncu, st));
+        g.err = c->derr.p; g.herr = c->herr ? c->herr_dev : nullptr; g.part = ksh ? PF_ROUTED : PF_ALL;
+        TRY(c, launch_prefill_gemm(g, c->ncu, st));
         if (ksh && !side) { if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, st)) { return rc; } }
         TRY(c, launch_quant_q8k(c->h.p, (int64_t) (ksh ? P : P + n), H, c->hq.p, c->hd.p, st));   // (a K-quant shared expert's rows: shared_swiglu)
         prof_mark(c, ev, 5);
         if (lf[0] == FL_IQ2) {
             PrefillArgs d = g;
             d.w[0] = (const uint8_t *) L->down_exps; d.w[1] = nullptr; d.sh[0] = (const uint8_t *) L->sh_down; d.sh[1] = nullptr;
-            d.R = E; d.K = H; d.nmat = 1; d.bq = c->hq.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr; d.col0 = nshi;
-            TRY(c, launch_few_gemm(d, c->ncu, st));
+            d.R = E; d.K = H; d.nmat = 1; d.bq = c->hq.p; d.bd = c->hd.p; d.out = c->o.p; d.gdbg = nullptr; d.udbg = nullptr; d.part = PF_ROUTED;
+            TRY(c, launch_prefill_gemm(d, c->ncu, st));
         } else {
             TRY(c, routed_down_kq(c, L, P, E, H, ne));
         }

@@ -1,4 +1,4 @@
-// moe_few.hip -- the grouped IQ2_XXS x Q8_K expert products for columns of few slots (at most FEW_TOK = 8 tokens of one
+// moe_few.h -- the grouped IQ2_XXS x Q8_K expert products for columns of few slots (at most FEW_TOK = 8 tokens of one
 // expert) on the int8 matrix cores.
 //
 // Reference: fl_wide_moe's tc_matvec<F_IQ2> (src/fused_layer.cu:178-202, 540-561); the arithmetic is that of
@@ -23,6 +23,7 @@
 //   * A wave works alone: an item is (column, 16 h rows of gate and up / 32 down rows) over the whole K, its tokens' Q8_K
 //     copied block by block into the wave's own two LDS buffers (one 1 KB direct load per set), its weights two blocks
 //     ahead in registers. No workgroup barrier after the tables are in LDS.
+#pragma once
 #include "moe_device.h"
 #include "moe_kernels.h"
 #include <type_traits>
@@ -38,22 +39,35 @@ constexpr int F_BUF = FEW_TOK * QK;                   // one activation buffer o
 constexpr int F_LDS = TAB_BYTES + FW * 2 * F_BUF;
 static_assert(F_LDS <= 160 * 1024 && TAB_BYTES % (2 * F_BUF) == 0, "LDS budget; buffers toggled by one address bit");
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t few_rsrc(const void * p) {
+// raw buffer resource over p (gfx9 word 3; the record count only bounds offsets, which stay far below it)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t pf_rsrc(const void * p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short) 0, 0x7fffffff, 0x00020000);
 }
-__device__ __forceinline__ const uint8_t * few_uniform(const uint8_t * p) {
+// a wave-uniform pointer kept in scalar registers
+__device__ __forceinline__ const uint8_t * pf_uniform(const uint8_t * p) {
     const uint64_t v = (uint64_t) p;
     const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (v >> 32));
     const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) v);
     return (const uint8_t *) (((uint64_t) hi << 32) | (uint64_t) lo);
 }
-// 16 bytes per lane from a buffer straight into LDS (lane L at dst + 16 L); the builtin exists for the device pass only
-__device__ __forceinline__ void few_lds16(__amdgpu_buffer_rsrc_t r, LK_LOCAL uint8_t * dst, uint32_t voff, uint32_t soff) {
+// SZ bytes per lane from a buffer straight into LDS (lane L at dst + SZ L); the builtin exists for the device pass only,
+// so the host pass (which instantiates the kernels' launch stubs) sees an empty body
+template <int SZ> __device__ __forceinline__ void buf_lds(__amdgpu_buffer_rsrc_t r, LK_LOCAL uint8_t * dst, uint32_t voff, uint32_t soff) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 16, voff, soff, 0, 0);
+    if constexpr (SZ == 16) { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 16, voff, soff, 0, 0); }
+    else { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 4, voff, soff, 0, 0); }
 #else
     (void) r; (void) dst; (void) voff; (void) soff;
 #endif
+}
+// the tables' addressing needs a 64 KB aligned LDS base: false (and the error reported) without one
+__device__ __forceinline__ bool pf_base_ok(const PrefillArgs & a, uint32_t base) {
+    if (!(base & 0xFFFFu)) { return true; }
+    if (threadIdx.x == 0) {
+        __hip_atomic_fetch_or(gptr(a.err), 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a.herr) { __hip_atomic_store(gptr(a.herr), 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+    }
+    return false;
 }
 // vmcnt(N), nothing moved across it
 template <int N> __device__ __forceinline__ void few_wait() {
@@ -78,33 +92,25 @@ __device__ __forceinline__ int few_add16(int a, int b) {
 
 struct FewW { u32x4 q; uint16_t d; };
 
-}  // namespace
-
+// the columns of class PF_FEW (those of the table's part, pf_runs) on the workgroup's 16 waves
 template <int NMAT, int NB>
-__global__ void __launch_bounds__(FNT, 1) k_few_gemm(const PrefillArgs a) {
+__device__ __forceinline__ void few_body(const PrefillArgs & a, LK_LOCAL uint8_t * lds) {
 #pragma clang fp contract(off)
     constexpr int K = NB * QK, C = 2;   // the wave's two 16-row tiles: gate and up of the same h rows, or 32 down rows
-    extern __shared__ __attribute__((aligned(16))) uint8_t few_lds[];
-    LK_LOCAL uint8_t * lds = (LK_LOCAL uint8_t *) few_lds;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+    const uint32_t base = (uint32_t) (size_t) lds;
     const PfRuns runs = pf_runs(a, PF_FEW);
     const int nt = a.R / (NMAT == 2 ? 16 : 32), items = runs.count() * nt;
     if ((int) blockIdx.x * 4 >= items) { return; }
-    if (lds_addr(few_lds) & 0xFFFFu) {   // table addressing needs a 64 KB aligned base
-        if (threadIdx.x == 0) {
-            __hip_atomic_fetch_or(gptr(a.err), 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (a.herr) { __hip_atomic_store(gptr(a.herr), 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
-        }
-        return;
-    }
+    if (!pf_base_ok(a, base)) { return; }
     tables_fill(reinterpret_cast<const uint8_t *>(a.tab), lds, threadIdx.x, FNT);
     const int r = lane & 15, g = lane >> 4, q = lane & 3;
-    const uint32_t tr = tab_word_grid(lds_addr(few_lds), lane), trs = tab_sign_word(tr);
+    const uint32_t tr = tab_word_grid(base, lane), trs = tab_sign_word(tr);
     // the activation operand's LDS address at MFMA m: lanes whose row's chunk ((lane >> 2) & 3) is their K slice g read
     // token q's bytes 64 g + 16 m of the block (slot (4 g + m) ^ q of the token's row: the 16 such lanes hit 16 bank
     // quads), the others 16 zero bytes (the sign entry of no negative weight)
     const bool diag = ((lane >> 2) & 3) == g;
-    const uint32_t xbase = lds_addr(few_lds) + (uint32_t) (TAB_BYTES + wave * 2 * F_BUF);
+    const uint32_t xbase = base + (uint32_t) (TAB_BYTES + wave * 2 * F_BUF);
     const uint32_t xa = diag ? xbase + (uint32_t) (q * QK) + ((uint32_t) (4 * g + q) << 4) : trs;
     const uint32_t tog = diag ? (uint32_t) F_BUF : 0u, set1 = diag ? 4u * QK : 0u;
     const int tk = ((g & 1) << 1) | (g >> 1);   // the token of a set whose sums end in this lane
@@ -122,7 +128,7 @@ __global__ void __launch_bounds__(FNT, 1) k_few_gemm(const PrefillArgs a) {
             const int s = sb + (t < sc ? t : 0);
             return NMAT == 2 ? (routed ? gptr(a.perm)[s] / a.topk : s - a.P) : s;
         };
-        const __amdgpu_buffer_rsrc_t rb = few_rsrc(a.bq), rd = few_rsrc(a.bd);
+        const __amdgpu_buffer_rsrc_t rb = pf_rsrc(a.bq), rd = pf_rsrc(a.bd);
         const size_t dreg = (size_t) (a.R / 64) * NB * 4096;   // d region offset of a tiled matrix
         __amdgpu_buffer_rsrc_t uq[C], ud[C];
 #pragma unroll
@@ -130,8 +136,8 @@ __global__ void __launch_bounds__(FNT, 1) k_few_gemm(const PrefillArgs a) {
             const int mat = NMAT == 2 ? c : 0, row0 = NMAT == 2 ? ti * 16 : ti * 32 + c * 16;
             const uint8_t * Wm = routed ? a.w[mat] + (size_t) ex * a.estride : a.sh[mat];
             const int g64 = row0 >> 6, r0 = row0 & 63;
-            uq[c] = few_rsrc(few_uniform(Wm + (size_t) g64 * NB * 4096 + r0 * 16));
-            ud[c] = few_rsrc(few_uniform(Wm + dreg + (size_t) g64 * NB * 128 + r0 * 2));
+            uq[c] = pf_rsrc(pf_uniform(Wm + (size_t) g64 * NB * 4096 + r0 * 16));
+            ud[c] = pf_rsrc(pf_uniform(Wm + dreg + (size_t) g64 * NB * 128 + r0 * 2));
         }
         const uint32_t lq = (uint32_t) g * 1024 + (uint32_t) r * 16, ldo = (uint32_t) r * 2;
         auto load_w = [&](int j, FewW (&w)[C]) {
@@ -153,7 +159,7 @@ __global__ void __launch_bounds__(FNT, 1) k_few_gemm(const PrefillArgs a) {
             auto load_x = [&](int j, int buf, float (&dx)[S]) {
                 LK_LOCAL uint8_t * dst = lds + TAB_BYTES + wave * 2 * F_BUF + buf * F_BUF;
 #pragma unroll
-                for (int s = 0; s < S; ++s) { few_lds16(rb, dst + s * 1024, ob[s], j * QK); }
+                for (int s = 0; s < S; ++s) { buf_lds<16>(rb, dst + s * 1024, ob[s], j * QK); }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int s = 0; s < S; ++s) { dx[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, ox[s], j * 4, 0)); }
@@ -289,23 +295,6 @@ __global__ void __launch_bounds__(FNT, 1) k_few_gemm(const PrefillArgs a) {
     }
 }
 
-template <int NMAT, int NB> static hipError_t few_setup() {
-    return hipFuncSetAttribute((const void *) k_few_gemm<NMAT, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, F_LDS);
-}
-hipError_t few_init() {
-    const hipError_t e = few_setup<2, 28>();
-    return e == hipSuccess ? few_setup<1, 8>() : e;
-}
-hipError_t launch_few_gemm(const PrefillArgs & a, int grid, hipStream_t st) {
-    if (grid < 1 || !a.tab || !a.cols || !a.ncols || !a.bq || !a.bd || !a.out || !a.err || a.R % 64) { return hipErrorInvalidValue; }
-    if (a.nmat == 2) {
-        if (a.K != 28 * QK || !a.w[0] || !a.w[1] || !a.sh[0] || !a.sh[1] || !a.perm) { return hipErrorInvalidValue; }
-        k_few_gemm<2, 28><<<grid, FNT, F_LDS, st>>>(a);
-    } else {
-        if (a.nmat != 1 || a.K != 8 * QK || !a.w[0] || !a.sh[0]) { return hipErrorInvalidValue; }
-        k_few_gemm<1, 8><<<grid, FNT, F_LDS, st>>>(a);
-    }
-    return hipGetLastError();
-}
+}  // namespace
 
 }  // namespace lk

@@ -136,31 +136,34 @@ hipError_t launch_moe_decode1(const DecodeArgs & a, bool cooperative, hipStream_
 
 // Column tables. launch_prefill_cols cuts every expert's slots (the shared expert's first) into columns of at most tok
 // slots (the shared expert's stok), the fewest possible and of equal size (rounded up to 16); the routed columns are ordered
-// by class. Sized >= P / tok + n / stok + NEXP_MAX + 2 entries. Classes by slots: broad 65..112, wide 33..64, narrow few + 1..32, few 1..few.
+// by class. few > 0 (a split table, IQ2_XXS): experts of at most few slots get one column of the few kernel, and where that
+// costs less the others' columns are cut at few slots too (k_pf_cols). Sized pf_table_cols(). Classes by slots: broad
+// 65..112, wide 33..64, narrow few + 1..32, few 1..few.
 // ncols[0] all columns; [1 + k] end of the shared columns of class k; [PF_NCLS + 1 + k] end of the routed ones.
-constexpr int PF_TOK = 112, KQ_TOK = 64, FEW_TOK = 8;   // tok of the IQ2_XXS GEMMs, the K-quant GEMM, the few kernel
 enum { PF_BROAD = 0, PF_WIDE = 1, PF_NARROW = 2, PF_FEW = 3, PF_NCLS = 4 };
 constexpr int PF_NCOLS = 2 * PF_NCLS + 1;
-struct PfTable { int4 * cols; int * ncols; int tok, few, stok; };
+struct PfTable { int4 * cols; int * ncols; int tok, few, stok, n; };   // n: the shared expert's slots (0: not in this table)
+// the IQ2_XXS table of n shared and P routed slots of n_exp experts, none with more than most (launch_rules.h), and the
+// K-quant one
+constexpr PfTable iq2_table(int4 * cols, int * ncols, int n, int P, int n_exp, int most) {
+    return most <= FEW_TOK ? PfTable { cols, ncols, FEW_TOK, FEW_TOK, FEW_TOK, n } : pf_split(n, P, n_exp) ? PfTable { cols, ncols, SPLIT_TOK, FEW_TOK, split_shared_tok(n, P), n } : PfTable { cols, ncols, PF_TOK, 0, PF_TOK, n };
+}
+constexpr PfTable kq_table(int4 * cols, int * ncols, int n) { return PfTable { cols, ncols, KQ_TOK, 0, kq_shared_tok(n), n }; }
+constexpr size_t pf_table_cols(const PfTable & t, int P) {   // its entries for P routed slots
+    const int lo = t.few > 0 ? t.few : t.tok, slo = t.few > 0 ? t.few : t.stok;
+    return (size_t) P / lo + (size_t) t.n / slo + NEXP_MAX + 4;
+}
 // one or two tables (t1.cols may be null)
-hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, const PfTable & t0, const PfTable & t1, hipStream_t st);
-constexpr int prefill_shared_cols(int n, int tok) { return (n + tok - 1) / tok; }   // the shared expert's columns (the first ones)
-// IQ2_XXS tables by batch size: up to PF_SPLIT_N tokens every column has at most 8 slots (launch_few_gemm alone: 100 tokens
-// 610 -> 567 us; at 201 the cut columns read the weights too often), up to PF_FEW_N the columns of at most 8 run on the few
-// kernel, above on the narrow one (at 512 tokens the few kernel beside the others costs more in clocks than it saves in
-// work: 1295 -> 1350 us, an unchanged router 5% slower too)
-constexpr int PF_SPLIT_N = 128, PF_FEW_N = 256;
-constexpr int pf_tok(int n) { return n <= PF_SPLIT_N ? FEW_TOK : PF_TOK; }
-// the K-quant shared expert's columns: enough (column, 128 rows) items of its gate and up for the 256 CUs (at 201 tokens
-// 64-slot columns are 128 items in two launches, 32-slot ones 224 in one)
-constexpr int kq_shared_tok(int n) { return n <= 128 ? 16 : n <= 256 ? 32 : KQ_TOK; }
-constexpr int pf_few(int n) { return n <= PF_FEW_N ? FEW_TOK : 0; }
+hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int P, const PfTable & t0, const PfTable & t1, hipStream_t st);
+constexpr int prefill_shared_cols(int n, int tok) { return (n + tok - 1) / tok; }   // the shared expert's columns of a table that is not split (the first ones)
 
 // ---------------------------------------------------------------- prefill grouped GEMM on MFMA (moe_prefill.hip)
+enum { PF_ALL = 0, PF_ROUTED = 1, PF_SHARED = 2 };
 struct PrefillArgs {
     const uint4 * ptab;                  // digit table image (build_prefill_tables)
     int most;                            // no expert has more slots than this (classes above it are not launched)
-    int few;                             // the table's few: columns of at most so many slots are the few kernel's (0: none)
+    int few;                             // the table's few (0: not split)
+    int part;                            // the table's columns to run: PF_ALL, PF_ROUTED or PF_SHARED (launch_prefill_gemm)
     const uint8_t * w[2]; size_t estride;   // routed matrices (tiled), expert e at + e * estride
     const uint8_t * sh[2];               // shared expert matrices (tiled)
     const int * perm; int topk, P;       // gate/up: slot -> token = perm[slot] / topk (shared slots P + t -> t)
@@ -168,47 +171,39 @@ struct PrefillArgs {
     const int4 * cols; const int * ncols;   // launch_prefill_cols
     const int8_t * bq; const float * bd; // activations: Q8_K integers [rows][K] and scales [rows][K/256]
     const _Float16 * bh;                 // the integers as fp16 (launch_kq_gemm's Q5_K and Q6_K)
-    const uint4 * tab;                   // the decode table image (build_table_image), for that kernel
+    const uint4 * tab;                   // the decode table image (build_table_image), for the few kernel
     float * out;                         // gate/up: h [P+n][R] (silu(g) * u); down: o [P+n][R]
     float * gdbg, * udbg;                // optional gate / up outputs
     int * err;                           // bit 4: the LDS base is not 64 KB aligned
     int * herr;                          // host-mapped copy of the code (may be null)
-    // the columns col0 .. col1 - 1 of launch_prefill_cols (col1 <= 0: to the last); the shared expert's come first,
-    // ceil(n / 64) of them
+    // launch_kq_gemm: the columns col0 .. col1 - 1 of the table (col1 <= 0: to the last); the shared expert's come first,
+    // prefill_shared_cols(n, stok) of them
     int col0, col1;
     // launch_kq_gemm with Q5_K: udbg != null: the output of a second matrix sh[1] of the shared expert, in the same launch
     // launch_kq_gemm: activation row = slot - arow0, output row = slot - orow0 (the shared expert's gate / up
     // read the tokens' rows and write rows 0 .. n - 1 of their own outputs)
     int arow0, orow0;
 };
-// the columns of one class inside [col0, col1): two runs [a0, a0 + na) and [b0, b0 + nb) of the column table
+// the columns of one class: the shared expert's [a0, a0 + na) and the routed ones [b0, b0 + nb) of the column table, those of
+// the part asked for
 struct PfRuns {
     int a0, na, b0, nb;
     __device__ int count() const { return na + nb; }
     __device__ int col(int j) const { return j < na ? a0 + j : b0 + (j - na); }
 };
-__device__ __forceinline__ int pf_clip(int lo, int hi, int c0, int c1, int & start) {
-    start = lo > c0 ? lo : c0;
-    const int end = hi < c1 ? hi : c1;
-    return end > start ? end - start : 0;
-}
 __device__ __forceinline__ PfRuns pf_runs(const PrefillArgs & a, int cls) {
     const LK_GLOBAL int * nc = gptr(a.ncols);
-    const int c0 = a.col0, c1 = a.col1 > 0 ? a.col1 : nc[0];
     PfRuns r;
-    r.na = pf_clip(cls == 0 ? 0 : nc[cls], nc[1 + cls], c0, c1, r.a0);
-    r.nb = pf_clip(nc[PF_NCLS + cls], nc[PF_NCLS + 1 + cls], c0, c1, r.b0);
+    r.a0 = cls == 0 ? 0 : nc[cls]; r.na = a.part == PF_ROUTED ? 0 : nc[1 + cls] - r.a0;
+    r.b0 = nc[PF_NCLS + cls]; r.nb = a.part == PF_SHARED ? 0 : nc[PF_NCLS + 1 + cls] - r.b0;
     return r;
 }
 hipError_t prefill_init();
 size_t prefill_table_bytes();
 hipError_t build_prefill_tables(uint4 * img, hipStream_t st);
 hipError_t launch_q8_to_h(const int8_t * q, _Float16 * h, int64_t n, hipStream_t st);
-// every column of a.cols in [col0, col1), each on the kernel of its class
+// the table's columns (a.part of them), each on the kernel of its class
 hipError_t launch_prefill_gemm(const PrefillArgs & a, int grid, hipStream_t st);
-// the columns of few slots only (moe_few.hip)
-hipError_t few_init();
-hipError_t launch_few_gemm(const PrefillArgs & a, int grid, hipStream_t st);
 
 // K-quant matrices on the matrix cores, bit-identical to launch_kq_matvec: columns col0 .. col1 - 1 of a KQ_TOK table
 // (routed: expert e at w[0] + e * estride; the shared expert's: sh[0]), ggml's blocks read in place; activation row = slot -

@@ -3,10 +3,10 @@
 // Reference: fl_wide_moe (src/fused_layer.cu:540-561) runs tc_matvec<F_IQ2> (:178-202) per arena batch of <= 72 slots
 // of <= 8 rows each with mma.m16n8k32 s8 tiles, then swiglu_q8 (:334-341) and the down pass; the semantics are ggml's
 // mul_mat_id over IQ2_XXS x Q8_K (ggml_vec_dot_iq2_xxs_q8_K per output). Here one launch per class of columns covers
-// every expert of the layer:
-//   * A column is up to PF_TOK = 112 dispatch slots of one expert (the shared expert's slots P .. P + n - 1 included); an
-//     item is (column, row group). The workgroups (one per CU: the tables fill most of the LDS) take the items
-//     round-robin.
+// every expert of the layer, or one launch both classes of a split table (k_split_gemm; launch_rules.h has the line):
+//   * A column is up to PF_TOK = 112 dispatch slots of one expert (the shared expert's slots P .. P + n - 1 included; in a
+//     split table SPLIT_TOK = 32, those of at most 8 on moe_few.h's kernel); an item is (column, row group). The workgroups
+//     (one per CU: the tables fill most of the LDS) take the items round-robin.
 //   * The weights are dequantised once per item into int8 MFMA operands. A scaled weight v = sign * grid * (2s + 1) is one
 //     of 6 values per sub-block (three magnitudes, two signs) and has at most 11 bits, so it is taken as two int8 digits,
 //     v = 64 h + l, |l| <= 32, |h| <= 21. The codebook table holds, per entry, 8 selector bytes (the magnitude's index
@@ -25,13 +25,13 @@
 // 64 g + 16 m .. + 15 of the block, i.e. entries 2 (m % 2), 2 (m % 2) + 1 of sub-block 2 g + m / 2.
 #include "moe_device.h"
 #include "moe_kernels.h"
+#include "moe_few.h"
 #include <type_traits>
 
 namespace lk {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
-typedef int i4 __attribute__((ext_vector_type(4)));
 
 // Table image: selector lines (entry e: 32 copies of the 8 magnitude indices of grid[e]), sign lines (the 7 stored sign
 // bits: 32 copies of 8 bytes 0 / 4), then the 16 scale lines {l of + magnitudes, l of -, h of +, h of -} (bytes 0..2).
@@ -74,36 +74,56 @@ size_t prefill_table_bytes() { return PTAB_BYTES; }
 // Columns: the shared expert's slots first, then every active expert's slots. An expert's slots go into the fewest columns
 // of at most tok slots, of equal size rounded up to 16 (the last one takes the rest). The routed columns are written class
 // by class, each in act order. Block b writes table b.
+// A split table (T.few) is cut on the device, since only the counts tell a prompt whose tokens spread over the experts from
+// one whose tokens share a few: every column costs about its expert's bytes, whether it has 3 slots or 30, so columns of few
+// slots waste little while most experts have at most T.few, and repeat the weights (and their decoding) where they have more.
+// The larger class saves the difference of the column counts and costs a round of its own.
 __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, const int * __restrict__ nact_p, const int * __restrict__ offsets,
-                                                int n, int P, const PfTable t0, const PfTable t1) {
-    __shared__ int sc[PF_NCLS][256];
+                                                int P, const PfTable t0, const PfTable t1) {
+    static_assert(PF_NCLS == 4, "two classes to a word");
+    __shared__ uint32_t tot[4], part[2][4];
     const PfTable T = blockIdx.x ? t1 : t0;
-    const int i = threadIdx.x, nact = *nact_p;
+    const int i = threadIdx.x, nact = *nact_p, n = T.n;
     auto cls = [&](int slots) -> int { return slots > 64 ? PF_BROAD : slots > 32 ? PF_WIDE : slots > T.few ? PF_NARROW : PF_FEW; };
-    auto cut = [](int cnt, int tok, int & cols, int & size) {   // cols columns of size slots, the last one the rest
-        cols = (cnt + tok - 1) / tok;
-        size = cols > 0 ? min(tok, ((cnt + cols - 1) / cols + 15) / 16 * 16) : 0;
-    };
     int e = 0, s0 = 0, cnt = 0, cols, size;
     if (i < nact) { e = act[i]; s0 = offsets[e]; cnt = offsets[e + 1] - s0; }
+    bool fine = false;                                  // every column cut at T.few
+    if (T.few > 0 && T.tok > T.few) {
+        // three totals in one scan: columns of T.few, columns of T.tok, experts of at most T.few slots (a split table holds
+        // at most 3328 slots of 256 experts: 672, 360 and 256)
+        const uint32_t v = (uint32_t) ((cnt + T.few - 1) / T.few) | (uint32_t) ((cnt + T.tok - 1) / T.tok) << 11 | (cnt > 0 && cnt <= T.few ? 1u << 22 : 0u);
+        const uint32_t w = wave_scan_u32(v);
+        if ((i & 63) == 63) { tot[i >> 6] = w; }
+        __syncthreads();
+        const uint32_t t = tot[0] + tot[1] + tot[2] + tot[3];
+        const int kf = (int) (t & 2047u) + (n + T.few - 1) / T.few, kt = (int) (t >> 11 & 2047u) + (n + T.stok - 1) / T.stok;
+        fine = (t >> 22) > 0 && kf - kt < SPLIT_GAIN;
+    }
+    auto cut = [&](int cnt, int tok, int & cols, int & size) {   // cols columns of size slots, the last one the rest
+        if (fine) { tok = T.few; }
+        cols = (cnt + tok - 1) / tok;
+        size = cols > 0 ? min(tok, ((cnt + cols - 1) / cols + 15) / 16 * 16) : 0;
+        if (!fine && cols > 1 && cnt - size * (cols - 1) <= T.few) { size = (cnt + cols - 1) / cols; }   // (no rest for the few kernel)
+    };
     cut(cnt, T.tok, cols, size);
     int nk[PF_NCLS] = { 0, 0, 0, 0 };                   // this expert's columns of each class
     if (cols > 0) { nk[cls(size)] += cols - 1; nk[cls(cnt - size * (cols - 1))] += 1; }
-    for (int k = 0; k < PF_NCLS; ++k) { sc[k][i] = nk[k]; }
+    // inclusive scans over the experts, two classes to a word (a class has fewer than 2^16 columns)
+    uint32_t sc[2], all[2] = { 0, 0 };
+    for (int h = 0; h < 2; ++h) {
+        sc[h] = wave_scan_u32((uint32_t) nk[2 * h] | (uint32_t) nk[2 * h + 1] << 16);
+        if ((i & 63) == 63) { part[h][i >> 6] = sc[h]; }
+    }
     __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {   // inclusive scans
-        int v[PF_NCLS];
-        for (int k = 0; k < PF_NCLS; ++k) { v[k] = i >= off ? sc[k][i - off] : 0; }
-        __syncthreads();
-        for (int k = 0; k < PF_NCLS; ++k) { sc[k][i] += v[k]; }
-        __syncthreads();
+    for (int h = 0; h < 2; ++h) {
+        for (int w = 0; w < 4; ++w) { sc[h] += w < (i >> 6) ? part[h][w] : 0u; all[h] += part[h][w]; }
     }
     int nsh, ssize;
     cut(n, T.stok, nsh, ssize);
     int at[PF_NCLS], end = nsh;
     for (int k = 0; k < PF_NCLS; ++k) {
-        at[k] = end + sc[k][i] - nk[k];
-        end += sc[k][255];
+        at[k] = end + (int) (sc[k >> 1] >> (16 * (k & 1)) & 0xFFFFu) - nk[k];
+        end += (int) (all[k >> 1] >> (16 * (k & 1)) & 0xFFFFu);
         if (i == 0) { T.ncols[PF_NCLS + 1 + k] = end; }
     }
     for (int c = 0; c < cols; ++c) {
@@ -118,8 +138,8 @@ __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, c
         for (int k = 0; k < PF_NCLS; ++k) { at2 += ns[k]; T.ncols[1 + k] = at2; }
     }
 }
-hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int n, int P, const PfTable & t0, const PfTable & t1, hipStream_t st) {
-    k_pf_cols<<<t1.cols ? 2 : 1, 256, 0, st>>>(act, nact, offsets, n, P, t0, t1);
+hipError_t launch_prefill_cols(const int * act, const int * nact, const int * offsets, int P, const PfTable & t0, const PfTable & t1, hipStream_t st) {
+    k_pf_cols<<<t1.cols ? 2 : 1, 256, 0, st>>>(act, nact, offsets, P, t0, t1);
     return hipGetLastError();
 }
 
@@ -174,46 +194,16 @@ struct PfGeo {
 // one block of one 16-row tile: the tiled chunk g of row r (qs) and d
 struct PfW { u32x4 q; uint16_t d; };
 
-// raw buffer resource over p (gfx9 word 3; the record count only bounds offsets, which stay far below it)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t pf_rsrc(const void * p) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short) 0, 0x7fffffff, 0x00020000);
-}
-// a wave-uniform pointer kept in scalar registers
-__device__ __forceinline__ const uint8_t * pf_uniform(const uint8_t * p) {
-    const uint64_t v = (uint64_t) p;
-    const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (v >> 32));
-    const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) v);
-    return (const uint8_t *) (((uint64_t) hi << 32) | (uint64_t) lo);
-}
-
-// SZ bytes per lane from a buffer straight into LDS (lane L at dst + SZ L); the builtin exists for the device pass only,
-// so the host pass (which instantiates the kernel's launch stub) sees an empty body
-template <int SZ> __device__ __forceinline__ void buf_lds(__amdgpu_buffer_rsrc_t r, LK_LOCAL uint8_t * dst, uint32_t voff, uint32_t soff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (SZ == 16) { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 16, voff, soff, 0, 0); }
-    else { __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LK_LOCAL void *) dst, 4, voff, soff, 0, 0); }
-#else
-    (void) r; (void) dst; (void) voff; (void) soff;
-#endif
-}
-
+// the columns of class CLS (those of the table's part, pf_runs): workgroup bid of gridDim.x
 template <int NMAT, int NB, int W, int C, int NTM, int CLS>
-__global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
+__device__ __forceinline__ void pf_body(const PrefillArgs & a, LK_LOCAL uint8_t * lds, int bid) {
 #pragma clang fp contract(off)
     using Geo = PfGeo<NMAT, NB, W, C, NTM>;
-    extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
-    LK_LOCAL uint8_t * lds = (LK_LOCAL uint8_t *) dyn_lds;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
     const PfRuns runs = pf_runs(a, CLS);
     const int nrg = a.R / Geo::ROWS;
-    if ((int) blockIdx.x >= runs.count() * nrg) { return; }   // nothing to do: not even the tables
-    if (lds_addr(dyn_lds) & 0xFFFFu) {   // table addressing needs a 64 KB aligned base
-        if (threadIdx.x == 0) {
-            __hip_atomic_fetch_or(gptr(a.err), 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (a.herr) { __hip_atomic_store(gptr(a.herr), 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
-        }
-        return;
-    }
+    if (bid >= runs.count() * nrg) { return; }   // nothing to do: not even the tables
+    if (!pf_base_ok(a, (uint32_t) (size_t) lds)) { return; }
     tables_fill(reinterpret_cast<const uint8_t *>(a.ptab), lds, threadIdx.x, W * 64);
     if (threadIdx.x < 16) { reinterpret_cast<LK_LOCAL u32x4 *>(lds + L_SCL)[threadIdx.x] = *(const LK_GLOBAL u32x4 *) (a.ptab + L_SCL / 16 + threadIdx.x); }
     const int r = lane & 15, g = lane >> 4;
@@ -290,7 +280,7 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
 
     const int items = runs.count() * nrg;
     PfW w0[C], w1[C];
-    Item cur = item_of(blockIdx.x);
+    Item cur = item_of(bid);
     auto begin = [&]() {
         rows_of(cur);
         aim(cur);
@@ -300,7 +290,7 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
         __syncthreads();
     };
     if (AHEAD) { begin(); }
-    for (int it = blockIdx.x; it < items; it += gridDim.x) {
+    for (int it = bid; it < items; it += (int) gridDim.x) {
         const Item nxt = item_of(it + (int) gridDim.x < items ? it + (int) gridDim.x : it);   // (none: its loads are not used)
         if (!AHEAD) { begin(); }
         const int sb = cur.sb, sc = cur.sc, rg = cur.rg;
@@ -489,6 +479,27 @@ __global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
     }
 }
 
+template <int NMAT, int NB, int W, int C, int NTM, int CLS>
+__global__ void __launch_bounds__(W * 64, 1) k_pf_gemm(const PrefillArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
+    pf_body<NMAT, NB, W, C, NTM, CLS>(a, (LK_LOCAL uint8_t *) dyn_lds, (int) blockIdx.x);
+}
+template <int NMAT, int NB> __global__ void __launch_bounds__(FNT, 1) k_few_gemm(const PrefillArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
+    few_body<NMAT, NB>(a, (LK_LOCAL uint8_t *) dyn_lds);
+}
+// A split table's two classes in one launch, so that the table may choose on the device and an empty class costs no launch of
+// its own (4.5 us each): the narrow columns first (a workgroup's whole items, from the last workgroup down), then the few
+// ones (a wave's items, from the first workgroup up).
+template <int NMAT, int NB> __global__ void __launch_bounds__(FNT, 1) k_split_gemm(const PrefillArgs a) {
+    static_assert(FNT == 16 * 64, "both on 16 waves");
+    extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
+    LK_LOCAL uint8_t * lds = (LK_LOCAL uint8_t *) dyn_lds;
+    pf_body<NMAT, NB, 16, 1, 2, PF_NARROW>(a, lds, (int) (gridDim.x - 1 - blockIdx.x));
+    __syncthreads();   // its tables and buffers are no longer read
+    few_body<NMAT, NB>(a, lds);
+}
+
 template <int NMAT, int NB, int W, int C, int NTM, int CLS> struct PfKernel {
     using Geo = PfGeo<NMAT, NB, W, C, NTM>;
     static hipError_t setup() {
@@ -500,27 +511,36 @@ template <int NMAT, int NB> struct PfKernels {
     using Broad = PfKernel<NMAT, NB, 8, 1, 7, PF_BROAD>;
     using Wide = PfKernel<NMAT, NB, 8, 2, 4, PF_WIDE>;
     using Narrow = PfKernel<NMAT, NB, 16, 1, 2, PF_NARROW>;
+    static constexpr int SPLIT_LDS = Narrow::Geo::LDS > F_LDS ? Narrow::Geo::LDS : F_LDS;
     static hipError_t setup() {
         hipError_t e = Broad::setup();
         if (e == hipSuccess) { e = Wide::setup(); }
-        return e == hipSuccess ? Narrow::setup() : e;
+        if (e == hipSuccess) { e = Narrow::setup(); }
+        if (e == hipSuccess) { e = hipFuncSetAttribute((const void *) k_split_gemm<NMAT, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, SPLIT_LDS); }
+        return e == hipSuccess ? hipFuncSetAttribute((const void *) k_few_gemm<NMAT, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, F_LDS) : e;
     }
-    static bool rows_ok(int R) { return R % Broad::Geo::ROWS == 0 && R % Wide::Geo::ROWS == 0 && R % Narrow::Geo::ROWS == 0; }
+    static bool rows_ok(int R) { return R % Broad::Geo::ROWS == 0 && R % Wide::Geo::ROWS == 0 && R % Narrow::Geo::ROWS == 0 && R % 64 == 0; }
     static void go(const PrefillArgs & a, int grid, hipStream_t st) {   // classes that cannot occur are not launched
+        if (a.few > 0) {
+            if (a.most > a.few) { k_split_gemm<NMAT, NB><<<grid, FNT, SPLIT_LDS, st>>>(a); }
+            else { k_few_gemm<NMAT, NB><<<grid, FNT, F_LDS, st>>>(a); }
+            return;
+        }
         if (a.most > 64) { Broad::go(a, grid, st); }
         if (a.most > 32) { Wide::go(a, grid, st); }
         Narrow::go(a, grid, st);
     }
 };
 hipError_t prefill_init() {
-    hipError_t e = PfKernels<2, 28>::setup();
-    if (e == hipSuccess) { e = PfKernels<1, 8>::setup(); }
-    return e == hipSuccess ? few_init() : e;
+    const hipError_t e = PfKernels<2, 28>::setup();
+    return e == hipSuccess ? PfKernels<1, 8>::setup() : e;
 }
 
-// the broad, wide, narrow and few kernels over the columns col0 .. col1 - 1 (each takes its class)
+// the kernels of the table's classes over the columns of its part (a.part), each taking its own
 hipError_t launch_prefill_gemm(const PrefillArgs & a, int grid, hipStream_t st) {
-    if (grid < 1 || !a.ptab || !a.cols || !a.ncols || !a.bq || !a.bd || !a.out || !a.err) { return hipErrorInvalidValue; }
+    if (grid < 1 || !a.ptab || !a.tab || !a.cols || !a.ncols || !a.bq || !a.bd || !a.out || !a.err || a.most < 1 || (a.few != 0 && a.few != FEW_TOK)) {
+        return hipErrorInvalidValue;
+    }
     if (a.nmat == 2) {
         if (a.K != 28 * QK || !PfKernels<2, 28>::rows_ok(a.R) || !a.w[0] || !a.w[1] || !a.sh[0] || !a.sh[1] || !a.perm) { return hipErrorInvalidValue; }
         PfKernels<2, 28>::go(a, grid, st);
@@ -530,8 +550,7 @@ hipError_t launch_prefill_gemm(const PrefillArgs & a, int grid, hipStream_t st) 
     } else {
         return hipErrorInvalidValue;
     }
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess && a.few > 0 ? launch_few_gemm(a, grid, st) : e;   // (an empty launch takes 4.5 us)
+    return hipGetLastError();
 }
 
 }  // namespace lk

@@ -239,6 +239,61 @@ def test_wide_pass_row_loop(ctx, small_layer):
         ctx.set_debug(False)
 
 
+def test_wide_pass_time_follows_the_rows(ctx, small_layer):
+    """fl_wide_moe's kernels are chosen by the pairs that come in, not by fl_wide_init's maximum: 72 rows cost the same GPU time
+    with room for 2048 as with room for 72 (280 and 282 us; where the room chose, 304 and 332). 64 resident experts, tiled."""
+    import torch
+    from loki_amd import FLOut, MoeLayerWeights, lib
+    n, ne = 72, 64
+    layer = MoeLayerWeights.synthetic(ctx, 9100, n_exp=ne)
+    mats = [layer.gate, layer.up, layer.down, layer.sh_gate, layer.sh_up, layer.sh_down]
+    x, fi = gen.uniform(8, 23, (n, E), 2.0), gen.uniform(8, 24, (n, E), 1.0)
+    out, took = FLOut(), {72: [], 2048: []}
+    ctx.set_experts(ne)
+    for m in mats:
+        ctx.register_tiled(m)
+    try:
+        flw = _flw(dict(W=layer.gate_inp, b=layer.probs_b, sh=[layer.sh_gate, layer.sh_up, layer.sh_down]))
+        for rnd in range(2):
+            for room in took:
+                assert lib().fl_wide_init(ctx.ctx, room, KE) == 1
+                sel, wts = np.empty((n, KE), np.int32), np.empty((n, KE), np.float32)
+                for r in range(0, n, 64):
+                    g = min(64, n - r)
+                    ctx.check(lib().fl_ffn_begin(ctx.ctx, ctypes.byref(flw), g, cptr(x[r:r + g].copy()), cptr(fi[r:r + g].copy()), r))
+                    lib().fl_fetch(ctx.ctx, g, 1, ctypes.byref(out))
+                    sel[r:r + g] = np.ctypeslib.as_array(out.sel, shape=(g * KE,)).reshape(g, KE)
+                    wts[r:r + g] = np.ctypeslib.as_array(out.wts, shape=(g * KE,)).reshape(g, KE)
+                ids, rows, kidx, wk = [], [], [], []
+                for e in range(ne):
+                    lst = [(i, k) for i in range(n) for k in range(KE) if sel[i, k] == e]
+                    for i0 in range(0, len(lst), 8):
+                        part = lst[i0:i0 + 8]
+                        ids.append(e)
+                        rows += [i for i, _ in part] + [-1] * (8 - len(part)); kidx += [k for _, k in part] + [0] * (8 - len(part))
+                        wk += [wts[i, k] for i, k in part] + [0.0] * (8 - len(part))
+                args = (np.int32(ids), np.int32(rows), np.int32(kidx), f32(wk))
+                t = []
+                for rep in range(25):
+                    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                    a.record()
+                    lib().fl_wide_moe(ctx.ctx, layer.gate.data_ptr(), layer.up.data_ptr(), layer.down.data_ptr(), 4, ne, *(cptr(v) for v in args),
+                                      len(ids), KE, rep & 1)
+                    b.record(); b.synchronize()
+                    t.append(a.elapsed_time(b) * 1e3)
+                took[room].append(sorted(t[5:])[10])
+                lib().fl_wide_finish(ctx.ctx, n, KE, ctypes.byref(out))
+    finally:
+        for m in mats:
+            ctx.unregister_tiled(m)
+        ctx.set_experts(16)   # this module's other tests route over 16 experts
+    print("fl_wide_moe of 72 rows, us: %s" % took, flush=True)
+    a, b = min(took[72]), min(took[2048])
+    assert max(a, b) < 1.07 * min(a, b)
+    del layer
+    torch.cuda.empty_cache()
+
+
 def _wide_pass(ctx, small_layer, waits):
     from loki_amd import FLOut, lib
     (W, b, gate, up, down, sh), dev = small_layer

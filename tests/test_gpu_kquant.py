@@ -557,8 +557,9 @@ def test_prefill_mixed_formats_mfma(ctx, fm, n):
 
 
 # rows at the edges of the kernels' column sizes: the decode batches (from 16 slots on the columns of at most 8), the
-# 16-token tiles and 64-token columns of the K-quant downs, the 8- and 112-token columns of the IQ2_XXS matrices
-EDGE_N = {orc.Q3K: (2, 8, 9, 16, 17, 48, 49, 65, 129), orc.Q2K: (2, 7, 9, 17, 33, 64, 129), 4: (3, 8, 129, 161, 224, 257, 300)}
+# 16-token tiles and 64-token columns of the K-quant downs, the IQ2_XXS matrices' columns of 8 and 32 slots (up to 224 rows of
+# 8 picks) and of 112
+EDGE_N = {orc.Q3K: (2, 8, 9, 16, 17, 48, 49, 65, 129), orc.Q2K: (2, 7, 9, 17, 33, 64, 129), 4: (3, 8, 33, 129, 161, 224, 257, 300, 336, 337)}
 
 
 @pytest.mark.parametrize("fm", [PF_FMTS[0], PF_FMTS[1], PF_FMTS[2], (4, 4, 4, 4)], ids=["q3k_q5q5q6", "q2k_iq2", "iq2_q5q5q6", "iq2"])

@@ -948,15 +948,70 @@ def test_decode1_selection_crafted_logits(ctx, kind):
 
 @pytest.mark.parametrize("n,hot", [(9, True), (12, False), (17, True), (33, False), (64, True), (65, False), (72, True), (200, True)])
 def test_few_slot_columns_match_per_pass(ctx, n, hot):
-    """Columns of 1..8 slots on the int8 matrix-core kernel (every column up to 64 tokens, the small remainders above):
-    one and two sets of four tokens, partly filled ones, the shared expert's last column of 1..8, and hot experts whose
-    slots fill many columns. Bit for bit the per-pass kernels."""
+    """Columns of 1..8 slots on the int8 matrix-core kernel, alone (few columns to save) and beside the narrow ones: one and
+    two sets of four tokens, partly filled ones, the shared expert's columns, and hot experts whose slots fill several
+    columns. Bit for bit the per-pass kernels."""
     layer = make_layer(ctx, seed=2100 + n, bias_sigma=0.05, hot=list(range(5, 256, 32)) if hot else None)
     x = make_x(ctx, n, seed=61 + n)
     ref = _prefill_state(ctx, layer, x, False)
     got = _prefill_state(ctx, layer, x, True)
     for k in ref:
         assert np.array_equal(got[k].view(np.uint8), ref[k].view(np.uint8)), k
+
+
+@pytest.mark.parametrize("ne,n,keep,same", [(256, 9, 0, True), (256, 12, 0, True), (256, 33, 0, True), (256, 40, 0, True), (256, 65, 0, True),
+                                            (256, 200, 0, True), (16, 40, 0, False), (32, 100, 0, False), (64, 128, 0, False), (64, 224, 0, False),
+                                            (64, 225, 0, False), (256, 416, 0, False), (256, 417, 0, False), (256, 300, 2, False), (256, 10, 1, True)])
+def test_split_tables_match_per_pass(ctx, ne, n, keep, same):
+    """Column tables of a prompt's two classes in one launch, bit for bit the per-pass kernels (g, u, h, its Q8_K, o, y): only
+    narrow columns (identical rows: every expert picked has n slots; 33, 65 and 200 are cut into equal parts), narrow beside
+    few (few experts), and both sides of the line to the other table (64 experts 224 / 225 rows, 256 experts 416 / 417)."""
+    import torch
+    from loki_amd import MoeLayerWeights
+    layer = MoeLayerWeights.synthetic(ctx, 2300 + ne + n, n_exp=ne, bias_sigma=0.05)
+    x = make_x(ctx, n, seed=83 + n)
+    if same:
+        x[:] = x[:1].clone()
+    try:
+        if keep:
+            ctx.set_keep(keep, 2.5)
+        ref = _prefill_state(ctx, layer, x, False)
+        got = _prefill_state(ctx, layer, x, True)
+    finally:
+        ctx.set_keep(0)
+    for k in ref:
+        assert np.array_equal(got[k].view(np.uint8), ref[k].view(np.uint8)), k
+    del layer
+    torch.cuda.empty_cache()
+
+
+def _layer_us(ctx, layer, x):
+    """Median GPU time of fl_moe_layer on these rows."""
+    import torch
+    y, t = torch.empty_like(x), []
+    for k in range(30):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record(); ctx.moe_layer(layer, x, y); b.record(); b.synchronize()
+        t.append(a.elapsed_time(b) * 1e3)
+    ctx.sync()
+    return sorted(t[10:])[10]
+
+
+def test_prompt_time_follows_the_experts_used(ctx, layer):
+    """A prompt of 128 rows that use few experts must not stream (and decode) each expert's weights once per 8 rows. Against
+    rows that use nearly all 256 experts (745 us here; 765 with every column cut at 8 slots) identical rows, which use 8 and
+    the shared one, take 240 us (so cut 418), and the rows on a layer of 32 experts 300 (472). The bounds lie between."""
+    import torch
+    from loki_amd import MoeLayerWeights
+    x = make_x(ctx, 128, seed=77)
+    same = x[:1].repeat(128, 1).contiguous()
+    full, one = _layer_us(ctx, layer, x), _layer_us(ctx, layer, same)
+    small = MoeLayerWeights.synthetic(ctx, 2401, n_exp=32)
+    few = _layer_us(ctx, small, x)
+    print("128 rows: %.0f us, identical %.0f us, 32 experts %.0f us" % (full, one, few), flush=True)
+    assert one < 0.42 * full and few < 0.5 * full
+    del small
+    torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("n,ne", [(9, 256), (16, 256), (17, 256), (20, 256), (21, 256), (31, 256), (32, 256), (33, 256), (128, 256),
