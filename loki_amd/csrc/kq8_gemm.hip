@@ -65,7 +65,7 @@ template <int SZ> __device__ __forceinline__ void k8_lds(__amdgpu_buffer_rsrc_t 
 // 201 tokens). Two direct loads copy, per row, the 128-byte window of eight 16-byte units that holds the block (window start:
 // the block's offset rounded down to 16); unit u of row r sits at slot u ^ ((r / 2) % 8) of the row's 128 bytes, so the 16
 // rows of a read hit 16 bank quads. The block's offset in its window, DL, is the same for every row; a field of 16 bytes is
-// two units shifted by DL.
+// two units shifted by DL. (Units count from the matrix's base, which need only be 4-byte aligned, as the loads do.)
 constexpr int K8_WB = 16 * 128;
 template <int F, int J> constexpr int k8_delta() { return (J * kbytes<F>()) & 15; }
 __device__ __forceinline__ uint32_t k8_slot(int r, int u) { return (uint32_t) (r * 128 + ((u ^ ((r >> 1) & 7)) << 4)); }

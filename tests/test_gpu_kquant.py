@@ -556,6 +556,43 @@ def test_prefill_mixed_formats_mfma(ctx, fm, n):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("down_fmt", [orc.Q2K, orc.Q3K], ids=["q2_K", "q3_K"])
+def test_kquant_matrices_off_16_bytes(ctx, down_fmt):
+    """The K-quant matrices are taken from 4-byte aligned addresses: every kernel that reads them in place (the int8 and fp16
+    GEMMs at 40 rows, the mat-vecs at 6, the one-token kernel) gives the same bits from copies 4, 8 and 12 bytes off a
+    16-byte boundary as from the aligned matrices. A 64-expert layer in the real shards' formats."""
+    import torch
+    from loki_amd import MoeLayerWeights
+    from tests._helpers import make_x
+    ne, seed, fm = 64, 8700 + down_fmt, (down_fmt, orc.Q5K, orc.Q5K, orc.Q6K)
+    base = MoeLayerWeights.synthetic(ctx, seed, n_exp=ne, bias_sigma=0.05)
+    mats = [_kq_device(torch, f, r, c, seed + 1 + i) for i, (f, r, c) in enumerate(((fm[0], ne * E, H), (fm[1], H, E), (fm[2], H, E), (fm[3], E, H)))]
+    assert all(m.data_ptr() % 16 == 0 for m in mats)
+    xs = {n: make_x(ctx, n, seed=seed + 10 + n) for n in (1, 6, 40)}
+    ctx.set_layer_formats(*fm)
+    try:
+        want = {}
+        for off in (0, 4, 8, 12):
+            moved = mats
+            if off:
+                moved = []
+                for m in mats:
+                    b = torch.empty(m.numel() + 16, dtype=torch.uint8, device="cuda")
+                    moved.append(b[off:off + m.numel()].copy_(m))
+                assert all(m.data_ptr() % 16 == off for m in moved)
+            layer = MoeLayerWeights(base.gate_inp, base.probs_b, base.gate, base.up, *moved, n_exp=ne)
+            for n, x in xs.items():
+                print("K-quant matrices %s: %d bytes off, %d rows" % (NAMES[down_fmt], off, n), flush=True)
+                y = ctx.moe_layer(layer, x).clone()
+                ctx.sync()
+                want.setdefault(n, y)
+                assert torch.equal(y.view(torch.int32), want[n].view(torch.int32)), (off, n)
+    finally:
+        ctx.set_layer_formats()
+    del base, mats, moved, layer
+    torch.cuda.empty_cache()
+
+
 # rows at the edges of the kernels' column sizes: the decode batches (from 16 slots on the columns of at most 8), the
 # 16-token tiles and 64-token columns of the K-quant downs, the IQ2_XXS matrices' columns of 8 and 32 slots (up to 224 rows of
 # 8 picks) and of 112
