@@ -57,12 +57,10 @@ constexpr int L_NRM = L_CTL + (16 + DW) * 4;                      // pre-norm sc
 // the caller's picks (ext_sel): per token its distinct ids ascending as [first k][summed weight], then their count
 constexpr int L_EXT = L_NRM + DMAX_N * 4, EXT_TOK = 2 * MAXK + 1;
 constexpr int DEC_LDS = L_EXT + DMAX_N * EXT_TOK * 4;
-// the last round's block terms [task][2][7][64] floats: in the rows of the tokens that the call does not have, two tasks
-// a row; with all eight, one task in the early shared task's area (which eight tokens do not use)
+// the last round's block terms [task][7][64] floats, in the row of the first token that the call does not have (with all eight
+// tokens there is no last round: 2048 (keep + 1) tasks are whole rounds of 256 workgroups)
 constexpr int TAIL_MAX = 2;
-static_assert(2 * PRE_BYTES <= GG::XROW, "two tasks' terms in a token row");
-__device__ __forceinline__ int tail_tasks(int n) { return n == DMAX_N ? 1 : TAIL_MAX; }
-__device__ __forceinline__ int tail_terms(int n) { return n == DMAX_N ? L_PRE : L_XS + n * GG::XROW; }
+static_assert(TAIL_MAX * PRE_BYTES / 2 <= GG::XROW, "the tasks' terms in a token row");
 static_assert(DEC_LDS <= 160 * 1024, "LDS budget");
 static_assert(DMAX_N * 4 * 8 <= PRE_BYTES && DW * 112 * 4 <= PRE_BYTES, "router sums and selection scratch overlay the early task terms");
 
@@ -603,9 +601,9 @@ __device__ __forceinline__ void pre_shared_split(const DArgs & a, lds_t lds, con
     }
 }
 
-// The last round's tasks t0 + blockIdx.x + G i < t_end when they leave many waves idle (at most tail_tasks(n) of the eight a
-// workgroup runs in a round): a workgroup's waves share its tasks' steps. Items (task, step) are claimed from an LDS counter, each
-// wave with the next item's loads in flight; block terms go to LDS, and the wave completing a task folds them in block
+// The last round's tasks t0 + blockIdx.x + G i < t_end when they leave many waves idle (at most TAIL_MAX of the eight a
+// workgroup runs in a round): a workgroup's waves share its tasks' steps. Items (task, step) are claimed from an LDS counter,
+// each wave with the next item's loads in flight; block terms go to LDS, and the wave completing a task folds them in block
 // order and publishes h -- the arithmetic of a pass. 3 rows of 3 picks (9 experts:
 // a ninth of the tasks left for a second round) 64.8 -> 56.1 us, with the shared keep 65.1 -> 58.6, 2 rows of 1 pick 35.8 ->
 // 32.5. At three or four tasks a workgroup it gained nothing (4 rows of 3 shared picks 67.1 -> 68.3), at six it lost (2 rows
@@ -615,7 +613,7 @@ __device__ __forceinline__ void gate_up_tail(const DArgs & a, lds_t lds, const L
     const int G = gridDim.x, lane = lane_id();
     const int nt = t0 + (int) blockIdx.x < t_end ? (t_end - 1 - t0 - (int) blockIdx.x) / G + 1 : 0;
     LK_LOCAL unsigned * ctl = reinterpret_cast<LK_LOCAL unsigned *>(lds + L_CTL) + 8 + DW;   // [0] claims, [1 + i] steps of task i done
-    LK_LOCAL float * terms = reinterpret_cast<LK_LOCAL float *>(lds + tail_terms(a.n));
+    LK_LOCAL float * terms = reinterpret_cast<LK_LOCAL float *>(lds + L_XS + a.n * GG::XROW);
     struct Item { GuTask t; uint4 w[4]; uint16_t d; int i, s; };
     auto take = [&](Item & x) -> bool {
         unsigned c = 0;
@@ -628,22 +626,17 @@ __device__ __forceinline__ void gate_up_tail(const DArgs & a, lds_t lds, const L
         x.d = *gptr(reinterpret_cast<const uint16_t *>(x.t.dl + x.s * GU_DSTEP));
         return true;
     };
-    auto run = [&](const Item & x) {
+    auto run = [&](const Item & x) {   // (a task of the routing's list is one token)
         const int j = x.s * 4 + ln.q;
-        GuTask t = x.t;
-        for (t.u = 0; t.u < t.c; ++t.u) {   // both tokens from one load
-            const uint8_t * xr = gu_xrow(a, lds, t, P);
-            const int bsum = block_bsum_dpp(x.w, ln.tr, xr + j * GG::XBLK, ln.r);
-            const float dx = reinterpret_cast<const float *>(xr + GG::NB * GG::XBLK)[j];
-            terms[((2 * x.i + t.u) * GU_STEPS + x.s) * 64 + lane] = (h2f(x.d) * dx) * (float) bsum;
-        }
+        const uint8_t * xr = gu_xrow(a, lds, x.t, P);
+        const int bsum = block_bsum_dpp(x.w, ln.tr, xr + j * GG::XBLK, ln.r);
+        const float dx = reinterpret_cast<const float *>(xr + GG::NB * GG::XBLK)[j];
+        terms[(x.i * GU_STEPS + x.s) * 64 + lane] = (h2f(x.d) * dx) * (float) bsum;
         if (!lds_arrive(ctl + 1 + x.i, GU_STEPS)) { return; }
-        for (t.u = 0; t.u < t.c; ++t.u) {
-            float acc = 0.f;
+        float acc = 0.f;
 #pragma unroll
-            for (int s = 0; s < GU_STEPS; ++s) { acc = fold_rows(acc, terms[((2 * x.i + t.u) * GU_STEPS + s) * 64 + lane]); }
-            gu_publish(a, ln, t, acc);
-        }
+        for (int s = 0; s < GU_STEPS; ++s) { acc = fold_rows(acc, terms[(x.i * GU_STEPS + s) * 64 + lane]); }
+        gu_publish(a, ln, x.t, acc);
     };
     Item x0, x1;
     bool more = take(x0);
@@ -974,7 +967,7 @@ __global__ void __launch_bounds__(DNT, 1) k_moe_decode(const DecodeArgs args) {
     const int t_gu = (nps - ps0) * NGU;
     TRACE(wave, 8);
     const int rest = t_gu % (G * DW);
-    const bool tail = rest > 0 && rest <= tail_tasks(n) * G;
+    const bool tail = rest > 0 && rest <= TAIL_MAX * G && n < DMAX_N;
     const int ntask = gate_up_stream<GU_PD>(a, lds, ln, blockIdx.x * DW + wave, G * DW, tail ? t_gu - rest : t_gu, false, ps0, P, nact);
     if (tail) { gate_up_tail(a, lds, ln, t_gu - rest, t_gu, ps0, P, nact); }
     TRACE(wave, 7);

@@ -837,7 +837,7 @@ def test_decode1_kept_matches_general(ctx, nexp, keep):
 def test_decode_last_round_matches_per_pass(ctx, layer, hot_layer, n, keep):
     """The n <= 8 block where its gate/up tasks leave a last round of one or two tasks a workgroup, whose waves then share
     the tasks' steps (and where they do not): several batches, whose distinct experts and pairs differ, and a layer whose
-    rows share experts (two tokens a task), bit for bit against the per-pass kernels."""
+    rows share experts, bit for bit against the per-pass kernels."""
     ctx.set_keep(keep, 2.5)
     try:
         for lay in (layer, hot_layer):
