@@ -242,7 +242,9 @@ typedef struct FLDebug {
     const float * g, * u;                              /* gate / up outputs when debug capture is on (per-pass path) */
     int n, P, topk;                                    /* topk: slots per row of the last call (the kept count) */
     int fused;                                         /* 1: the last call ran as the single-launch decode block, which
-                                                        * keeps h and o internal (h .. u are NULL then) */
+                                                        * keeps h and o internal (h .. u are NULL then): up to 8 rows of an
+                                                        * all-IQ2_XXS layer, one row of one in the real shards' formats, any
+                                                        * number of kept picks (fl_set_fused(0): the per-pass kernels) */
     int kernel;                                        /* the last call's decode launch: 0 none (per-pass or wide path),
                                                         * 1 the general block, 2 the one-token block organised by XCD,
                                                         * 3 that block launched by fl_ffn_begin on its own picks (fl_moe) */
@@ -264,11 +266,13 @@ int fl_set_debug(FLCtx *, int flags);
 int fl_set_fused(FLCtx *, int mode);
 /* single-token decode with 8 picks drawn, on a 256-CU device: 1 (default) = the single launch organised by XCD
  * (with all 8 kept pick k's expert runs on the 32 CUs of XCD k, with 3 or 4 kept on two XCDs, with 1 or 2 on four; its
- * down split by K-block among the workgroups that produce each h block), 0 = the general single-launch decode block. Both give bit-identical outputs. */
+ * down split by K-block among the workgroups that produce each h block), 0 = the general single-launch decode block
+ * (a layer in the real shards' formats: the per-pass kernels). Both give bit-identical outputs. */
 int fl_set_decode1(FLCtx *, int on);
 /* batches above the decode sizes (n > 8, E 7168, H 2048): 1 (default) = the expert products as grouped GEMMs on the
- * matrix cores (no counterpart in the reference, whose wide path is tc_matvec per arena batch, src/fused_layer.cu:540-561);
- * 0 = the per-pass mat-vec kernels. Both give bit-identical outputs. */
+ * matrix cores (no counterpart in the reference, whose wide path is tc_matvec per arena batch, src/fused_layer.cu:540-561),
+ * and so the IQ2_XXS matrices of 2 .. 8 rows of a layer with K-quants from 16 kept pairs on; 0 = the per-pass mat-vec
+ * kernels. Both give bit-identical outputs. */
 int fl_set_prefill_mfma(FLCtx *, int on);
 
 /* stage timing with HIP events on the context's stream: stages 0..5 = quant_x, router_logits, router_select, dispatch,

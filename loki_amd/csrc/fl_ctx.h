@@ -71,7 +71,7 @@ struct FLCtx {
     int lf[4] = { FL_IQ2, FL_IQ2, FL_IQ2, FL_IQ2 };
     DBuf<float> ksg, ksu;                      // K-quant shared gate / up outputs
     DBuf<unsigned> rcnt;                       // the one-launch routing's self-resetting counter (launch_router_fused)
-    DBuf<double> rpart;                        // the K-split router tiles' parts [KS][n][n_exp]
+    DBuf<double> rpart;                        // the matrix-core router's parts [router_parts][n][n_exp]
     DBuf<int> dscr;                            // the multi-workgroup dispatch's per-round counts and bases
     size_t h2d_zc = 0, h2d_ce = 0; int h2d_said = 0;   // fl_h2d bytes by kernel (mapped pinned) / by copy engine
     // fl_ffn_begin's event pairs (recorded, not yet folded into ms_ffn by fl_gpu_ms) and the reusable ones

@@ -499,7 +499,7 @@ static hipError_t routed_down_kq(FLCtx * c, const FLMoeLayer * L, int P, int E, 
     return launch_kq_matvec(k, c->lf[0], (P + ne - 1) / ne, ne < P ? ne : P, c->st);
 }
 
-// the grouped GEMMs' one-time set-up on this context: fp16 table image, launch attributes, error word
+// the grouped GEMMs' one-time set-up on this context: digit table image, launch attributes, error word
 int prefill_ready(FLCtx * c) {
     if (c->pf_ready) { return FL_OK; }
     ALLOC(c, c->ptab, prefill_table_bytes() / 16);
@@ -585,8 +585,8 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
     const bool fused = (!kq || kq1) && c->fused && n <= 8 && E == 7168 && H == 2048 && decode_rule_ok(ne, c->n_group) && decode_ready(c);
     const bool mfma = !fused && c->pf_mfma && n > 8 && E == 7168 && H == 2048;
     // a decode batch of a K-quant layer: its IQ2_XXS matrices on the matrix-core kernel of columns of at most 8 slots. Two
-    // more launches (the columns, Q8_K of h), so from 16 slots: 2 rows of 8 picks 98.8 -> 95.8 us, 6 rows 195 -> 164, 8 rows
-    // 238 -> 202, 8 rows of 2 picks 109 -> 99; at 6 slots (3 rows of 2) 75.4 -> 77.6
+    // more launches (the columns, Q8_K of h), so from 16 slots (Q2_K downs): 2 rows of 8 picks 106 -> 103 us, 4 rows 158 -> 139,
+    // 6 rows 207 -> 176, 8 rows 254 -> 208, 8 rows of 2 picks 112 -> 102; below, at 6 slots (3 rows of 2), 75.4 -> 77.6
     const bool few = !fused && !mfma && kq && c->pf_mfma && P >= 16 && E == 7168 && H == 2048;
     const int nsi = lf[1] == FL_IQ2 || lf[3] == FL_IQ2 ? n : 0;   // the shared expert's slots in the IQ2_XXS column table
     const bool q5 = lf[1] == FL_Q5K && lf[2] == FL_Q5K, q6 = lf[3] == FL_Q6K;   // shared matrices on fp16 activations

@@ -1,10 +1,11 @@
-"""CPU: the block-sum bound behind the prefill GEMM's exactness, on the adversarial blocks the GPU test uses.
+"""CPU: the block sums that hold the prefill GEMMs to exact integer arithmetic, on the adversarial blocks the GPU test uses.
 
-The MFMA kernel forms each 256-value block sum as two chains of four matrix-core steps (sub-blocks 0, 2, 4, 6 and
-1, 3, 5, 7) and adds the two chain totals once in fp32. These checks pin, with the checker, that (1) on the adversarial
-rows every block sum is odd and above 2^24 -- so a rounding anywhere would show --, (2) each chain's absolute sum stays
-below 2^24 (exact), (3) the two-chain value equals ggml's float(int32 bsum) on every block, and (4) one fp32 chain over
-all eight steps (what the kernel did before) rounds differently on some of them.
+The matrix-core kernels form each 256-value block sum in int32 (int8 digits v = 64 h + l of a scaled weight, or unscaled
+weights whose sub-block sums are scaled in int32) and round it to fp32 once, as ggml rounds its int32 block sum. These
+checks pin, with the checker, that (1) on the adversarial rows every block sum is odd and above 2^24 -- so a second
+rounding anywhere would show --, (2) even two fp32 chains of four steps each (sub-blocks 0, 2, 4, 6 and 1, 3, 5, 7), whose
+absolute sums stay below 2^24, added once, give that value, and (3) one fp32 chain over all eight steps rounds differently
+on some of them. A block's absolute sum stays below 25574752, far inside int32.
 """
 import numpy as np
 

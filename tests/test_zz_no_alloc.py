@@ -67,18 +67,20 @@ def test_noalloc_matches_moe_layer():
         na.close(); ref.close()
 
 
-@pytest.mark.parametrize("n", [1, 8])
-def test_noalloc_graph_replays(n):
+@pytest.mark.parametrize("n,keep", [(1, 0), (8, 0), (1, 2), (1, 4), (1, 6)])
+def test_noalloc_graph_replays(n, keep):
     """One call captured into a HIP graph (torch.cuda.CUDAGraph on the context's stream), replayed nine times over
     three inputs copied into the captured x, with the program's own eager work and a synchronisation between replays:
-    every replay's y equals fl_moe_layer's on that input bit for bit (the one-token kernel at n = 1, the n <= 8 block at
-    n = 8), and fl_sync reports no device error afterwards."""
+    every replay's y equals fl_moe_layer's on that input bit for bit (the one-token kernel at n = 1, with all 8 picks kept and
+    with 2, 4 and 6, whose slots run on 4, 2 and 1 XCDs; the n <= 8 block at n = 8), and fl_sync reports no device error
+    afterwards."""
     import torch
     from loki_amd import FL_OK, Context, lib
     na = Context()
     ref = Context()
     try:
         layer = make_layer(ref, seed=4243)
+        na.set_keep(keep, 2.5); ref.set_keep(keep, 2.5)
         xs = [make_x(ref, n, seed=300 + 10 * n + i) for i in range(3)]
         want = [ref.moe_layer(layer, x).cpu().numpy() for x in xs]
         ref.sync()
