@@ -11,7 +11,7 @@ bench.py in its JSON line), so bench.py can refuse figures that belong to anothe
   bench.py --copy-probe): `profiles/traffic_<key>_<workload>.json`. FETCH_SIZE and WRITE_SIZE are in KiB per dispatch;
   each is scaled by what the same counter reads for the probe's plain 1 GiB device copy (1 GiB read + 1 GiB written).
 
-* matrix-core, LDS and VALU counters (`rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES SQ_INSTS_VALU_MFMA_MOPS_F16
+* matrix-core, LDS and VALU counters (`rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES SQ_INSTS_VALU_MFMA_MOPS_I8
   SQ_LDS_BANK_CONFLICT SQ_LDS_IDX_ACTIVE SQ_ACTIVE_INST_LDS SQ_ACTIVE_INST_VALU SQ_BUSY_CU_CYCLES SQ_INSTS_LDS
   GRBM_GUI_ACTIVE ...`, one run per workload): a markdown table `profiles/<out>.md`, one row per (workload, kernel).
 
@@ -88,7 +88,7 @@ def _durations(trace_csv, pat):
 
 def _grouped(d, g):
     """Consecutive dispatches summed in groups of g (a stage launched as g kernels back to back, e.g. the prefill
-    GEMM's wide and narrow kernels); trailing partial groups are dropped."""
+    GEMM's broad, wide and narrow kernels); trailing partial groups are dropped."""
     if g <= 1:
         return d
     return [sum(d[i:i + g]) for i in range(0, len(d) - len(d) % g, g)]
@@ -179,7 +179,7 @@ def traffic(a):
     print(json.dumps(out, indent=1))
 
 
-PMC = ("SQ_VALU_MFMA_BUSY_CYCLES", "SQ_INSTS_VALU_MFMA_MOPS_F16", "SQ_LDS_BANK_CONFLICT", "SQ_LDS_IDX_ACTIVE",
+PMC = ("SQ_VALU_MFMA_BUSY_CYCLES", "SQ_INSTS_VALU_MFMA_MOPS_I8", "SQ_LDS_BANK_CONFLICT", "SQ_LDS_IDX_ACTIVE",
        "SQ_ACTIVE_INST_LDS", "SQ_ACTIVE_INST_VALU", "SQ_BUSY_CU_CYCLES", "SQ_INSTS_LDS", "GRBM_GUI_ACTIVE")
 
 
@@ -191,7 +191,7 @@ def counters(a):
     md = ["# %s -- rocprofv3 counters" % a.out, "",
           "Command (repo root, on the MI355X box; WL = each workload below, one run each):", "", "    " + a.cmd, ""]
     shas = set()
-    table = ["| workload | kernel | dispatches | MFMA busy | MFMA ops (F16 MOPs) | LDS instructions | LDS conflicts / access | "
+    table = ["| workload | kernel | dispatches | MFMA busy | MFMA ops (int8 MOPs) | LDS instructions | LDS conflicts / access | "
              "LDS active | VALU active |", "|---|---|---:|---:|---:|---:|---:|---:|---:|"]
     for spec in a.runs:
         wl, d, log = spec.split("=")
@@ -214,7 +214,7 @@ def counters(a):
                 conf = m["SQ_LDS_BANK_CONFLICT"] / acc if acc > 0 else 0.0
                 cu = m["SQ_BUSY_CU_CYCLES"] or 1.0
                 table.append("| %s | `%s` | %d | %.1f %% | %.0f M | %.1f M | %.3f | %.0f %% | %.0f %% |" % (
-                    wl, _short(name), len(ds), 100 * busy, m["SQ_INSTS_VALU_MFMA_MOPS_F16"] / 1e6, m["SQ_INSTS_LDS"] / 1e6,
+                    wl, _short(name), len(ds), 100 * busy, m["SQ_INSTS_VALU_MFMA_MOPS_I8"] / 1e6, m["SQ_INSTS_LDS"] / 1e6,
                     conf, 100 * m["SQ_ACTIVE_INST_LDS"] / cu, 100 * m["SQ_ACTIVE_INST_VALU"] / cu))
     md.insert(1, "Library `libloki_moe.so` sha256 prefix %s (the bench lines' `lib_sha16`)." % ", ".join("`%s`" % s for s in sorted(shas)))
     md.insert(2, "")

@@ -16,7 +16,10 @@ def rules(tmp_path_factory):
     d = tmp_path_factory.mktemp("rules")
     src, so = d / "rules.cpp", d / "rules.so"
     src.write_text('#include "%s"\n' % HEADER +
-                   'extern "C" int parts(int n, int ne, int K) { return lk::router_parts(n, ne, K); }\n')
+                   'extern "C" int parts(int n, int ne, int K) { return lk::router_parts(n, ne, K); }\n'
+                   'extern "C" int split(int n, int P, int ne) { return lk::pf_split(n, P, ne); }\n'
+                   'extern "C" int shared_tok(int n, int P) { return lk::split_shared_tok(n, P); }\n'
+                   'extern "C" int few() { return lk::FEW_TOK; }\n')
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
     return ctypes.CDLL(str(so))
 
@@ -37,3 +40,21 @@ def test_router_parts_fill_the_device(rules):
                 continue
             assert p == 8 or (p > 0 and p * tiles >= 128), (n, ne, p)
             assert by_tiles.setdefault(tiles, p) == p, (n, ne, p)
+
+
+def test_split_tables_fit_their_scan(rules):
+    """A split table's three totals share one 32-bit word (k_pf_cols): columns of 8 slots (11 bits), columns of 32 (11 bits) and
+    experts of few slots (10 bits). The line between the tables goes by pairs and experts, so more experts never narrow it,
+    a batch below it stays below with fewer pairs, and the shared expert's rows do not move it."""
+    few = rules.few()
+    for ne in NEXPS:
+        inside = [P for P in range(1, 6000) if rules.split(0, P, ne)]
+        assert inside == list(range(1, len(inside) + 1))
+        top = inside[-1]
+        assert top // few + ne < 1 << 11 and ne < 1 << 10, ne
+        assert all(rules.split(n, top, ne) and not rules.split(n, top + 1, ne) for n in (0, 1, 500, 65536))
+        assert ne == NEXPS[0] or rules.split(0, last, ne)
+        last = top
+    assert rules.split(300, 600, 256) and not rules.split(512, 4096, 256)   # 2 picks a row split, 8 not, whatever the rows
+    for n in NS:
+        assert rules.shared_tok(n, 0) in (8, 16, 32) and rules.shared_tok(n, 8 * n) == 32
