@@ -512,11 +512,13 @@ int prefill_ready(FLCtx * c) {
     return FL_OK;
 }
 
-// The second stream's work of one call: forked from the context's stream (what is queued there so far), joined into it by
-// join(), or by the destructor on every return in between: what that stream still reads and writes (x's Q8_K, the shared
-// rows) belongs to the next call on the context's stream, so an error return must not leave it behind.
+// The second stream's work of one call: forked from the context's stream (what is queued there so far), its end marked when all
+// of it is queued (at once: a mark queued only at the join would hold the join up by its own latency, 2 us of 75 on 2 rows),
+// joined into the context's stream by join(), or by the destructor on every return in between: what that stream still reads
+// and writes (x's Q8_K, the shared rows) belongs to the next call on the context's stream, so an error return must not leave
+// it behind.
 struct SideFork {
-    FLCtx * c; bool live = false;
+    FLCtx * c; bool live = false, marked = false;
     explicit SideFork(FLCtx * ctx) : c(ctx) {}
     SideFork(const SideFork &) = delete;
     SideFork & operator=(const SideFork &) = delete;
@@ -526,10 +528,15 @@ struct SideFork {
         live = e == hipSuccess;
         return e;
     }
+    hipError_t mark() {
+        const hipError_t e = hipEventRecord(c->ejoin, c->side);
+        marked = e == hipSuccess;
+        return e;
+    }
     hipError_t join() {
         if (!live) { return hipSuccess; }
         live = false;
-        hipError_t e = hipEventRecord(c->ejoin, c->side);
+        hipError_t e = marked ? hipSuccess : mark();
         if (e == hipSuccess) { e = hipStreamWaitEvent(c->st, c->ejoin, 0); }
         if (e != hipSuccess) { (void) hipStreamSynchronize(c->side); }   // (no event: wait here instead)
         return e;
@@ -660,6 +667,7 @@ static int moe_layer(FLCtx * c, const FLMoeLayer * L, const float * x, int n, fl
         TRY(c, beside.fork());
         if (int rc = shared_gateup_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
         if (int rc = shared_down_sep(c, L, n, P, E, H, tk, c->side)) { return rc; }
+        TRY(c, beside.mark());
         if (c->dbg_fail) { return fail(c, FL_EHIP, "failure after the second stream's start, asked for by fl_set_debug"); }
     }
     TRY(c, launch_router_logits(L->gate_inp, x, n, ne, E, c->logits.p, rp, st));

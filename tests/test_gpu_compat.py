@@ -241,10 +241,10 @@ def test_wide_pass_row_loop(ctx, small_layer):
 
 def test_wide_pass_time_follows_the_rows(ctx, small_layer):
     """fl_wide_moe's kernels are chosen by the pairs that come in, not by fl_wide_init's maximum: 72 rows cost the same GPU time
-    with room for 2048 as with room for 72 (280 and 282 us; where the room chose, 304 and 332). 64 resident experts, tiled."""
+    with room for 2048 as with room for 72 (600 and 620 us; where the room chose, 776 and 611). 256 resident experts, tiled."""
     import torch
     from loki_amd import FLOut, MoeLayerWeights, lib
-    n, ne = 72, 64
+    n, ne = 72, 256
     layer = MoeLayerWeights.synthetic(ctx, 9100, n_exp=ne)
     mats = [layer.gate, layer.up, layer.down, layer.sh_gate, layer.sh_up, layer.sh_down]
     x, fi = gen.uniform(8, 23, (n, E), 2.0), gen.uniform(8, 24, (n, E), 1.0)
@@ -289,7 +289,7 @@ def test_wide_pass_time_follows_the_rows(ctx, small_layer):
         ctx.set_experts(16)   # this module's other tests route over 16 experts
     print("fl_wide_moe of 72 rows, us: %s" % took, flush=True)
     a, b = min(took[72]), min(took[2048])
-    assert max(a, b) < 1.07 * min(a, b)
+    assert max(a, b) < 1.1 * min(a, b)
     del layer
     torch.cuda.empty_cache()
 
