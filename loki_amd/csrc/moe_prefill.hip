@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, c
     auto cls = [&](int slots) -> int { return slots > 64 ? PF_BROAD : slots > 32 ? PF_WIDE : slots > T.few ? PF_NARROW : PF_FEW; };
     int e = 0, s0 = 0, cnt = 0, cols, size;
     if (i < nact) { e = act[i]; s0 = offsets[e]; cnt = offsets[e + 1] - s0; }
-    bool fine = false;                                  // every column cut at T.few
+    bool fine = false, even = false;                    // every column cut at T.few; no column for the few kernel but rests
     if (T.few > 0 && T.tok > T.few) {
         // three totals in one scan: columns of T.few, columns of T.tok, experts of at most T.few slots (a split table holds
         // at most 3328 slots of 256 experts: 672, 360 and 256)
@@ -97,13 +97,14 @@ __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, c
         __syncthreads();
         const uint32_t t = tot[0] + tot[1] + tot[2] + tot[3];
         const int kf = (int) (t & 2047u) + (n + T.few - 1) / T.few, kt = (int) (t >> 11 & 2047u) + (n + T.stok - 1) / T.stok;
-        fine = (t >> 22) > 0 && kf - kt < SPLIT_GAIN;
+        even = (t >> 22) == 0;
+        fine = !even && kf - kt < SPLIT_GAIN;
     }
     auto cut = [&](int cnt, int tok, int & cols, int & size) {   // cols columns of size slots, the last one the rest
         if (fine) { tok = T.few; }
         cols = (cnt + tok - 1) / tok;
         size = cols > 0 ? min(tok, ((cnt + cols - 1) / cols + 15) / 16 * 16) : 0;
-        if (!fine && cols > 1 && cnt - size * (cols - 1) <= T.few) { size = (cnt + cols - 1) / cols; }   // (no rest for the few kernel)
+        if (even && cols > 1 && cnt - size * (cols - 1) <= T.few) { size = (cnt + cols - 1) / cols; }   // (then no rests either: one class)
     };
     cut(cnt, T.tok, cols, size);
     int nk[PF_NCLS] = { 0, 0, 0, 0 };                   // this expert's columns of each class
