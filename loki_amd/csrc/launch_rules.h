@@ -32,9 +32,11 @@ constexpr int PF_TOK = 112, SPLIT_TOK = 32, FEW_TOK = 8, KQ_TOK = 64;
 // would tell them are on the device). The shared expert alone (its pass over a prompt's rows): 256 rows 359 / 461, 512 648 /
 // 746, 1000 1245 / 1245.
 constexpr bool pf_split(int n, int P, int n_exp) { return P > 0 ? P <= 1280 + 8 * n_exp : n <= 768; }
-// A split table takes the columns of 9 .. 32 slots where they are at least so many fewer than columns of 8 (they cost a round of
-// their own): 24 tokens on 16 hot experts 188 -> 179 us at 8 against 16; none (0) loses 20 us at 12 tokens.
-constexpr int SPLIT_GAIN = 8;
+// A split table takes narrow columns where they replace at least so many columns of 8 for each round of 16 narrow ones: a narrow
+// column is 16 gate/up items, a round of them about 37 us more than the few columns beside it, a column of 8 about 2.2. At 17
+// against always 8, and against 10 and 22: 84 rows of 2 picks, where the shared expert alone would be narrow, 286 / 286 us, 298
+// at 10; 24 rows on 32 experts 139 / 139, 158 at 10; 64 rows of 8 picks 399 / 408, 404 at 22; 76 rows 435 / 461, 446 at 22.
+constexpr int SPLIT_GAIN = 17;
 // the shared expert's columns in a split table; alone (no routed slots) it takes smaller ones, to occupy the CUs: 65 rows 141
 // us in columns of 8, 146 of 16, 157 of 32; 190 rows 315, 292, 292; 300 rows of 16 444, of 32 417
 constexpr int split_shared_tok(int n, int P) { return P > 0 ? SPLIT_TOK : n <= 80 ? FEW_TOK : n <= 256 ? 16 : SPLIT_TOK; }

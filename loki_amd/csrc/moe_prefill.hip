@@ -77,7 +77,8 @@ size_t prefill_table_bytes() { return PTAB_BYTES; }
 // A split table (T.few) is cut on the device, since only the counts tell a prompt whose tokens spread over the experts from
 // one whose tokens share a few: every column costs about its expert's bytes, whether it has 3 slots or 30, so columns of few
 // slots waste little while most experts have at most T.few, and repeat the weights (and their decoding) where they have more.
-// The larger class saves the difference of the column counts and costs a round of its own.
+// Narrow columns save the ones of 8 that they replace and cost rounds of their own (SPLIT_GAIN); with nothing else in the
+// table they are taken anyway.
 __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, const int * __restrict__ nact_p, const int * __restrict__ offsets,
                                                 int P, const PfTable t0, const PfTable t1) {
     static_assert(PF_NCLS == 4, "two classes to a word");
@@ -88,24 +89,32 @@ __global__ void __launch_bounds__(256) k_pf_cols(const int * __restrict__ act, c
     int e = 0, s0 = 0, cnt = 0, cols, size;
     if (i < nact) { e = act[i]; s0 = offsets[e]; cnt = offsets[e + 1] - s0; }
     bool fine = false, even = false;                    // every column cut at T.few; no column for the few kernel but rests
-    if (T.few > 0 && T.tok > T.few) {
-        // three totals in one scan: columns of T.few, columns of T.tok, experts of at most T.few slots (a split table holds
-        // at most 3328 slots of 256 experts: 672, 360 and 256)
-        const uint32_t v = (uint32_t) ((cnt + T.few - 1) / T.few) | (uint32_t) ((cnt + T.tok - 1) / T.tok) << 11 | (cnt > 0 && cnt <= T.few ? 1u << 22 : 0u);
-        const uint32_t w = wave_scan_u32(v);
-        if ((i & 63) == 63) { tot[i >> 6] = w; }
-        __syncthreads();
-        const uint32_t t = tot[0] + tot[1] + tot[2] + tot[3];
-        const int kf = (int) (t & 2047u) + (n + T.few - 1) / T.few, kt = (int) (t >> 11 & 2047u) + (n + T.stok - 1) / T.stok;
-        even = (t >> 22) == 0;
-        fine = !even && kf - kt < SPLIT_GAIN;
-    }
     auto cut = [&](int cnt, int tok, int & cols, int & size) {   // cols columns of size slots, the last one the rest
         if (fine) { tok = T.few; }
         cols = (cnt + tok - 1) / tok;
         size = cols > 0 ? min(tok, ((cnt + cols - 1) / cols + 15) / 16 * 16) : 0;
         if (even && cols > 1 && cnt - size * (cols - 1) <= T.few) { size = (cnt + cols - 1) / cols; }   // (then no rests either: one class)
     };
+    if (T.few > 0 && T.tok > T.few) {
+        // of cnt slots: the columns of T.few that narrow ones replace, and those
+        auto narrow = [&](int cnt, int tok, int & replaced, int & cols) {
+            int size;
+            cut(cnt, tok, cols, size);
+            const int rest = cols > 0 && cnt - size * (cols - 1) <= T.few ? 1 : 0;
+            replaced = (cnt + T.few - 1) / T.few - rest; cols -= rest;
+        };
+        // three totals in one scan: those two, and the experts of at most T.few slots (a split table holds at most 3328 slots
+        // of 256 experts: 672, 360 and 256)
+        int r, m, rs, ms;
+        narrow(cnt, T.tok, r, m);
+        narrow(n, T.stok, rs, ms);
+        const uint32_t w = wave_scan_u32((uint32_t) r | (uint32_t) m << 11 | (cnt > 0 && cnt <= T.few ? 1u << 22 : 0u));
+        if ((i & 63) == 63) { tot[i >> 6] = w; }
+        __syncthreads();
+        const uint32_t t = tot[0] + tot[1] + tot[2] + tot[3];
+        even = (t >> 22) == 0;
+        fine = !even && (int) (t & 2047u) + rs < SPLIT_GAIN * (((int) (t >> 11 & 2047u) + ms + 15) / 16);
+    }
     cut(cnt, T.tok, cols, size);
     int nk[PF_NCLS] = { 0, 0, 0, 0 };                   // this expert's columns of each class
     if (cols > 0) { nk[cls(size)] += cols - 1; nk[cls(cnt - size * (cols - 1))] += 1; }
