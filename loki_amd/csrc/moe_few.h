@@ -7,7 +7,7 @@
 //
 // Most experts of a prompt see few of its tokens (at 37 tokens 123 of 126 used experts at most 8, at 201 116 of 188, at
 // 512 78 of 207), and for those the tiles of k_pf_gemm pay for 16 tokens with the scale in every operand byte. The expert
-// products of 37 tokens took 473 us there (in fp16), 294 here (gate/up 196, down 98; the call 585 -> 336 us, both sides timed
+// products of 37 tokens took 473 us there (in fp16), 294 here (gate/up 196, down 98; the call 593 -> 329 us, both sides timed
 // in turn). It is bound by the weights' bytes: a gate/up without the products took 159 of then 180 us. Here:
 //   * Lane (r, g) of a wave owns row r of a 16-row tile and the 16-byte chunk g (sub-blocks 2g, 2g + 1) of each block, and
 //     builds signed int8 weights from the decode tables (8-byte codebook entries, 16-byte sign entries): 4 VALU
